@@ -29,7 +29,7 @@ EXPORTS = [
     "dkv_attend_scores", "dkv_attend_values",
     "dkv_score_workspace_bytes", "dkv_score_begin", "dkv_score_layer", "dkv_topk_workspace_bytes", "dkv_topk",
     "dkv_gather_cold", "dkv_refine_rows", "dkv_wire_pack", "dkv_wire_unpack", "dkv_attend_layer_noalloc",
-    "dkv_quantize8", "dkv_centered_rows",
+    "dkv_quantize8", "dkv_centered_rows", "dkv_matmul_f32_workspace_bytes", "dkv_matmul_f32",
 ]
 NOALLOC_MAX_BYTES = 64 << 20  # DKV_NOALLOC_MAX_BYTES: the static workspace of dkv_attend_layer_noalloc
 
@@ -89,7 +89,8 @@ def lib() -> ctypes.CDLL:
         handle = ctypes.CDLL(str(LIB_PATH))
         handle.dkv_abi_version.restype = c_i32
         handle.dkv_last_error.restype = ctypes.c_char_p
-        for name in ("dkv_attend_workspace_bytes", "dkv_score_workspace_bytes", "dkv_topk_workspace_bytes"):
+        for name in ("dkv_attend_workspace_bytes", "dkv_score_workspace_bytes", "dkv_topk_workspace_bytes",
+                     "dkv_matmul_f32_workspace_bytes"):
             getattr(handle, name).restype = c_sz
         handle.dkv_topk_workspace_bytes.argtypes = [c_i32]
         if handle.dkv_abi_version() != ABI_VERSION:
@@ -218,6 +219,36 @@ def centered_rows(tensors, cos, sin, mean, start: int, end: int, out) -> None:
                                    c_i32(tokens), c_i32(head_dim), c_vp(ptr(cos)), c_vp(ptr(sin)), c_vp(ptr(mean)),
                                    c_i32(start), c_i32(end), c_vp(ptr(out)), c_vp(stream_handle())),
            "dkv_centered_rows")
+
+
+def matmul_f32(a: torch.Tensor, b: torch.Tensor, bias: torch.Tensor | None = None) -> torch.Tensor:
+    """a [M, K] @ b [K, N] (+ bias [N]) for float32 GPU matrices, on the fp16 matrix cores with float32's
+    accuracy (dkv_matmul_f32).  ``a`` has unit stride along its rows, ``b`` along either dimension (the
+    transpose of a row-major [N, K] is read as it lies)."""
+    for t, name, dims in ((a, "a", 2), (b, "b", 2), (bias, "bias", 1)):
+        if t is not None and (t.dtype != torch.float32 or not t.is_cuda or t.device != a.device or t.dim() != dims):
+            raise ValueError(f"matmul_f32: {name} must be a float32 GPU tensor of {dims} dimensions")
+    (m, k), (kb, n) = a.shape, b.shape
+    if k != kb or (bias is not None and bias.shape[0] != n) or min(m, n, k) == 0:
+        raise ValueError(f"matmul_f32: shapes {tuple(a.shape)} @ {tuple(b.shape)} do not match")
+    if a.stride(1) != 1 or a.stride(0) < k:
+        a = a.contiguous()
+    kn = b.stride(1) == 1 and b.stride(0) >= n
+    if not kn and not (b.stride(0) == 1 and b.stride(1) >= k):
+        b, kn = b.contiguous(), True
+    ldb = b.stride(0) if kn else b.stride(1)
+    if bias is not None:
+        bias = bias.contiguous()
+    out = torch.empty(m, n, dtype=torch.float32, device=a.device)
+    need = lib().dkv_matmul_f32_workspace_bytes(c_i64(m), c_i64(n), c_i64(k))
+    if need == 0:
+        _check(-2, "dkv_matmul_f32_workspace_bytes")
+    workspace = torch.empty(need, dtype=torch.uint8, device=a.device)
+    with torch.cuda.device(a.device):
+        _check(lib().dkv_matmul_f32(c_vp(a.data_ptr()), c_i64(a.stride(0)), c_vp(b.data_ptr()), c_i64(ldb), c_i32(kn),
+                                    c_vp(ptr(bias)), c_i64(m), c_i64(n), c_i64(k), c_vp(ptr(out)), c_i64(n),
+                                    c_vp(ptr(workspace)), c_sz(need), c_vp(stream_handle())), "dkv_matmul_f32")
+    return out
 
 
 def quantize8(coef, codes, low, span, errors=None) -> None:

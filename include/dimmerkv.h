@@ -194,6 +194,19 @@ int dkv_centered_rows(const uint64_t* layer_ptrs, int32_t dtype, int32_t layers,
 int dkv_dequantize_codes(const uint8_t* codes, const uint16_t* low, const uint16_t* span, const uint8_t* planes,
                          int32_t planes_rows, int32_t n, int32_t groups, float* out, void* stream);
 
+/* ---- float32 products on the fp16 matrix cores -----------------------------
+ * C[m][n] = sum_k A[m][k] B[n][k] + bias[n] (bias may be NULL), all float32:
+ * the projections onto a PCA basis and back (scripts/kvtc.py:88-97, :189;
+ * scripts/progressive.py:147-148).  A is [M][lda]; B is [N][ldb], or with
+ * b_is_kn [K][ldb]; C is [M][ldc].  Operands are split into two fp16 pieces per
+ * element in the workspace (4 bytes per element of each padded operand, and
+ * partial sums where a product has few tiles); errors against float64 are below a float32
+ * product's.  Rows with infinities or NaN are multiplied in plain float32. */
+size_t dkv_matmul_f32_workspace_bytes(int64_t M, int64_t N, int64_t K);
+int dkv_matmul_f32(const float* a, int64_t lda, const float* b, int64_t ldb, int32_t b_is_kn, const float* bias,
+                   int64_t M, int64_t N, int64_t K, float* c, int64_t ldc, void* workspace, size_t workspace_bytes,
+                   void* stream);
+
 /* ---- bases ----------------------------------------------------------------
  * basis f32 [F][r] (columns = components, F = L*Hkv*d, row f = (l*Hkv+h)*d+dd;
  * scripts/kvtc.py:100-105, :88-97) -> the fp16 layouts the attention kernels

@@ -1,0 +1,86 @@
+"""The float32 product on the fp16 matrix cores (dkv_matmul_f32) against float64.
+
+Bound: hi + lo holds an element to 2^-22 of itself and the dropped lo lo is below 2^-22 of a product, so the
+split costs at most 3 * 2^-22 of sum |a b|; each of the 3 K / 16 fp32 accumulations rounds by at most 2^-24 of
+sum |a b|, and the scaling, the sum over k ranges and the bias by a few more."""
+
+from __future__ import annotations
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+
+
+def _pair(m, n, k, kn, seed):
+    g = torch.Generator(DEV).manual_seed(seed)
+    a = torch.randn(m, k, generator=g, device=DEV)
+    b = torch.randn(k, n, generator=g, device=DEV) if kn else torch.randn(n, k, generator=g, device=DEV).t()
+    return a, b, torch.randn(n, generator=g, device=DEV)
+
+
+def _check(got, a, b, bias=None):
+    ref = a.double() @ b.double()
+    size = a.double().abs() @ b.double().abs()
+    if bias is not None:
+        ref, size = ref + bias.double(), size + bias.double().abs()
+    bound = (3 * 2.0 ** -22 + (3 * a.shape[1] / 16 + 24) * 2.0 ** -24) * size
+    worst = float(((got.double() - ref).abs() / bound.clamp_min(1e-300)).max())
+    assert got.shape == ref.shape and worst <= 1.0, worst
+    return float((got.double() - ref).norm() / ref.norm()), float((torch.matmul(a, b).double() - a.double() @ b.double()).norm()
+                                                                  / (a.double() @ b.double()).norm())
+
+
+@pytest.mark.parametrize("kn", [True, False])
+@pytest.mark.parametrize("m,n,k", [(1, 1, 1), (37, 65, 63), (256, 256, 64), (257, 255, 65), (300, 513, 130),
+                                   (511, 512, 4099), (64, 100, 40000)])
+def test_matmul_against_float64(m, n, k, kn):
+    import dkv_hip
+
+    a, b, bias = _pair(m, n, k, kn, m + n + k)
+    print(f"[case] matmul {m} x {n} x {k} kn={kn}", flush=True)
+    _check(dkv_hip.matmul_f32(a, b), a, b)
+    mine, lib = _check(dkv_hip.matmul_f32(a, b, bias), a, b, bias)
+    if k >= 1000:  # long sums: closer to float64 than the library's float32 product
+        assert mine <= lib
+
+
+def test_matmul_rows_of_any_scale_strides_and_specials():
+    """Rows over the whole float32 range keep float32's relative accuracy; unaligned and strided operands are
+    read as they lie; infinities and NaN come out where torch puts them."""
+    import dkv_hip
+
+    a, b, _ = _pair(300, 200, 256, True, 5)
+    wide = a * torch.logspace(-37, 30, 300, device=DEV)[:, None]
+    _check(dkv_hip.matmul_f32(wide, b), wide, b)
+    big = torch.randn(300, 261, device=DEV)
+    part = big[:, 3:259]  # rows 1,044 bytes apart, from an address that is no multiple of 16
+    _check(dkv_hip.matmul_f32(part, b[:, 7:150]), part, b[:, 7:150])
+    assert (dkv_hip.matmul_f32(torch.zeros_like(a), b) == 0).all()
+    a[5, 3], a[7, 9], b[4, 11] = float("inf"), float("nan"), float("-inf")
+    got, want = dkv_hip.matmul_f32(a, b), a @ b
+    for same in (torch.isnan, torch.isposinf, torch.isneginf):
+        assert torch.equal(same(got), same(want))
+    fine = torch.isfinite(want)
+    assert torch.allclose(got[fine], want[fine], rtol=1e-4, atol=1e-4)
+
+
+def test_float_product_route():
+    """Small products, watched ones and other types stay with torch, bit for bit."""
+    import kvtc
+
+    a, b, bias = _pair(128, 64, 512, True, 6)
+    assert torch.equal(kvtc.float_product(a, b, bias), a @ b + bias)
+    a, b, bias = _pair(3000, 2048, 1024, True, 7)
+    assert a.shape[0] * a.shape[1] * b.shape[1] >= kvtc.SPLIT_PRODUCT_MIN
+    got = kvtc.float_product(a, b, bias)
+    assert not torch.equal(got, a @ b + bias)
+    _check(got, a, b, bias)
+    weight = b.clone().requires_grad_(True)
+    assert torch.equal(kvtc.float_product(a, weight), a @ weight) and kvtc.float_product(a, weight).requires_grad
+    with torch.autocast("cuda", dtype=torch.float16):
+        assert kvtc.float_product(a, b).dtype == torch.float16
+    assert kvtc.float_product(a.half(), b.half()).dtype == torch.float16
+    out, tangent = torch.func.jvp(lambda x: kvtc.float_product(x, b), (a,), (a,))
+    assert torch.equal(out, a @ b) and torch.equal(tangent, a @ b)
