@@ -23,7 +23,7 @@ ROOT = HERE.parent
 CSRC = HERE / "csrc"
 INCLUDE = ROOT / "include"
 LIB = HERE / "libdimmerkv_hip.so"
-SOURCES = ["dkv_pack.hip", "dkv_attend.hip", "dkv_gemm.hip"]
+SOURCES = ["dkv_pack.hip", "dkv_attend.hip", "dkv_gemm.hip", "dkv_codec.hip"]
 ARCH = os.environ.get("DKV_OFFLOAD_ARCH", "gfx950")
 
 

@@ -30,6 +30,7 @@ EXPORTS = [
     "dkv_score_workspace_bytes", "dkv_score_begin", "dkv_score_layer", "dkv_topk_workspace_bytes", "dkv_topk",
     "dkv_gather_cold", "dkv_refine_rows", "dkv_wire_pack", "dkv_wire_unpack", "dkv_attend_layer_noalloc",
     "dkv_quantize8", "dkv_centered_rows", "dkv_matmul_f32_workspace_bytes", "dkv_matmul_f32",
+    "dkv_ladder_errors", "dkv_ladder_code", "dkv_rows_to_caches", "dkv_copy_tokens",
 ]
 NOALLOC_MAX_BYTES = 64 << 20  # DKV_NOALLOC_MAX_BYTES: the static workspace of dkv_attend_layer_noalloc
 
@@ -219,6 +220,54 @@ def centered_rows(tensors, cos, sin, mean, start: int, end: int, out) -> None:
                                    c_i32(tokens), c_i32(head_dim), c_vp(ptr(cos)), c_vp(ptr(sin)), c_vp(ptr(mean)),
                                    c_i32(start), c_i32(end), c_vp(ptr(out)), c_vp(stream_handle())),
            "dkv_centered_rows")
+
+
+def ladder_errors(coef, bits) -> torch.Tensor:
+    """coef f32 [n, 64G], bits u8 [R, G] -> squared quantization error of every token at every rung [n, R]."""
+    rungs, groups = bits.shape
+    errors = torch.empty(coef.shape[0], rungs, dtype=torch.float32, device=coef.device)
+    _check(lib().dkv_ladder_errors(c_vp(ptr(coef)), c_i32(coef.shape[0]), c_i32(groups), c_vp(ptr(bits)), c_i32(rungs),
+                                   c_vp(ptr(errors)), c_vp(stream_handle())), "dkv_ladder_errors")
+    return errors
+
+
+def ladder_code(coef, bits, level):
+    """coef f32 [n, 64G] at each token's level (int64 [n]: a rung of bits u8 [R, G], R as it is, -1 dropped) ->
+    decoded f32 [n, 64G], codes u8 [n, G, 64], low and scale f16 [n, G]."""
+    (n, features), (rungs, groups) = coef.shape, bits.shape
+    decoded = torch.empty_like(coef)
+    codes = torch.empty(n, groups, features // groups, dtype=torch.uint8, device=coef.device)
+    low = torch.empty(n, groups, dtype=torch.float16, device=coef.device)
+    scale = torch.empty_like(low)
+    _check(lib().dkv_ladder_code(c_vp(ptr(coef)), c_i32(n), c_i32(groups), c_vp(ptr(bits)), c_i32(rungs), c_vp(ptr(level)),
+                                 c_vp(ptr(decoded)), c_vp(ptr(codes)), c_vp(ptr(low)), c_vp(ptr(scale)),
+                                 c_vp(stream_handle())), "dkv_ladder_code")
+    return decoded, codes, low, scale
+
+
+def _pointer_table(tensors) -> torch.Tensor:
+    return torch.tensor([ptr(t) for t in tensors], dtype=torch.int64).to(tensors[0].device)
+
+
+def rows_to_caches(rows, caches, first: int, gap_start: int, gap_len: int, cos=None, sin=None) -> None:
+    """Token-matrix rows f32 [n, L*H*D] into per-layer caches [1, H, T, D] (contiguous, one dtype): row i is token
+    first + i, plus gap_len from token gap_start on; keys are rotated when cos / sin [T, D] are given."""
+    head = caches[0]
+    _, heads, tokens, dim = head.shape
+    table = _pointer_table(caches)
+    _check(lib().dkv_rows_to_caches(c_vp(ptr(rows)), c_i32(rows.shape[0]), c_i32(first), c_i32(gap_start), c_i32(gap_len),
+                                    c_vp(ptr(table)), c_i32(dtype_code(head.dtype)), c_i32(len(caches)), c_i32(heads),
+                                    c_i32(tokens), c_i32(dim), c_vp(ptr(cos)), c_vp(ptr(sin)), c_vp(stream_handle())),
+           "dkv_rows_to_caches")
+
+
+def copy_tokens(src, dst, skip: int, skip_len: int) -> None:
+    """Every token outside [skip, skip + skip_len) of per-layer caches [1, H, T, D] (contiguous, one dtype) into others."""
+    _, heads, tokens, dim = src[0].shape
+    a, b = _pointer_table(src), _pointer_table(dst)
+    _check(lib().dkv_copy_tokens(c_vp(ptr(a)), c_vp(ptr(b)), c_i32(dtype_code(src[0].dtype)), c_i32(len(src)), c_i32(heads),
+                                 c_i32(tokens), c_i32(dim), c_i32(skip), c_i32(skip_len), c_vp(stream_handle())),
+           "dkv_copy_tokens")
 
 
 def matmul_f32(a: torch.Tensor, b: torch.Tensor, bias: torch.Tensor | None = None) -> torch.Tensor:

@@ -251,20 +251,26 @@ class _Parsed:
 def decode_bytes(codec, data: bytes, dtype=torch.float16):
     """Rebuild per-layer keys and values [1, heads, tokens, dim] from ``encode_bytes`` output
     (scripts/kvtc_storage.py:82-135)."""
-    from kvtc import inverse_transform, rope_tables, split_token_matrix
+    from kvtc import _plain_gpu, inverse_transform, rope_tables, rows_to_caches, split_token_matrix
 
     p = _Parsed(codec, data)
     features = codec.layers * codec.heads * codec.head_dim
     cos, sin = rope_tables(codec._model, p.tokens, codec.device)
+    in_kernel = dtype in (torch.float16, torch.bfloat16, torch.float32) and codec.head_dim % 8 == 0
     out = {}
     for kind in ("key", "value"):
-        stream = codec.streams[kind]
+        rows = inverse_transform(p.coefficients(kind), codec.streams[kind], codec.group)
+        idx, stored = p.exact_rows[kind]
+        if stored is not None:
+            rows[idx] = stored
+        if in_kernel and _plain_gpu(rows, cos, sin):
+            like = torch.empty(1, codec.heads, p.tokens, codec.head_dim, dtype=dtype, device=rows.device)
+            out[kind] = rows_to_caches(rows, like, codec.layers, (p.start, p.end), cos, sin, kind == "key")
+            if p.middle < p.tokens:
+                dkv_hip.rows_to_caches(p.exact_tokens[kind].float(), out[kind], 0, p.start, p.middle)
+            continue
         matrix = torch.empty(p.tokens, features, device=codec.device)
-        matrix[p.start:p.end] = inverse_transform(p.coefficients(kind), stream, codec.group)
-        idx, rows = p.exact_rows[kind]
-        if rows is not None:
-            middle_rows = matrix[p.start:p.end]
-            middle_rows[idx] = rows
+        matrix[p.start:p.end] = rows
         rebuilt = codec.from_matrix(matrix, kind, cos, sin, dtype)
         exact_layers = split_token_matrix(p.exact_tokens[kind], codec.layers, codec.heads, codec.head_dim)
         for layer, original in enumerate(exact_layers):

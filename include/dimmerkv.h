@@ -194,6 +194,31 @@ int dkv_centered_rows(const uint64_t* layer_ptrs, int32_t dtype, int32_t layers,
 int dkv_dequantize_codes(const uint8_t* codes, const uint16_t* low, const uint16_t* span, const uint8_t* planes,
                          int32_t planes_rows, int32_t n, int32_t groups, float* out, void* stream);
 
+/* ---- kvtc codec passes (scripts/kvtc.py:62-79, :142-155, :246-274) --------
+ * coefficients f32 [n][64G] (16-byte aligned), a ladder's widths bits u8
+ * [rungs][G] over {0, 2, 4, 8} (rungs <= 64, rungs * G <= 65,536).
+ * dkv_ladder_errors: errors f32 [n][rungs], each token's squared quantization
+ * error at each rung (fp32 sums, in this kernel's order).
+ * dkv_ladder_code: every token at level[t] (int64): a rung (codes u8 [n][G][64],
+ * low / scale f16 [n][G], decoded f32 [n][64G] = code * scale + low), `rungs`
+ * (decoded = the coefficients, no codes) or -1 (zeros). */
+int dkv_ladder_errors(const float* coef, int32_t n, int32_t groups, const uint8_t* bits, int32_t rungs, float* errors,
+                      void* stream);
+int dkv_ladder_code(const float* coef, int32_t n, int32_t groups, const uint8_t* bits, int32_t rungs,
+                    const int64_t* level, float* decoded, uint8_t* codes, uint16_t* low, uint16_t* scale, void* stream);
+
+/* Token-matrix rows f32 [n][layers*heads*head_dim] into per-layer caches
+ * [1][heads][tokens][head_dim] of `dtype` (layer_ptrs: a device array of their
+ * device pointers): row i is token first + i, plus gap_len from token
+ * gap_start on; with cos / sin (f32 [tokens][head_dim]) x cos + rotate_half(x) sin
+ * at that token (scripts/kvtc.py:46-47).  dkv_copy_tokens copies every token
+ * outside [skip, skip + skip_len) between two such sets of caches. */
+int dkv_rows_to_caches(const float* rows, int32_t n, int32_t first, int32_t gap_start, int32_t gap_len,
+                       const uint64_t* layer_ptrs, int32_t dtype, int32_t layers, int32_t heads, int32_t tokens,
+                       int32_t head_dim, const float* cos, const float* sin, void* stream);
+int dkv_copy_tokens(const uint64_t* src_ptrs, const uint64_t* dst_ptrs, int32_t dtype, int32_t layers, int32_t heads,
+                    int32_t tokens, int32_t head_dim, int32_t skip, int32_t skip_len, void* stream);
+
 /* ---- float32 products on the fp16 matrix cores -----------------------------
  * C[m][n] = sum_k A[m][k] B[n][k] + bias[n] (bias may be NULL), all float32:
  * the projections onto a PCA basis and back (scripts/kvtc.py:88-97, :189;
