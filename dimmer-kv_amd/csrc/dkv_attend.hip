@@ -23,8 +23,11 @@
 //                      (half tile, KV head) for the shortest contexts.
 //   K3a value_weights: per (1024-token split, 64-component group, 32 rows):
 //                      p @ value codes on MFMA plus sum(p * offset) ->
-//                      coefficient-space partial sums.
-//   K3b basis_apply  : sum the partials over the splits and multiply once by
+//                      coefficient-space partial sums.  With more query rows
+//                      per KV head than a decode step has (value_rows): one
+//                      fp16 product over the values as fp16 lines, which the
+//                      first such layer's K2 converts beside its scoring.
+//   K3b basis_apply  : (basis_rows, on MFMA, with many rows) sum the partials over the splits and multiply once by
 //                      the value basis of the KV head (per 128-component
 //                      chunk and 64-dimension slice); beside them, four
 //                      one-wave workgroups per output row compute the exact
@@ -70,7 +73,7 @@ struct RowMergeArgs {
   float* ex;              // [batch * R_total][kExactParts][D + 2] per row and share: Me, Le, then ve[D] (row_exact)
   void* out;              // [batch][q_len][Hq][D], out_dtype
   float scaling;
-  // nstats: softmax-statistics entries per row (ntiles, or 2 * ntiles for 128-token entries)
+  // nstats: softmax-statistics entries per row (ntiles; 2 * ntiles for 128-token entries, 4 * ntiles with many rows)
   int batch, n_total, layer, Hkv, Hq, q_len, D, R_total, E_total, query_dtype, nstats, nchunks, out_dtype;
   int e0_single, e_single;  // with one sequence: its first exact token and exact-token count
 };
@@ -94,6 +97,15 @@ struct K2Args {
   float* sub_max;
   float* sub_sum;
   int nstats;  // softmax-statistics entries per row: ntiles, or 2 * ntiles with 128-token entries
+  // many-row decodes: the workgroups past the scoring ones convert the values (value_lines) unless *lines_valid is
+  // set; other decodes clear it (their areas overlap the lines)
+  uint32_t* lines_valid;
+  const uint8_t* vcodes;
+  const float2* vaff;
+  const float* vtop;  // [G][n_slots / 64] (decode_values_block)
+  uint8_t* lines;
+  int* lines_exp;  // [G][n_slots / 64]: the lines hold the values times 2^this
+  int convert_wg;
 };
 
 DKV_DEVICE uint16_t f16_bits(float v) {
@@ -110,6 +122,20 @@ DKV_DEVICE uint32_t pack_f16x2(float lo, float hi) {
   return __builtin_bit_cast(uint32_t, v);
 }
 
+// What pack_f16x2(lo, hi) rounded away, rounded in turn.
+DKV_DEVICE uint32_t pack_f16x2_rest(uint32_t packed, float lo, float hi) {
+  typedef _Float16 half2_t __attribute__((ext_vector_type(2)));
+  const half2_t v = __builtin_bit_cast(half2_t, packed);
+  return pack_f16x2(lo - (float)v[0], hi - (float)v[1]);
+}
+
+// s plus the two halves of a packed pair, in fp32 (subnormal halves count).
+DKV_DEVICE float add_pair(uint32_t pair, float s) {
+  typedef _Float16 half2_t __attribute__((ext_vector_type(2)));
+  const half2_t one = {(half_t)1.0f, (half_t)1.0f};
+  return __builtin_amdgcn_fdot2(__builtin_bit_cast(half2_t, pair), one, s, false);
+}
+
 DKV_DEVICE half8 lds_half8(const half_t* p) { return *(const half8*)p; }
 
 // The query type as a compile-time tag: a kernel section instantiated per type issues its query
@@ -118,29 +144,6 @@ template <int T>
 struct QueryType {
   static constexpr int value = T;
 };
-
-// 8 consecutive query elements (idx a multiple of 8) of type T as fp16.
-template <int T>
-DKV_DEVICE half8 load_query8_t(const void* q, long idx) {
-  half8 r;
-  if constexpr (T == DKV_F16) {
-    r = *(const half8*)((const half_t*)q + idx);
-  } else if constexpr (T == DKV_BF16) {
-    const uint4 v = *(const uint4*)((const uint16_t*)q + idx);
-    const uint32_t w[4] = {v.x, v.y, v.z, v.w};
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      r[2 * i] = (half_t)__uint_as_float(w[i] << 16);
-      r[2 * i + 1] = (half_t)__uint_as_float(w[i] & 0xffff0000u);
-    }
-  } else {
-    const float4 x = *(const float4*)((const float*)q + idx);
-    const float4 y = *(const float4*)((const float*)q + idx + 4);
-    r[0] = (half_t)x.x; r[1] = (half_t)x.y; r[2] = (half_t)x.z; r[3] = (half_t)x.w;
-    r[4] = (half_t)y.x; r[5] = (half_t)y.y; r[6] = (half_t)y.z; r[7] = (half_t)y.w;
-  }
-  return r;
-}
 
 // One query element as the aligned 32-bit word that holds it: one unconditional load whatever the
 // type (a 16-bit tensor has an even element count, so the word never passes its end), converted
@@ -152,26 +155,6 @@ DKV_DEVICE uint32_t load_query_word(const void* q, long idx, int dtype) {
 DKV_DEVICE float query_word_value(uint32_t w, long idx, int dtype) {
   const uint16_t h = (uint16_t)(w >> ((idx & 1) * 16));
   return dtype == DKV_F32 ? __uint_as_float(w) : dtype == DKV_BF16 ? bf16_bits_to_float(h) : half_bits_to_float(h);
-}
-
-// A query fragment as it travels from memory to the MFMA: fp16 and bf16 fragments stay raw
-// 16-byte words until they are used, so their loads can be waited for late; fp32 fragments (two
-// 16-byte loads) are converted when loaded.
-template <int T>
-struct QueryFrag {
-  using type = uint4;
-};
-template <>
-struct QueryFrag<DKV_F32> {
-  using type = half8;
-};
-
-template <int T>
-DKV_DEVICE typename QueryFrag<T>::type load_query_frag(const void* q, long idx) {
-  if constexpr (T == DKV_F32)
-    return load_query8_t<DKV_F32>(q, idx);
-  else
-    return *(const uint4*)((const uint16_t*)q + idx);
 }
 
 // 8 query elements as loaded, before conversion (two 16-byte words for fp32), so that a batch of
@@ -198,38 +181,22 @@ DKV_DEVICE RawQuery8<T> load_raw_query8(const void* q, long idx) {
 }
 
 template <int T>
-DKV_DEVICE half8 query_frag_half(const typename QueryFrag<T>::type& f);
-
-template <int T>
 DKV_DEVICE half8 raw_query8_half(const RawQuery8<T>& r) {
+  half8 h;
   if constexpr (T == DKV_F32) {
-    half8 h;
     h[0] = (half_t)r.x.x; h[1] = (half_t)r.x.y; h[2] = (half_t)r.x.z; h[3] = (half_t)r.x.w;
     h[4] = (half_t)r.y.x; h[5] = (half_t)r.y.y; h[6] = (half_t)r.y.z; h[7] = (half_t)r.y.w;
-    return h;
-  } else {
-    return query_frag_half<T>(r.w);
-  }
-}
-
-template <int T>
-DKV_DEVICE half8 query_frag_half(const typename QueryFrag<T>::type& f) {
-  if constexpr (T == DKV_F32) {
-    return f;
   } else if constexpr (T == DKV_F16) {
-    half8 r;
-    __builtin_memcpy(&r, &f, 16);
-    return r;
+    __builtin_memcpy(&h, &r.w, 16);
   } else {
-    half8 r;
-    const uint32_t w[4] = {f.x, f.y, f.z, f.w};
+    const uint32_t w[4] = {r.w.x, r.w.y, r.w.z, r.w.w};
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-      r[2 * i] = (half_t)__uint_as_float(w[i] << 16);
-      r[2 * i + 1] = (half_t)__uint_as_float(w[i] & 0xffff0000u);
+      h[2 * i] = (half_t)__uint_as_float(w[i] << 16);
+      h[2 * i + 1] = (half_t)__uint_as_float(w[i] & 0xffff0000u);
     }
-    return r;
   }
+  return h;
 }
 
 // ---------------------------------------------------------------------------
@@ -322,11 +289,74 @@ DKV_DEVICE long prob_index(long row, long slot, int R_total) {
   return ((slot >> 4) * R_total + row) * 16 + (slot & 15);
 }
 
-// Question scoring's per-quarter statistics, [R/8][nsub][8]: eight consecutive rows sit together for
+// Many-row decodes: value_rows_kernel's operands (probabilities by row, values by component) as lines, byte offset of
+// (row, 64-slot block t): 128 bytes of 64 tokens, 16-byte piece c stored at c ^ (row & 7), 32 rows consecutive (4 KB).
+DKV_DEVICE long operand_line(long row, int t, int n_slots) {
+  return ((row >> 5) * (n_slots >> 6) + t) * 4096 + (row & 31) * 128;
+}
+
+constexpr float kLn2 = 0.693147180559945309f;
+
+// Question scoring's and many-row decodes' per-quarter statistics, [R/8][nsub][8]: eight consecutive rows sit together for
 // each 64-token quarter t, so a wave's 32 rows store four 32-byte pieces and the row-statistics
 // kernel reads its eight rows' quarters as one contiguous run.
 DKV_DEVICE long sub_index(long row, int t, int nsub) { return ((row >> 3) * nsub + t) * 8 + (row & 7); }
 
+
+// ---------------------------------------------------------------------------
+// Softmax statistics of the compressed part of sequence b, row `row`.
+// ---------------------------------------------------------------------------
+DKV_DEVICE int tiles_before(const int32_t* cu, int b, int tile) {
+  int base = 0;
+  for (int i = 0; i < b; ++i) base += (cu[i + 1] - cu[i] + tile - 1) / tile;
+  return base;
+}
+
+// Part `part` of `parts` of the values as operand lines (many-row decodes): a wave takes one group's 64 components
+// (a lane each) over a 64-slot block: 64 codes and 64 (scale, offset) pairs, the pairs through its LDS area.  The
+// values of a sequence's group are scaled by the power of two that brings their bound into [2^14, 2^15), so a group
+// of small variance keeps fp16's whole precision and one of large values stays finite.
+DKV_DEVICE void value_lines(const K2Args& a, int part, int parts, float2* pairs) {
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, waves = blockDim.x >> 6;
+  const int NTB = a.n_slots >> 6, blocks = a.ntiles * (kTileTok / 64);
+  float2* mine = pairs + wave * 64;
+  for (int u = part * waves + wave; u < a.G * blocks; u += parts * waves) {
+    const int g = u / blocks, t = u % blocks;
+    uint4 c[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) c[i] = *(const uint4*)(a.vcodes + vcode_index(g, lane, t * 64 + i * 16, a.n_slots));
+    const float2 pair = a.vaff[(long)g * a.n_slots + t * 64 + lane];
+    const int b = find_tile(a.cu_seqlens, a.batch, a.n_total, kTileTok, t / (kTileTok / 64)).x;
+    const int2 sr = seq_range(a.cu_seqlens, a.batch, a.n_total, b);
+    const int first = tiles_before(a.cu_seqlens, b, kTileTok) * (kTileTok / 64), n = (sr.y - sr.x + 63) / 64;
+    float top = 0.0f;
+    for (int i = lane; i < n; i += 64) top = fmaxf(top, a.vtop[(long)g * NTB + first + i]);
+    top = wave_max(top);
+    int e = 0;
+    if (top > 0.0f) {
+      (void)frexpf(top, &e);
+      e = min(max(15 - e, -126), 126);
+    }
+    if (lane == 0) a.lines_exp[(long)g * NTB + t] = e;
+    mine[lane] = make_float2(ldexpf(pair.x, e), ldexpf(pair.y, e));
+    __builtin_amdgcn_wave_barrier();  // a wave's LDS accesses run in order: the reads below see the write
+    uint8_t* line = a.lines + operand_line(g * 64 + lane, t, a.n_slots);
+#pragma unroll
+    for (int o = 0; o < 8; ++o) {
+      const uint4 cq = c[o >> 1];
+      const uint32_t w0 = o & 1 ? cq.z : cq.x, w1 = o & 1 ? cq.w : cq.y;
+      uint32_t v[4];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const float4 af = *(const float4*)(mine + o * 8 + 2 * i);  // two slots' pairs
+        const uint32_t cw = (i < 2 ? w0 : w1) >> (16 * (i & 1));
+        v[i] = pack_f16x2(__builtin_fmaf((float)(cw & 0xffu), af.x, af.y), __builtin_fmaf((float)((cw >> 8) & 0xffu), af.z, af.w));
+      }
+      *(uint4*)(line + ((o ^ (lane & 7)) << 4)) = make_uint4(v[0], v[1], v[2], v[3]);
+    }
+    __builtin_amdgcn_wave_barrier();  // the next block's pairs stay behind these reads
+  }
+}
 
 // ---------------------------------------------------------------------------
 // K1 (fp16 operand form): decode the hot key codes of every token into the
@@ -595,6 +625,7 @@ DKV_DEVICE void keys_scores_small_epilogue(const K2Args& a, floatx16 (&acc)[2][4
       const long o = (long)((h0 + hl) * RH + r) * a.nstats + tile;
       a.tile_max[o] = M;
       a.tile_sum[o] = S;
+      if (o == 0) *a.lines_valid = 0u;
     }
   }
   // probabilities relative to the tile maximum, fp16, for the value side; every slot of the
@@ -637,6 +668,12 @@ __global__ __launch_bounds__(kK2Threads) void keys_scores_kernel(K2Args a) {
   __shared__ float q_s[HPW * kSmallRows * D];      // the workgroup's query rows (decode epilogue)
 
   const int bid = blockIdx.x;
+  if constexpr (!SMALL && !ROWMAJOR) {
+    if (bid >= 8 * a.per_xcd) {
+      if (*a.lines_valid == 0) value_lines(a, bid - 8 * a.per_xcd, a.convert_wg, (float2*)lds);
+      return;
+    }
+  }
   const int lin = (bid & 7) * a.per_xcd + (bid >> 3);
   if (lin >= a.total_wg) return;
   const int nhg = a.Hkv / HPW;
@@ -856,7 +893,10 @@ __global__ __launch_bounds__(kK2Threads) void keys_scores_kernel(K2Args a) {
   // 32-63 keep their chunk 2 ks + 1 half and get lanes 0-31's.
   constexpr int HPWAVE = HPW / 2;  // heads handled by each wave in the epilogue
   constexpr int KS = D / 16;       // MFMA k-steps over the head dimension
-  half8 kf[HPWAVE][KS][2];
+  // A decode's keys keep what that rounding takes away as a second fp16 piece (two products per score): it makes up
+  // for the rounding of the value lines, and the scores are then the closer ones.
+  constexpr int KP = ROWMAJOR ? 1 : 2;  // pieces
+  half8 kf[KP][HPWAVE][KS][2];
   {
     const float* cs = (const float*)((const char*)lds + kDmaCosOffset);
     float* sn = (float*)lds;
@@ -866,7 +906,7 @@ __global__ __launch_bounds__(kK2Threads) void keys_scores_kernel(K2Args a) {
 #pragma unroll
     for (int tb = 0; tb < 2; ++tb) {
       const int n = tq * 64 + tb * 32 + l32;
-      uint32_t own[HPWAVE][D / 8][2];  // chunk c of head hh: this lane's 4 halves as 2 dwords
+      uint32_t own[KP][HPWAVE][D / 8][2];  // chunk c of head hh: this lane's 4 halves as 2 dwords
 #pragma unroll
       for (int rb = 0; rb < 4; ++rb) {
         if ((rb % DB) >= HALF_BLK) continue;
@@ -880,75 +920,59 @@ __global__ __launch_bounds__(kK2Threads) void keys_scores_kernel(K2Args a) {
           const float4 s4 = *(const float4*)(sn + o);
           const float cv[4] = {c4.x, c4.y, c4.z, c4.w};
           const float sv[4] = {s4.x, s4.y, s4.z, s4.w};
-          uint32_t lo[2], hi[2];
+          const int clo = (rb % DB) * 4 + v4, chi = (rb2 % DB) * 4 + v4;
 #pragma unroll
           for (int e = 0; e < 4; e += 2) {
             const float klo0 = acc[tb][rb][v4 * 4 + e], khi0 = acc[tb][rb2][v4 * 4 + e];
             const float klo1 = acc[tb][rb][v4 * 4 + e + 1], khi1 = acc[tb][rb2][v4 * 4 + e + 1];
-            lo[e / 2] = pack_f16x2(klo0 * cv[e] - khi0 * sv[e], klo1 * cv[e + 1] - khi1 * sv[e + 1]);
-            hi[e / 2] = pack_f16x2(khi0 * cv[e] + klo0 * sv[e], khi1 * cv[e + 1] + klo1 * sv[e + 1]);
+            const float l0 = klo0 * cv[e] - khi0 * sv[e], l1 = klo1 * cv[e + 1] - khi1 * sv[e + 1];
+            const float h0_ = khi0 * cv[e] + klo0 * sv[e], h1_ = khi1 * cv[e + 1] + klo1 * sv[e + 1];
+            own[0][hh][clo][e / 2] = pack_f16x2(l0, l1);
+            own[0][hh][chi][e / 2] = pack_f16x2(h0_, h1_);
+            if constexpr (KP == 2) {
+              own[1][hh][clo][e / 2] = pack_f16x2_rest(own[0][hh][clo][e / 2], l0, l1);
+              own[1][hh][chi][e / 2] = pack_f16x2_rest(own[0][hh][chi][e / 2], h0_, h1_);
+            }
           }
-          const int clo = (rb % DB) * 4 + v4, chi = (rb2 % DB) * 4 + v4;
-          own[hh][clo][0] = lo[0];
-          own[hh][clo][1] = lo[1];
-          own[hh][chi][0] = hi[0];
-          own[hh][chi][1] = hi[1];
         }
       }
 #pragma unroll
-      for (int hh = 0; hh < HPWAVE; ++hh)
+      for (int p = 0; p < KP; ++p)
 #pragma unroll
-        for (int ks = 0; ks < KS; ++ks) {
-          const auto w0 = __builtin_amdgcn_permlane32_swap(own[hh][2 * ks][0], own[hh][2 * ks + 1][0], false, false);
-          const auto w1 = __builtin_amdgcn_permlane32_swap(own[hh][2 * ks][1], own[hh][2 * ks + 1][1], false, false);
-          const uint32_t f[4] = {w0[0], w1[0], w0[1], w1[1]};
-          __builtin_memcpy(&kf[hh][ks][tb], f, 16);
-        }
+        for (int hh = 0; hh < HPWAVE; ++hh)
+#pragma unroll
+          for (int ks = 0; ks < KS; ++ks) {
+            const auto w0 = __builtin_amdgcn_permlane32_swap(own[p][hh][2 * ks][0], own[p][hh][2 * ks + 1][0], false, false);
+            const auto w1 = __builtin_amdgcn_permlane32_swap(own[p][hh][2 * ks][1], own[p][hh][2 * ks + 1][1], false, false);
+            const uint32_t f[4] = {w0[0], w1[0], w0[1], w1[1]};
+            __builtin_memcpy(&kf[p][hh][ks][tb], f, 16);
+          }
     }
   }
   // the staged RoPE rows are read by every wave before any reuses their LDS
   __syncthreads();
 
   // ---- epilogue 2: scores = q . k * scaling on MFMA, per 32-row block, with the key fragments in
-  // registers; the query fragments of a row block are loaded together (rows past the end read the
-  // last row, whose scores are discarded), in the query's own type.
-  const int mblocks = (RH + 31) / 32;
-  // the query fragments of row block mb of head h (rows past the end read the last row)
-  auto load_queries = [&](auto qtype, auto (&qf)[KS], int h, int mb) {
-    constexpr int QT = decltype(qtype)::value;
-    const int r = min(mb * 32 + l32, RH - 1);
-    const int qh = h * gq + r / a.q_len, qi = r % a.q_len;
-    const long qbase = (((long)b * a.Hq + qh) * a.q_len + qi) * D + lhi * 8;
-#pragma unroll
-    for (int ks = 0; ks < KS; ++ks) qf[ks] = load_query_frag<QT>(a.query, qbase + ks * 16);
-  };
-  // sacc[tb][v] = q . k for token tq*64 + tb*32 + l32 and row mb*32 + 8*(v/4) + 4*lhi + (v&3), or,
-  // with the operands exchanged (TOKENS_IN_V), for token tq*64 + tb*32 + 8*(v/4) + 4*lhi + (v&3) and
-  // row mb*32 + l32
-  auto block_mfma = [&](auto qtype, auto tokens_in_v, floatx16 (&sacc)[2], const half8 (&kf)[KS][2],
-                        const auto (&qf)[KS]) {
-    constexpr int QT = decltype(qtype)::value;
-    constexpr bool TOKENS_IN_V = decltype(tokens_in_v)::value;
+  // registers.  sacc[tb][v] = q . k for token tq*64 + tb*32 + 8*(v/4) + 4*lhi + (v&3) and row mb*32 + l32
+  auto block_mfma = [&](floatx16 (&sacc)[2], int hh, const half8 (&qf)[KS]) {
 #pragma unroll
     for (int tb = 0; tb < 2; ++tb)
 #pragma unroll
       for (int v = 0; v < 16; ++v) sacc[tb][v] = 0.0f;
 #pragma unroll
-    for (int ks = 0; ks < KS; ++ks) {
-      const half8 q8 = query_frag_half<QT>(qf[ks]);
+    for (int p = KP - 1; p >= 0; --p)
 #pragma unroll
-      for (int tb = 0; tb < 2; ++tb) {
-        if constexpr (TOKENS_IN_V)
-          sacc[tb] = __builtin_amdgcn_mfma_f32_32x32x16_f16(kf[ks][tb], q8, sacc[tb], 0, 0, 0);
-        else
-          sacc[tb] = __builtin_amdgcn_mfma_f32_32x32x16_f16(q8, kf[ks][tb], sacc[tb], 0, 0, 0);
-      }
-    }
+      for (int ks = 0; ks < KS; ++ks)
+#pragma unroll
+        for (int tb = 0; tb < 2; ++tb)
+          sacc[tb] = __builtin_amdgcn_mfma_f32_32x32x16_f16(kf[p][hh][ks][tb], qf[ks], sacc[tb], 0, 0, 0);
   };
 
-  // question scoring: probabilities relative to this wave's 64 tokens (a tile quarter) and the
-  // quarter's (max, sum), written at once: no exchange between waves, so heads and row blocks run in
-  // any order (heads outer: one head's key fragments in registers at a time).  The scores come with
+  // Probabilities relative to this wave's 64 tokens (a tile quarter) and the quarter's (max, sum), written at
+  // once: no exchange between waves, so heads and row blocks run in any order (heads outer: one head's key
+  // fragments in registers at a time).  Question scoring takes them relative to the quarter's maximum, row by
+  // row for the importance kernel; decoding relative to the power of two above it, in the lines of
+  // value_rows_kernel (operand_line), which takes them to other maxima exactly.  The scores come with
   // the tokens in the accumulator registers and the rows across the lanes, so a row's quarter
   // statistics are 32 values in the lane and one exchange with lane l32 + 32.
   // The workgroup's query rows go to LDS once, as fp16, in chunks of up to QROWS rows per head: the
@@ -1006,7 +1030,7 @@ __global__ __launch_bounds__(kK2Threads) void keys_scores_kernel(K2Args a) {
         };
         auto quarter = [&](const half8 (&qf)[KS], int mb) {
           floatx16 sacc[2];
-          block_mfma(QueryType<DKV_F32>{}, QueryType<1>{}, sacc, kf[hh], qf);  // fp16 fragments as they are
+          block_mfma(sacc, hh, qf);
           // The maximum is taken over the raw dot products (the scale is positive) and the scale folds
           // into the exponent: p = 2^(q.k * scale * log2(e) - max * scale * log2(e)), one fma and one
           // exp2 per score.  Tokens past the tile's end (last tile only) score -inf.
@@ -1019,20 +1043,30 @@ __global__ __launch_bounds__(kK2Threads) void keys_scores_kernel(K2Args a) {
                 sacc[tb][v] = n < count ? sacc[tb][v] : -INFINITY;
               }
           }
+          float c2 = a.scaling * 1.44269504088896341f;
+          if constexpr (!ROWMAJOR) {
+            if (c2 < 0.0f) {  // (uniform) the maximum below is over the raw products
+              c2 = -c2;
+#pragma unroll
+              for (int tb = 0; tb < 2; ++tb)
+#pragma unroll
+                for (int v = 0; v < 16; ++v) sacc[tb][v] = sacc[tb][v] == -INFINITY ? -INFINITY : -sacc[tb][v];
+            }
+          }
           float mraw = -INFINITY;
 #pragma unroll
           for (int tb = 0; tb < 2; ++tb)
 #pragma unroll
             for (int v = 0; v < 16; ++v) mraw = fmaxf(mraw, sacc[tb][v]);
           mraw = max_xor32(mraw);
-          const float c2 = a.scaling * 1.44269504088896341f;
-          const float off2 = mraw == -INFINITY ? 0.0f : mraw * c2;
+          const float off2 = mraw == -INFINITY ? 0.0f : ROWMAJOR ? mraw * c2 : ceilf(mraw * c2);
 #pragma unroll
           for (int tb = 0; tb < 2; ++tb)
 #pragma unroll
             for (int v = 0; v < 16; ++v)
               sacc[tb][v] = __builtin_amdgcn_exp2f(__builtin_fmaf(sacc[tb][v], c2, -off2));  // -inf -> 0
-          const float mx = mraw * a.scaling;  // the quarter maximum of the scaled scores (-inf if empty)
+          // the quarter maximum of the scaled scores, or the logarithm of the power of two above it (-inf if empty)
+          const float mx = ROWMAJOR ? mraw * a.scaling : mraw == -INFINITY ? -INFINITY : off2 * kLn2;
           const int row0 = c0 + mb * 32;      // first row of the block
           // the fp16 probabilities: pw[tb][j] holds tokens tb*32 + 8j + 4lhi .. + 3 of row l32
           uint2 pw[2][4];
@@ -1042,12 +1076,19 @@ __global__ __launch_bounds__(kK2Threads) void keys_scores_kernel(K2Args a) {
             for (int j = 0; j < 4; ++j)
               pw[tb][j] = make_uint2(pack_f16x2(sacc[tb][4 * j], sacc[tb][4 * j + 1]),
                                      pack_f16x2(sacc[tb][4 * j + 2], sacc[tb][4 * j + 3]));
-          // the quarter sum of the fp32 probabilities (lanes l32 and l32 + 32 hold the row's halves)
+          // the quarter sum (lanes l32 and l32 + 32 hold the row's halves): of the fp32 probabilities, or decoding of
+          // the fp16 ones, so that a row's largest weights lose the same rounding above and below the line
           float sm = 0.0f;
 #pragma unroll
-          for (int tb = 0; tb < 2; ++tb)
+          for (int tb = 0; tb < 2; ++tb) {
+            if constexpr (ROWMAJOR) {
 #pragma unroll
-            for (int v = 0; v < 16; ++v) sm += sacc[tb][v];
+              for (int v = 0; v < 16; ++v) sm += sacc[tb][v];
+            } else {
+#pragma unroll
+              for (int j = 0; j < 4; ++j) sm = add_pair(pw[tb][j].y, add_pair(pw[tb][j].x, sm));
+            }
+          }
           sm = sum_xor32(sm);
           // row l32 of the block into the staging rows
 #pragma unroll
@@ -1065,7 +1106,13 @@ __global__ __launch_bounds__(kK2Threads) void keys_scores_kernel(K2Args a) {
           // the four reads go out together, ahead of the branch (the compiler would otherwise read and
           // wait once per store inside it)
           asm volatile("" ::"v"(pv[0]), "v"(pv[1]), "v"(pv[2]), "v"(pv[3]));
-          if (row0 + 32 <= RH) {  // a whole block: rows row0 + (lane >> 3) + 8 k, 8 rows apart
+          if constexpr (!ROWMAJOR) {
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+              const long r = (long)h * RH + min(row0 + (lane >> 3) + 8 * k, RH - 1);
+              *(u32x4*)((uint8_t*)a.probs + operand_line(r, tile * 4 + tq, a.n_slots) + (((lane & 7) ^ ((int)r & 7)) << 4)) = pv[k];
+            }
+          } else if (row0 + 32 <= RH) {  // a whole block: rows row0 + (lane >> 3) + 8 k, 8 rows apart
             uint16_t* dst = pbase + (long)(h * RH + row0) * pstride + lane_row;
 #pragma unroll
             for (int k = 0; k < 4; ++k) *(u32x4*)(dst + 8 * k * pstride) = pv[k];
@@ -1083,7 +1130,13 @@ __global__ __launch_bounds__(kK2Threads) void keys_scores_kernel(K2Args a) {
           a.sub_sum[sub_index(r_all, tile * 4 + tq, a.ntiles * 4)] = sm;
         };
         // two fragment buffers: the next row block's fragments are read while this block's MFMAs run
-        half8 qa[KS], qb[KS];
+        half8 qa[KS], qb[ROWMAJOR ? KS : 1];
+        if constexpr (!ROWMAJOR) {  // the second pieces take the second buffer's registers
+          for (int mb = 0; mb < nblk; ++mb) {
+            read_queries(qa, mb);
+            quarter(qa, mb);
+          }
+        } else {
         read_queries(qa, 0);
         for (int mb = 0; mb < nblk; mb += 2) {
           read_queries(qb, min(mb + 1, nblk - 1));
@@ -1094,103 +1147,17 @@ __global__ __launch_bounds__(kK2Threads) void keys_scores_kernel(K2Args a) {
           __builtin_amdgcn_sched_barrier(0);
           quarter(qb, mb + 1);
         }
+        }
       }
     }
   };
 
-  // decoding many rows: the four waves of a head exchange their quarters' statistics per row block,
-  // then write probabilities relative to the tile maximum in the value side's layout
-  auto row_blocks = [&](auto qtype) {
-    for (int mb = 0; mb < mblocks; ++mb) {
-      float xs[HPWAVE][16][2];
-#pragma unroll
-      for (int hh = 0; hh < HPWAVE; ++hh) {
-        const int hl = hs * HPWAVE + hh;
-        typename QueryFrag<decltype(qtype)::value>::type qf[KS];
-        load_queries(qtype, qf, h0 + hl, mb);
-        __builtin_amdgcn_sched_barrier(0);
-        floatx16 sacc[2];
-        block_mfma(qtype, QueryType<0>{}, sacc, kf[hh], qf);
-#pragma unroll
-        for (int v = 0; v < 16; ++v) {
-          const int row = mb * 32 + 8 * (v >> 2) + 4 * lhi + (v & 3);
-#pragma unroll
-          for (int tb = 0; tb < 2; ++tb) {
-            const int n = tq * 64 + tb * 32 + l32;
-            xs[hh][v][tb] = (row < RH) && (n < count) ? sacc[tb][v] * a.scaling : -INFINITY;
-          }
-          const float mx = max32(fmaxf(xs[hh][v][0], xs[hh][v][1]));
-          float sm = 0.0f;
-          if (mx != -INFINITY) sm = __expf(xs[hh][v][0] - mx) + __expf(xs[hh][v][1] - mx);
-          sm = sum32(sm);
-          if (l32 == 0) {
-            const int rr = 8 * (v >> 2) + 4 * lhi + (v & 3);
-            stat_m[hl][tq][rr] = mx;
-            stat_s[hl][tq][rr] = sm;
-          }
-        }
-      }
-      __syncthreads();
-      if (tid < HPW * 32) {
-        const int hl = tid >> 5, rr = tid & 31;
-        const int row = mb * 32 + rr;
-        if (row < RH) {
-          float M = -INFINITY;
-#pragma unroll
-          for (int q = 0; q < 4; ++q) M = fmaxf(M, stat_m[hl][q][rr]);
-          float S = 0.0f;
-          if (M != -INFINITY) {
-#pragma unroll
-            for (int q = 0; q < 4; ++q) {
-              const float mq = stat_m[hl][q][rr];
-              if (mq != -INFINITY) S += stat_s[hl][q][rr] * __expf(mq - M);
-            }
-          }
-          const long o = (long)((h0 + hl) * RH + row) * a.nstats + tile;
-          a.tile_max[o] = M;
-          a.tile_sum[o] = S;
-        }
-      }
-      // probabilities relative to the tile maximum (fp16), from the registers; 0 past the tokens
-#pragma unroll
-      for (int hh = 0; hh < HPWAVE; ++hh) {
-        const int hl = hs * HPWAVE + hh;
-#pragma unroll
-        for (int v = 0; v < 16; ++v) {
-          const int rr = 8 * (v >> 2) + 4 * lhi + (v & 3);
-          const int row = mb * 32 + rr;
-          if (row >= RH) continue;
-          float M = -INFINITY;
-#pragma unroll
-          for (int q = 0; q < 4; ++q) M = fmaxf(M, stat_m[hl][q][rr]);
-          const long r_all = (long)(h0 + hl) * RH + row;
-#pragma unroll
-          for (int tb = 0; tb < 2; ++tb) {
-            const float x = xs[hh][v][tb];
-            const int n = tq * 64 + tb * 32 + l32;
-            a.probs[prob_index(r_all, (long)tile * kTileTok + n, a.Hq * a.q_len)] =
-                f16_bits(x == -INFINITY ? 0.0f : __expf(x - M));
-          }
-        }
-      }
-      __syncthreads();
-    }
-  };
-  if constexpr (ROWMAJOR) {
-    if (a.query_dtype == DKV_F16)
-      row_blocks_quarters(QueryType<DKV_F16>{});
-    else if (a.query_dtype == DKV_BF16)
-      row_blocks_quarters(QueryType<DKV_BF16>{});
-    else
-      row_blocks_quarters(QueryType<DKV_F32>{});
-  } else {
-    if (a.query_dtype == DKV_F16)
-      row_blocks(QueryType<DKV_F16>{});
-    else if (a.query_dtype == DKV_BF16)
-      row_blocks(QueryType<DKV_BF16>{});
-    else
-      row_blocks(QueryType<DKV_F32>{});
-  }
+  if (a.query_dtype == DKV_F16)
+    row_blocks_quarters(QueryType<DKV_F16>{});
+  else if (a.query_dtype == DKV_BF16)
+    row_blocks_quarters(QueryType<DKV_BF16>{});
+  else
+    row_blocks_quarters(QueryType<DKV_F32>{});
   }
 }
 
@@ -1220,31 +1187,208 @@ DKV_DEVICE void static_for(Fn&& f) {
   static_for_seq(f, std::make_integer_sequence<int, N>{});
 }
 
+// ---------------------------------------------------------------------------
+// The head kernel's epilogue for many query rows: RoPE in registers and fp16 key fragments as in the 256-row
+// kernel (one 32-token block per wave), then the workgroup's heads' rows in blocks of 32: the block's queries from
+// LDS (staged a block ahead), q . k on MFMA, and the probabilities relative to the power of two above the maximum
+// of the tile quarter, which two waves hold: they exchange their maxima, and their sums a block later.
+// ---------------------------------------------------------------------------
+constexpr int kManyStage = 40;  // halves per staged probability row: 32 tokens and 8 of padding
+
+template <int D, int NW, int QT, int DB, int HALF_BLK>
+DKV_DEVICE void many_rows_epilogue(const K2Args& a, floatx16 (&acc)[DB], float4 (&cw)[HALF_BLK][4],
+                                        float4 (&sw)[HALF_BLK][4], half_t* lds, int tile, int part, int n, int count, int b,
+                                        int h0, int RH) {
+  constexpr int NT = NW * 64;
+  constexpr int HPG = 128 / D, KS = D / 16;
+  constexpr int QSTR = D + 8;  // staged query row (conflict-free 16-byte reads)
+  constexpr int C8 = D / 8;
+  constexpr int PIECES = HPG * 32 * C8 / NT;  // 16-byte query pieces per thread and block
+  static_assert(PIECES * NT == HPG * 32 * C8, "whole staging rounds");
+  __shared__ float smax[2][NW][HPG][32], ssum[2][NW][HPG][32];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int l32 = lane & 31, lhi = lane >> 5;
+  half8 kf[2][HPG][KS];  // fp16 keys and what their rounding took away (see the 256-row kernel)
+  {
+    uint32_t own[2][HPG][D / 8][2];  // chunk c of head hh: this lane's 4 halves as 2 dwords
+#pragma unroll
+    for (int hh = 0; hh < HPG; ++hh)
+#pragma unroll
+      for (int rb = 0; rb < HALF_BLK; ++rb)
+#pragma unroll
+        for (int v4 = 0; v4 < 4; ++v4) {
+          const float cv[4] = {cw[rb][v4].x, cw[rb][v4].y, cw[rb][v4].z, cw[rb][v4].w};
+          const float sv[4] = {sw[rb][v4].x, sw[rb][v4].y, sw[rb][v4].z, sw[rb][v4].w};
+          const int lo_b = hh * 2 * HALF_BLK + rb, hi_b = lo_b + HALF_BLK;
+          const int clo = rb * 4 + v4, chi = (rb + HALF_BLK) * 4 + v4;
+#pragma unroll
+          for (int e = 0; e < 4; e += 2) {
+            const float klo0 = acc[lo_b][v4 * 4 + e], khi0 = acc[hi_b][v4 * 4 + e];
+            const float klo1 = acc[lo_b][v4 * 4 + e + 1], khi1 = acc[hi_b][v4 * 4 + e + 1];
+            const float l0 = klo0 * cv[e] - khi0 * sv[e], l1 = klo1 * cv[e + 1] - khi1 * sv[e + 1];
+            const float h0_ = khi0 * cv[e] + klo0 * sv[e], h1_ = khi1 * cv[e + 1] + klo1 * sv[e + 1];
+            own[0][hh][clo][e / 2] = pack_f16x2(l0, l1);
+            own[0][hh][chi][e / 2] = pack_f16x2(h0_, h1_);
+            own[1][hh][clo][e / 2] = pack_f16x2_rest(own[0][hh][clo][e / 2], l0, l1);
+            own[1][hh][chi][e / 2] = pack_f16x2_rest(own[0][hh][chi][e / 2], h0_, h1_);
+          }
+        }
+#pragma unroll
+    for (int p = 0; p < 2; ++p)
+#pragma unroll
+      for (int hh = 0; hh < HPG; ++hh)
+#pragma unroll
+        for (int ks = 0; ks < KS; ++ks) {
+          const auto w0 = __builtin_amdgcn_permlane32_swap(own[p][hh][2 * ks][0], own[p][hh][2 * ks + 1][0], false, false);
+          const auto w1 = __builtin_amdgcn_permlane32_swap(own[p][hh][2 * ks][1], own[p][hh][2 * ks + 1][1], false, false);
+          const uint32_t f[4] = {w0[0], w1[0], w0[1], w1[1]};
+          __builtin_memcpy(&kf[p][hh][ks], f, 16);
+        }
+  }
+  const int mblocks = (RH + 31) / 32;
+  const long qrow0 = (long)b * a.Hq * a.q_len + (long)h0 * RH;  // row r of head h0 + hh is query row qrow0 + hh * RH + r
+  half_t* stage = lds + 2 * HPG * 32 * QSTR + wave * 32 * kManyStage;
+  RawQuery8<QT> qv[PIECES];
+  auto load_queries = [&](int mb) {  // rows past the end repeat the last row
+#pragma unroll
+    for (int p = 0; p < PIECES; ++p) {
+      const int e = tid + p * NT, row = e / C8 % 32, hh = e / C8 / 32;
+      qv[p] = load_raw_query8<QT>(a.query, (qrow0 + hh * RH + min(mb * 32 + row, RH - 1)) * D + e % C8 * 8);
+    }
+  };
+  auto store_queries = [&](int buf) {
+#pragma unroll
+    for (int p = 0; p < PIECES; ++p) {
+      const int e = tid + p * NT;
+      *(half8*)(lds + (buf * HPG * 32 + e / C8) * QSTR + e % C8 * 8) = raw_query8_half<QT>(qv[p]);
+    }
+  };
+  const int quarter = tile * 4 + (part * NW + wave) / 2, nsub = a.nstats;
+  // the quarter's statistics of row block mb, by its even wave, once both waves' sums are in
+  auto write_stats = [&](int mb) {
+    if ((wave & 1) || lhi) return;
+#pragma unroll
+    for (int hh = 0; hh < HPG; ++hh) {
+      const float m0 = smax[mb & 1][wave][hh][l32], m1 = smax[mb & 1][wave + 1][hh][l32];
+      const float m = fmaxf(m0, m1);
+      const long r = (long)(h0 + hh) * RH + min(mb * 32 + l32, RH - 1);
+      a.sub_max[sub_index(r, quarter, nsub)] = m == -INFINITY ? -INFINITY : m * kLn2;
+      a.sub_sum[sub_index(r, quarter, nsub)] = ssum[mb & 1][wave][hh][l32] + ssum[mb & 1][wave + 1][hh][l32];
+    }
+  };
+  const float c2s = a.scaling * 1.44269504088896341f;
+  const float c2 = fabsf(c2s);
+  load_queries(0);
+  __syncthreads();  // the main loop's basis blocks are read
+  store_queries(0);
+  for (int mb = 0; mb < mblocks; ++mb) {
+    __syncthreads();  // this block's queries are in, the previous block's sums too
+    if (mb > 0) write_stats(mb - 1);
+    load_queries(min(mb + 1, mblocks - 1));
+    floatx16 sacc[HPG];
+    float E[HPG];
+#pragma unroll
+    for (int hh = 0; hh < HPG; ++hh) {
+#pragma unroll
+      for (int v = 0; v < 16; ++v) sacc[hh][v] = 0.0f;
+      const half_t* src = lds + ((mb & 1) * HPG * 32 + hh * 32 + l32) * QSTR + lhi * 8;
+#pragma unroll
+      for (int ks = 0; ks < KS; ++ks) {
+        const half8 qf = lds_half8(src + ks * 16);
+        sacc[hh] = __builtin_amdgcn_mfma_f32_32x32x16_f16(kf[1][hh][ks], qf, sacc[hh], 0, 0, 0);
+        sacc[hh] = __builtin_amdgcn_mfma_f32_32x32x16_f16(kf[0][hh][ks], qf, sacc[hh], 0, 0, 0);
+      }
+      if (c2s < 0.0f) {  // (uniform) the maximum is over the raw products
+#pragma unroll
+        for (int v = 0; v < 16; ++v) sacc[hh][v] = -sacc[hh][v];
+      }
+      if (count < kTileTok) {  // token n - l32 + 8 (v / 4) + 4 lhi + (v & 3) of the tile
+#pragma unroll
+        for (int v = 0; v < 16; ++v)
+          if (n - l32 + 8 * (v >> 2) + 4 * lhi + (v & 3) >= count) sacc[hh][v] = -INFINITY;
+      }
+      float m = -INFINITY;
+#pragma unroll
+      for (int v = 0; v < 16; ++v) m = fmaxf(m, sacc[hh][v]);
+      m = max_xor32(m);
+      E[hh] = m == -INFINITY ? -INFINITY : ceilf(m * c2);
+      if (lhi == 0) smax[mb & 1][wave][hh][l32] = E[hh];
+    }
+    __syncthreads();  // the waves' maxima
+    store_queries((mb + 1) & 1);
+#pragma unroll
+    for (int hh = 0; hh < HPG; ++hh) {
+      const float top = fmaxf(E[hh], smax[mb & 1][wave ^ 1][hh][l32]);
+      const float off = top == -INFINITY ? 0.0f : top;
+      float s = 0.0f;
+#pragma unroll
+      for (int v = 0; v < 16; ++v) sacc[hh][v] = __builtin_amdgcn_exp2f(__builtin_fmaf(sacc[hh][v], c2, -off));  // -inf -> 0
+      uint2 pw[4];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        pw[j] = make_uint2(pack_f16x2(sacc[hh][4 * j], sacc[hh][4 * j + 1]), pack_f16x2(sacc[hh][4 * j + 2], sacc[hh][4 * j + 3]));
+        s = add_pair(pw[j].y, add_pair(pw[j].x, s));
+      }
+      s = sum_xor32(s);
+      if (lhi == 0) ssum[mb & 1][wave][hh][l32] = s;
+      // row l32 of the block: this wave's 32 tokens, then 64 bytes of each row (half its line) by four lanes
+#pragma unroll
+      for (int j = 0; j < 4; ++j) *(uint2*)(stage + l32 * kManyStage + 8 * j + 4 * lhi) = pw[j];
+      __builtin_amdgcn_wave_barrier();  // a wave's LDS accesses run in order: the reads see the writes
+#pragma unroll
+      for (int k = 0; k < 2; ++k) {
+        const int rl = (lane >> 2) + 16 * k, c = (wave & 1) * 4 + (lane & 3);
+        const uint4 v = *(const uint4*)(stage + rl * kManyStage + (lane & 3) * 8);
+        const long r = (long)(h0 + hh) * RH + min(mb * 32 + rl, RH - 1);  // rows past the end store the last row's bytes
+        *(uint4*)((uint8_t*)a.probs + operand_line(r, quarter, a.n_slots) + ((c ^ ((int)r & 7)) << 4)) = v;
+      }
+      __builtin_amdgcn_wave_barrier();  // the next head's writes stay behind these reads
+    }
+  }
+  __syncthreads();
+  write_stats(mblocks - 1);
+}
+
 // NW waves of 32 tokens: the whole tile (8), or half of it (4) when short contexts leave CUs idle
 // even with one workgroup per (tile, head); the softmax statistics then cover the workgroup's 128
 // tokens (entry 2 * tile + half).
-template <int D, int NW>
+//
+// MANY: more query rows per head than the few-row epilogue holds (k2_rows_waves).  The workgroup then covers 128
+// basis rows (one head at D = 128, two at D = 64) and 32 NW tokens, down to a tile quarter (NW = 2), and
+// many_rows_epilogue writes what the 256-row kernel's many-row epilogue writes.
+template <int D, int NW, bool MANY = false>
 __global__ __launch_bounds__(NW * 64) void keys_scores_head_kernel(K2Args a) {
   constexpr int NT = NW * 64;       // threads
   constexpr int TT = NW * 32;       // tokens of the workgroup
   constexpr int PARTS = kTileTok / TT;
-  constexpr int DB = D / 32;        // 32-row blocks of the head
-  constexpr int HALF_BLK = DB / 2;  // RoPE partner offset in blocks
+  constexpr int ROWS = MANY ? 128 : D;  // basis rows of the workgroup
+  constexpr int HPG = ROWS / D;     // heads of the workgroup
+  constexpr int DB = ROWS / 32;     // 32-row blocks
+  constexpr int HALF_BLK = D / 64;  // RoPE partner offset in blocks (within a head)
   constexpr int HALF_D = D / 2;
-  constexpr int BQ = D * 8 / NT;    // basis loads per thread and group: [D][64] fp16 = D * 8 x 16 B
-  constexpr int RING = 4;           // groups whose loads are in flight
-  constexpr int BLK = D * kStride;  // halves per LDS basis block
-  constexpr int QE = (kSmallRows * D + NT - 1) / NT;  // query elements per thread
-  static_assert(NW == 8 || NW == 4, "a tile or half of it");
-  static_assert(BQ * NT == D * 8, "whole rounds of basis loads");
-  __shared__ __attribute__((aligned(16))) half_t lds[2 * BLK];  // two basis blocks
+  constexpr int BQ = ROWS * 8 / NT;    // basis loads per thread and group: [ROWS][64] fp16 = ROWS * 8 x 16 B
+  constexpr int RING = NW == 2 ? 2 : 4;  // groups whose loads are in flight (two waves hold 16 KB of basis a group)
+  constexpr int BLK = ROWS * kStride;  // halves per LDS basis block
+  constexpr int QE = MANY ? 1 : (kSmallRows * D + NT - 1) / NT;  // query elements per thread (few rows)
+  static_assert(NW == 8 || NW == 4 || (MANY && NW == 2), "a tile, half of it or a quarter");
+  static_assert(BQ * NT == ROWS * 8, "whole rounds of basis loads");
+  // two basis blocks; afterwards the many-row epilogue's staging (two blocks of query rows, the waves' probabilities)
+  constexpr int MANY_HALVES = 2 * HPG * 32 * (D + 8) + NW * 32 * kManyStage;
+  __shared__ __attribute__((aligned(16))) half_t lds[MANY && MANY_HALVES > 2 * BLK ? MANY_HALVES : 2 * BLK];
   __shared__ __attribute__((aligned(16))) float stat_m[NW][kSmallRows];
   __shared__ __attribute__((aligned(16))) float stat_s[NW][kSmallRows];
   __shared__ __attribute__((aligned(16))) float q_s[kSmallRows * D];  // rows past RH are 0
 
+  if constexpr (MANY) {
+    if ((int)blockIdx.x >= 8 * a.per_xcd) {
+      if (*a.lines_valid == 0) value_lines(a, blockIdx.x - 8 * a.per_xcd, a.convert_wg, (float2*)lds);
+      return;
+    }
+  }
   const int lin = (blockIdx.x & 7) * a.per_xcd + (blockIdx.x >> 3);
   if (lin >= a.total_wg) return;
-  const int tp = lin / a.Hkv, h = lin % a.Hkv;  // tp = PARTS * tile + part: the statistics entry
+  const int nhg = a.Hkv / HPG;
+  const int tp = lin / nhg, h = lin % nhg * HPG;  // tp = PARTS * tile + part: the statistics entry; h: first head
   const int tile = tp / PARTS, part = tp % PARTS;
   const int2 bt = find_tile(a.cu_seqlens, a.batch, a.n_total, kTileTok, tile);
   const int b = bt.x;
@@ -1267,6 +1411,7 @@ __global__ __launch_bounds__(NW * 64) void keys_scores_head_kernel(K2Args a) {
   // switch made the conversion wait for the value before anything else was issued
   const bool q32 = a.query_dtype == DKV_F32;
   uint32_t qlo_bits[QE], qhi_bits[QE];
+  if constexpr (!MANY)
 #pragma unroll
   for (int i = 0; i < QE; ++i) {
     const int e = min(tid + i * NT, kSmallRows * D - 1);
@@ -1300,7 +1445,7 @@ __global__ __launch_bounds__(NW * 64) void keys_scores_head_kernel(K2Args a) {
   // basis pieces of the groups in flight: one vector per slot (as arrays, the compiler kept them
   // in scratch memory)
   typedef uint32_t BasisVec __attribute__((ext_vector_type(4 * BQ)));
-  static_assert(RING == 4, "four basis slots");
+  static_assert(RING <= 4, "at most four basis slots");
   BasisVec bq0, bq1, bq2, bq3;
   auto bq_slot = [&](auto slot) -> BasisVec& {
     constexpr int s = decltype(slot)::value;
@@ -1351,6 +1496,7 @@ __global__ __launch_bounds__(NW * 64) void keys_scores_head_kernel(K2Args a) {
       }
   };
   auto write_query = [&]() {
+    if constexpr (MANY) return;
 #pragma unroll
     for (int i = 0; i < QE; ++i) {
       const int e = tid + i * NT;
@@ -1394,6 +1540,16 @@ __global__ __launch_bounds__(NW * 64) void keys_scores_head_kernel(K2Args a) {
   for (int g0 = 0; g0 < G - RING; g0 += RING) static_for<RING>([&](auto s) { group(g0 + decltype(s)::value, s, T{}); });
   issue_rope();
   static_for<RING>([&](auto s) { group(G - RING + decltype(s)::value, s, F{}); });
+
+  if constexpr (MANY) {
+    if (a.query_dtype == DKV_F16)
+      many_rows_epilogue<D, NW, DKV_F16>(a, acc, cw, sw, lds, tile, part, n, count, b, h, RH);
+    else if (a.query_dtype == DKV_BF16)
+      many_rows_epilogue<D, NW, DKV_BF16>(a, acc, cw, sw, lds, tile, part, n, count, b, h, RH);
+    else
+      many_rows_epilogue<D, NW, DKV_F32>(a, acc, cw, sw, lds, tile, part, n, count, b, h, RH);
+    return;
+  } else {
 
   // ---- epilogue: RoPE on the lane's dimension pairs (d and d + D/2 sit in the same lane), then the
   // dot with every query row slot (rows past RH are zero) in fp32; the two dimension halves of a
@@ -1465,6 +1621,7 @@ __global__ __launch_bounds__(NW * 64) void keys_scores_head_kernel(K2Args a) {
       const long o = (long)(h * RH + lane) * a.nstats + tp;
       a.tile_max[o] = M;
       a.tile_sum[o] = S;
+      if (o == 0) *a.lines_valid = 0u;
     }
   }
   // probabilities relative to the workgroup's maximum, fp16; every slot of its tokens is written (0
@@ -1476,16 +1633,9 @@ __global__ __launch_bounds__(NW * 64) void keys_scores_head_kernel(K2Args a) {
     const float p = (xs[r] == -INFINITY) ? 0.0f : __expf(xs[r] - Mt[r]);
     a.probs[prob_index((long)h * RH + r, (long)tile * kTileTok + n, a.Hq * a.q_len)] = f16_bits(p);
   }
+  }
 }
 
-// ---------------------------------------------------------------------------
-// Softmax statistics of the compressed part of sequence b, row `row`.
-// ---------------------------------------------------------------------------
-DKV_DEVICE int tiles_before(const int32_t* cu, int b, int tile) {
-  int base = 0;
-  for (int i = 0; i < b; ++i) base += (cu[i + 1] - cu[i] + tile - 1) / tile;
-  return base;
-}
 
 // ---------------------------------------------------------------------------
 // K3c: one workgroup per (sequence, output row).  It merges the tiles'
@@ -1538,8 +1688,7 @@ DKV_DEVICE float4 load_exact4(const void* base, long e) {
 
 template <int XT>
 __device__ void row_exact(const RowMergeArgs& a, int wg, int part, float* smem) {
-  const int lane = threadIdx.x;
-  if (lane >= 64) return;  // one wave
+  const int lane = threadIdx.x & 63;  // one wave
   float* q = smem;          // [128] the query row
   float* se = q + 128;      // [kExactShare] this share's scores, then weights
   const int row = wg % a.R_total;
@@ -1671,7 +1820,8 @@ __device__ void row_exact(const RowMergeArgs& a, int wg, int part, float* smem) 
 //   out = (e_c * (sum of the chunk partials) + e_c * L_c * mean_v + e_e * ve) / (e_c * L_c + e_e * L_e),
 //   e_c = exp(M_c - M), e_e = exp(M_e - M), M = max(M_c, M_e).
 // All its loads (tile statistics, the exact results, the chunk partials, the mean) go out in one round.
-// PER_TILE: softmax-statistics entries per tile (1, or 2 for 128-token entries).
+// PER_TILE: softmax-statistics entries per tile (1, 2 for 128-token entries, or 4: many-row decodes' quarters, in
+// sub_index order).
 template <int NT, int PER_TILE>
 __device__ void row_merge(const RowMergeArgs& a, int wg, float* smem) {
   float* bc = smem;      // [2] the compressed part's (max, sum)
@@ -1689,15 +1839,17 @@ __device__ void row_merge(const RowMergeArgs& a, int wg, float* smem) {
   const int tb0 = tiles_before(a.cu_seqlens, b, kTileTok) * per_tile;
   const int2 sr = seq_range(a.cu_seqlens, a.batch, a.n_total, b);
   const int ntb = (sr.y - sr.x + kTileTok - 1) / kTileTok * per_tile;
-  const float* tm = ntb > 0 ? a.tile_max + (long)row * a.nstats + tb0 : a.mean_v;
-  const float* ts = ntb > 0 ? a.tile_sum + (long)row * a.nstats + tb0 : a.mean_v;
+  constexpr int STEP = PER_TILE == 4 ? 8 : 1;  // floats between a row's entries
+  const long stat0 = PER_TILE == 4 ? sub_index(row, tb0, a.nstats) : (long)row * a.nstats + tb0;
+  const float* tm = ntb > 0 ? a.tile_max + stat0 : a.mean_v;
+  const float* ts = ntb > 0 ? a.tile_sum + stat0 : a.mean_v;
   float m4[4], s4[4];
   if (wave == 0) {
 #pragma unroll
     for (int k = 0; k < 4; ++k) {
       const int t = min(lane + 64 * k, max(ntb - 1, 0));
-      m4[k] = tm[t];
-      s4[k] = ts[t];
+      m4[k] = tm[STEP * t];
+      s4[k] = ts[STEP * t];
     }
   }
   // the exact tail's shares (row_exact): (Me, Le) and ve[d] of each
@@ -1730,7 +1882,7 @@ __device__ void row_merge(const RowMergeArgs& a, int wg, float* smem) {
 #pragma unroll
     for (int k = 0; k < 4; ++k)
       if (lane + 64 * k < ntb) merge(m4[k], s4[k]);
-    for (int t = lane + 256; t < ntb; t += 64) merge(tm[t], ts[t]);
+    for (int t = lane + 256; t < ntb; t += 64) merge(tm[STEP * t], ts[STEP * t]);
     const float m = wave_max(mm);
     const float l = wave_sum(mm == -INFINITY ? 0.0f : ll * __expf(mm - m));
     if (lane == 0) {
@@ -1774,7 +1926,7 @@ struct K3aArgs {
   const uint16_t* probs;  // fp16 exp(score - tile max), [n_slots/16][R][16] (prob_index)
   const float* tile_max;
   float* w_part;
-  // nstats: softmax-statistics entries per row (ntiles, or 2 * ntiles for 128-token entries)
+  // nstats: softmax-statistics entries per row (ntiles; 2 * ntiles for 128-token entries, 4 * ntiles with many rows)
   int batch, R_total, n_total, n_slots, nstats, G, rank, nsplits, row_blocks;
   int total_wg, per_xcd;  // workgroups, and consecutive workgroup indices per XCD
 };
@@ -1787,11 +1939,12 @@ constexpr int kK3WaveTok = 128;  // tokens per K3a wave
 // component, 8 consecutive slots) is one 8-byte load and a wave's 32
 // components of one 16-slot block are 512 contiguous bytes, plus the
 // per-(group, slot) affine form (scale = span / 256, offset = low + span *
-// 2^-(m+1); 0 and 0 for a group without planes or a padding slot).  One block
+// 2^-(m+1); 0 and 0 for a group without planes or a padding slot) and a bound on
+// the values of each (group, 64 slots).  One block
 // = 256 slots x one group, one thread per slot, whose codes are one contiguous
 // 16 KB run; the codes are transposed through LDS.
 // ---------------------------------------------------------------------------
-DKV_DEVICE void decode_values_block(const DecodeArgs& a, uint8_t* vcodes, float2* vaff, int2* tab, int id) {
+DKV_DEVICE void decode_values_block(const DecodeArgs& a, uint8_t* vcodes, float2* vaff, float* vtop, int2* tab, int id) {
   __shared__ uint32_t tile[64][kDecodeSlots / 4 + 1];  // [component][slot / 4], bytes of 4 slots per word
   const int nsb = a.n_slots / kDecodeSlots;
   const int2 bg = decode_block(a.G, nsb * a.G, id);
@@ -1832,6 +1985,10 @@ DKV_DEVICE void decode_values_block(const DecodeArgs& a, uint8_t* vcodes, float2
     aff = make_float2(dq.scale, dq.offset);
   }
   vaff[(long)g * a.n_slots + slot] = aff;
+  // a bound on the group's values in these 64 slots (value_lines); values that are not finite bound nothing
+  const float bound = fmaxf(fabsf(aff.y), fabsf(aff.y + 255.0f * aff.x));
+  const float top = wave_max(bound < INFINITY ? bound : 0.0f);
+  if ((tl & 63) == 0) vtop[(long)g * (a.n_slots / 64) + slot / 64] = top;
   uint8_t* tb8 = (uint8_t*)&tile[0][0];
   constexpr int ROWB = (kDecodeSlots / 4 + 1) * 4;
 #pragma unroll
@@ -1857,12 +2014,14 @@ DKV_DEVICE void decode_values_block(const DecodeArgs& a, uint8_t* vcodes, float2
 // drain and their segment reads overlap the key blocks' operand writes.  Block ids of each part
 // keep the XCD pattern (key_blocks is a multiple of 8).
 __global__ __launch_bounds__(kDecodeSlots) void decode_codes_kernel(DecodeArgs k, DecodeArgs v, uint8_t* vcodes,
-                                                                    float2* vaff, int key_blocks) {
+                                                                    float2* vaff, float* vtop, uint32_t* lines_valid,
+                                                                    int key_blocks) {
   extern __shared__ int2 tab[];
+  if (blockIdx.x == gridDim.x - 1 && threadIdx.x == 0 && lines_valid) *lines_valid = 0u;
   if ((int)blockIdx.x < key_blocks)
     decode_keys_block(k, tab, blockIdx.x);
   else
-    decode_values_block(v, vcodes, vaff, tab, blockIdx.x - key_blocks);
+    decode_values_block(v, vcodes, vaff, vtop, tab, blockIdx.x - key_blocks);
 }
 
 // 8 codes (bytes of lo, hi) -> 8 fp16 values equal to the codes.  (0x6400 | c)
@@ -2077,12 +2236,245 @@ __global__ __launch_bounds__(WAVES * 64) void value_weights_kernel(K3aArgs a) {
 }
 
 // ---------------------------------------------------------------------------
+// K3a for many query rows per KV head (a question's own forward, several new tokens): w[row][k] = sum_t
+// p[row][t] value[t][k] as one fp16 matrix product, rows x tokens by tokens x components, in place of a
+// value_weights workgroup per 32 rows, which each read and converted every code again.
+//
+// Both operands come as 128-byte lines of 64 tokens (operand_line), straight into LDS: the probabilities as K2
+// leaves them, the values as fp16 (code * scale + offset, rounded once), which the first many-row layer after a
+// decode of the codes converts (value_lines) and the others find.  K2's probabilities are relative to a power of
+// two per row and 64 tokens, so taking them to the split's maximum is an exact product in fp16 (down to 2^-28 of
+// the split's maximum), one packed multiply per token pair; the values' own power of two leaves with the sums.
+//
+// A workgroup takes 64 MW rows x 256 components over a split of the tokens, 64 tokens a stage; wave (wm, wn) of
+// the MW x 8 / MW takes 64 rows x 32 MW components.  The pipeline is gemm_split_kernel's: the operands of a 16-token
+// step are read while the step before is multiplied, and the stage's barrier stands before its last step, when the
+// next stage has landed.  1,536 rows x 16,348 tokens x 2,048 components: 106 us, 0.97 PFLOP/s (value_weights took
+// 324), bound by the LDS reads of its operands beside the products; converting the codes here instead, with the
+// pairs of each token read from LDS, took 194.  416 rows x 2,965 tokens x 1,024: 12 us against 20, latency.
+//
+// Error against float64: the values' rounding to fp16 (2^-12 relative) takes the place of that of probability x scale,
+// and the sums below the line are of the fp16 probabilities; with K2's two-piece keys the outputs' distance from
+// float64 went from 5.3e-4 to 4.8e-4 (13 query tokens, fp16 out) and from 1.754e-3 to 1.743e-3 (64, bf16 out).
+// ---------------------------------------------------------------------------
+struct K3RowsArgs {
+  const uint8_t* probs;   // operand lines [rows][slots] (K2)
+  const uint8_t* values;  // operand lines [components][slots] (value_lines)
+  uint32_t* lines_valid;  // set: the values are there for the next layers
+  const int* lines_exp;   // the power of two in each (group, 64 slots) of them, one over a sequence
+  const float* sub_max;   // [R][nsub] (sub_index): the power of two of each row and 64 tokens, as its logarithm
+  const int32_t* cu_seqlens;
+  float* w_part;          // [nsplits][R_total][rank], relative to the split's maximum
+  float* split_max;       // [nsplits][R_total]
+  int batch, n_total, n_slots, R_total, nsub, rank, split_tok, mt, nt, total_wg, per_xcd;
+};
+
+constexpr int kRowsCols = 256;  // components per workgroup
+constexpr int kRowsStage = 64;  // tokens per stage
+
+// 2^(k + kRowsUp) for a difference k ln 2 <= 0 of two entries of sub_max, as a packed fp16 pair (0 for empty entries):
+// a probability of 2^-28 of the split's maximum is then still a normal fp16 number.
+constexpr int kRowsUp = 14;
+DKV_DEVICE uint32_t pow2_pair(float m, float M) {
+  const float f = m == -INFINITY ? 0.0f : __builtin_ldexpf(1.0f, kRowsUp + (int)rintf((m - M) * 1.44269504f));
+  const uint32_t h = f16_bits(f);
+  return h | h << 16;
+}
+
+template <int MW>
+__global__ __launch_bounds__(512, 2) void value_rows_kernel(K3RowsArgs a) {
+  constexpr int MT = 64 * MW;         // rows
+  constexpr int JB = MW;              // 32-component blocks per wave
+  constexpr int ABYTES = MT * 128;    // a stage of probabilities
+  constexpr int BBYTES = kRowsCols * 128;
+  constexpr int ACH = MW;             // 1 KB copies per wave and stage: probabilities
+  constexpr int BCH = 4;              // ... values
+  __shared__ __attribute__((aligned(1024))) uint8_t S0[ABYTES + BBYTES];
+  __shared__ __attribute__((aligned(1024))) uint8_t S1[ABYTES + BBYTES];
+  __shared__ float rmax[512 / MT][MT];
+
+  if (blockIdx.x == 0 && threadIdx.x == 0) *a.lines_valid = 1u;
+  const int lin = (blockIdx.x & 7) * a.per_xcd + (blockIdx.x >> 3);
+  if (lin >= a.total_wg) return;
+  const int tn = lin % a.nt, tm = (lin / a.nt) % a.mt, sp = lin / (a.nt * a.mt);
+  const int2 bs = find_tile(a.cu_seqlens, a.batch, a.n_total, a.split_tok, sp);
+  const int2 sr = seq_range(a.cu_seqlens, a.batch, a.n_total, bs.x);
+  const int len = min(a.split_tok, sr.y - sr.x - bs.y * a.split_tok);
+  const int stages = (len + kTileTok - 1) / kTileTok * (kTileTok / kRowsStage);  // whole tiles: a multiple of 4
+  const int slot0 = tiles_before(a.cu_seqlens, bs.x, kTileTok) * kTileTok + bs.y * a.split_tok;
+  const int e0 = slot0 / kRowsStage;  // the split's first statistics entry, and its first 64-slot block
+  const int NTB = a.n_slots / kRowsStage;
+
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wm = wave % MW, wn = wave / MW;
+  const int l32 = lane & 31, lhi = lane >> 5;
+  const uint32_t lane16 = lane * 16;
+
+  // a stage's lines: 1 KB pieces wave * ACH .. of the rows' 4 KB blocks, wave * BCH .. of the components'
+  auto copy = [&](int s, uint8_t* S) {
+#pragma unroll
+    for (int i = 0; i < ACH; ++i) {
+      const int ch = wave * ACH + i;
+      const uint8_t* src = a.probs + ((long)(tm * (MT / 32) + (ch >> 2)) * NTB + e0 + s) * 4096 + (ch & 3) * 1024;
+      __builtin_amdgcn_global_load_lds(src + lane16, S + ch * 1024, 16, 0, 0);
+    }
+#pragma unroll
+    for (int i = 0; i < BCH; ++i) {
+      const uint8_t* src = a.values + ((long)(tn * (kRowsCols / 32) + wave) * NTB + e0 + s) * 4096 + i * 1024;
+      __builtin_amdgcn_global_load_lds(src + lane16, S + ABYTES + wave * 4096 + i * 1024, 16, 0, 0);
+    }
+  };
+  int vexp[(JB + 1) / 2];
+#pragma unroll
+  for (int j = 0; j < JB; j += 2) vexp[j / 2] = a.lines_exp[(long)((tn * kRowsCols + (wn * JB + j) * 32) / 64) * NTB + e0];
+  const int myrow[2] = {tm * MT + wm * 64 + l32, tm * MT + wm * 64 + 32 + l32};
+  const float* mptr[2];
+#pragma unroll
+  for (int i = 0; i < 2; ++i) mptr[i] = a.sub_max + sub_index(min(myrow[i], a.R_total - 1), e0, a.nsub);
+
+  floatx16 acc[2][JB];
+#pragma unroll
+  for (int i = 0; i < 2; ++i)
+#pragma unroll
+    for (int j = 0; j < JB; ++j)
+#pragma unroll
+      for (int v = 0; v < 16; ++v) acc[i][j][v] = 0.0f;
+
+  // first round: two stages (a split has at least four), and the rows' maxima over the split by 512 / MT threads each
+  copy(0, S0);
+  copy(1, S1);
+  float m0[2], m1[2];
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    m0[i] = mptr[i][0];
+    m1[i] = mptr[i][8];
+  }
+  {
+    constexpr int PARTS = 512 / MT;
+    const int r = tid % MT, part = tid / MT;
+    const float* src = a.sub_max + sub_index(min(tm * MT + r, a.R_total - 1), e0, a.nsub);
+    float m = -INFINITY;
+#pragma unroll 4
+    for (int e = part; e < stages; e += PARTS) m = fmaxf(m, src[8 * e]);
+    rmax[part][r] = m;
+  }
+  __syncthreads();  // drains the copies too
+  float M[2];
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    M[i] = -INFINITY;
+#pragma unroll
+    for (int p = 0; p < 512 / MT; ++p) M[i] = fmaxf(M[i], rmax[p][wm * 64 + i * 32 + l32]);
+  }
+
+  struct Operands {
+    half8 a[2], b[JB];
+  };
+  const int p0 = lhi ^ (l32 & 7);
+  const int arow = (wm * 64 + l32) * 128, brow = ABYTES + (wn * 32 * JB + l32) * 128;
+  auto read = [&](const uint8_t* S, int step, Operands& f) {
+    const int off = (p0 ^ (step * 2)) << 4;
+#pragma unroll
+    for (int i = 0; i < 2; ++i) f.a[i] = *(const half8*)(S + arow + off + i * 4096);
+#pragma unroll
+    for (int j = 0; j < JB; ++j) f.b[j] = *(const half8*)(S + brow + off + j * 4096);
+  };
+  uint32_t fac[2];  // 2^k of the rows' 64 tokens, as fp16 pairs
+  auto multiply = [&](const Operands& f) {
+    half8 pa[2];
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      typedef _Float16 half2_t __attribute__((ext_vector_type(2)));
+      const half2_t k2 = __builtin_bit_cast(half2_t, fac[i]);
+      const half8 k8 = {k2[0], k2[1], k2[0], k2[1], k2[0], k2[1], k2[0], k2[1]};
+      pa[i] = f.a[i] * k8;
+    }
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+      for (int j = 0; j < JB; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(pa[i], f.b[j], acc[i][j], 0, 0, 0);
+  };
+  auto meet = [&]() {
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_waitcnt(0x0070);  // vmcnt(0) lgkmcnt(0)
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+  };
+  // one step per scheduling region: the next step's reads (and the copies) between the products
+  auto spread = [&](auto reads_t, auto copies_t) {
+    static_for<2 * JB>([&](auto ii) {
+      constexpr int i = decltype(ii)::value, MF = 2 * JB;
+      constexpr int RD = decltype(reads_t)::value ? 2 + JB : 0, CP = decltype(copies_t)::value ? ACH + BCH : 0;
+      constexpr int rd = RD * (i + 1) / MF - RD * i / MF, cp = CP * (i + 1) / MF - CP * i / MF;
+      __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+      if constexpr (rd > 0) __builtin_amdgcn_sched_group_barrier(0x100, rd, 0);
+      if constexpr (cp > 0) __builtin_amdgcn_sched_group_barrier(0x010, cp, 0);
+    });
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  using T = std::true_type;
+  using F = std::false_type;
+  Operands f0, f1;
+  // Stage s.  In: f0 holds its step 0, mc its rows' entries; Sn is the other buffer.  COPY: stage s + 2 exists.
+  auto stage = [&](int s, uint8_t* S, uint8_t* Sn, float (&mc)[2], auto copy_t, auto next_t) {
+    constexpr bool COPY = decltype(copy_t)::value, NEXT = decltype(next_t)::value;
+#pragma unroll
+    for (int i = 0; i < 2; ++i) fac[i] = pow2_pair(mc[i], M[i]);
+    read(S, 1, f1);
+    multiply(f0);
+    spread(T{}, F{});
+    read(S, 2, f0);
+    multiply(f1);
+    spread(T{}, F{});
+    read(S, 3, f1);
+    multiply(f0);
+    spread(T{}, F{});
+    meet();
+    __builtin_amdgcn_sched_barrier(0);
+    if constexpr (COPY) {
+#pragma unroll
+      for (int i = 0; i < 2; ++i) mc[i] = mptr[i][8 * (s + 2)];
+      copy(s + 2, S);
+    }
+    if constexpr (NEXT) read(Sn, 0, f0);
+    multiply(f1);
+    spread(next_t, copy_t);
+  };
+  read(S0, 0, f0);
+  int s = 0;
+  for (; s + 2 < stages; s += 2) {
+    stage(s, S0, S1, m0, T{}, T{});
+    stage(s + 1, S1, S0, m1, T{}, T{});
+  }
+  stage(s, S0, S1, m0, F{}, T{});
+  stage(s + 1, S1, S0, m1, F{}, F{});
+
+  // acc[i][j][v]: row wm * 64 + i * 32 + 8 (v / 4) + 4 lhi + (v & 3) of the tile, component wn * 32 JB + j * 32 + l32
+  float* w = a.w_part + (long)sp * a.R_total * a.rank + tn * kRowsCols + wn * 32 * JB + l32;
+#pragma unroll
+  for (int i = 0; i < 2; ++i)
+#pragma unroll
+    for (int v = 0; v < 16; ++v) {
+      const int row = tm * MT + wm * 64 + i * 32 + 8 * (v >> 2) + 4 * lhi + (v & 3);
+      if (row >= a.R_total) continue;
+#pragma unroll
+      for (int j = 0; j < JB; ++j) w[(long)row * a.rank + j * 32] = __builtin_ldexpf(acc[i][j][v], -kRowsUp - vexp[j / 2]);
+    }
+  if (tn == 0 && wn == 0 && lhi == 0) {
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+      if (myrow[i] < a.R_total) a.split_max[(long)sp * a.R_total + myrow[i]] = M[i];
+  }
+}
+
+// ---------------------------------------------------------------------------
 // K3b: one workgroup per (sequence, KV head, 128-component chunk, 64-dimension
 // slice): sum the head's value partials over the sequence's splits, multiply
 // once by the value-basis block [128 components][64 dimensions].  Thread
 // (dp, part) holds dimension pair dp of the slice for components part * 16
-// .. +16; the head's rows go in passes of NR (4 covers a decoding step's rows:
-// GQA group x q_len <= 4).
+// .. +16; NR = 4 covers a decoding step's rows (GQA group x q_len <= 4; more go to
+// basis_rows_kernel).
 // ---------------------------------------------------------------------------
 struct K3bArgs {
   const int32_t* cu_seqlens;
@@ -2099,15 +2491,16 @@ constexpr int kK3bComp = kChunk / kK3bParts;  // 16 components per thread
 constexpr int kK3bDims = 64;                  // dimensions per workgroup
 
 // (at most two waves per SIMD: the exact-tail role's registers are not capped for occupancy)
-template <int NR, int XT>
+template <int XT>
 __global__ __launch_bounds__(kRowThreads) __attribute__((amdgpu_waves_per_eu(1, 2)))
 void basis_apply_kernel(K3bArgs a, RowMergeArgs ex) {
   if ((int)blockIdx.x < a.n_exact_wg) {  // share blockIdx.x % kExactParts of output row blockIdx.x / kExactParts
     __shared__ __attribute__((aligned(16))) float xsm[kExactLds];
-    row_exact<XT>(ex, blockIdx.x / kExactParts, blockIdx.x % kExactParts, xsm);
+    if (threadIdx.x < 64) row_exact<XT>(ex, blockIdx.x / kExactParts, blockIdx.x % kExactParts, xsm);
     return;
   }
-  __shared__ __attribute__((aligned(16))) float W[NR][kChunk];  // the pass's summed weights
+  constexpr int NR = kSmallRows;
+  __shared__ __attribute__((aligned(16))) float W[NR][kChunk];  // the head's summed weights
   __shared__ float red[kK3bParts][NR][kK3bDims + 2];             // per-part outputs
   const int nds = a.D / kK3bDims;
   const int bid = blockIdx.x - a.n_exact_wg;
@@ -2132,71 +2525,236 @@ void basis_apply_kernel(K3bArgs a, RowMergeArgs ex) {
   for (int ii = 0; ii < kK3bComp; ++ii) bw[ii] = bv[(long)ii * npair];
   const long sp_stride4 = (long)a.R_total * a.rank / 4;  // split stride in float4 units
   const int rr = tid >> 5, k4 = tid & 31;                // the W element of this thread: row rr, components 4 k4 ..
-  // one pass over rows r0 .. r0 + NR - 1 (the first pass is not inside the loop: hoisted out of a
-  // loop, the basis conversions below would wait for the basis loads before the split loads go out)
-  auto pass = [&](int r0) {
-    const int nr = min(NR, RH - r0);
-    // W[rr][4 k4 ..] = sum over the sequence's splits, in split order (16 loads per batch in flight)
-    if (rr < nr) {
-      const float4* src = (const float4*)(a.w_part + ((long)sp0 * a.R_total + (long)h * RH + r0 + rr) * a.rank +
-                                          (long)c * kChunk) + k4;
-      float4 sum = make_float4(0.f, 0.f, 0.f, 0.f);
-      for (int s0 = 0; s0 < nsp; s0 += 16) {
-        float4 v[16];
+  // W[rr][4 k4 ..] = sum over the sequence's splits, in split order (16 loads per batch in flight)
+  if (rr < RH) {
+    const float4* src = (const float4*)(a.w_part + ((long)sp0 * a.R_total + (long)h * RH + rr) * a.rank +
+                                        (long)c * kChunk) + k4;
+    float4 sum = make_float4(0.f, 0.f, 0.f, 0.f);
+    for (int s0 = 0; s0 < nsp; s0 += 16) {
+      float4 v[16];
 #pragma unroll
-        for (int k = 0; k < 16; ++k) v[k] = src[(long)min(s0 + k, nsp - 1) * sp_stride4];
+      for (int k = 0; k < 16; ++k) v[k] = src[(long)min(s0 + k, nsp - 1) * sp_stride4];
 #pragma unroll
-        for (int k = 0; k < 16; ++k) {  // past the last split the (finite) repeat is added as exactly 0
-          const float keep = s0 + k < nsp ? 1.0f : 0.0f;
-          sum.x += v[k].x * keep;
-          sum.y += v[k].y * keep;
-          sum.z += v[k].z * keep;
-          sum.w += v[k].w * keep;
-        }
-      }
-      *(float4*)&W[rr][4 * k4] = sum;
-    }
-    __syncthreads();
-    // rows nr .. NR - 1 of W hold stale values; their sums are computed and never stored
-    float acc0[NR], acc1[NR];
-#pragma unroll
-    for (int r = 0; r < NR; ++r) acc0[r] = acc1[r] = 0.0f;
-#pragma unroll
-    for (int q = 0; q < kK3bComp / 4; ++q) {
-      float4 w4[NR];
-#pragma unroll
-      for (int r = 0; r < NR; ++r) w4[r] = *(const float4*)&W[r][part * kK3bComp + 4 * q];
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const uint32_t bb = bw[4 * q + e];
-        const float b0 = half_bits_to_float((uint16_t)(bb & 0xffffu));
-        const float b1 = half_bits_to_float((uint16_t)(bb >> 16));
-#pragma unroll
-        for (int r = 0; r < NR; ++r) {
-          const float wv = e == 0 ? w4[r].x : e == 1 ? w4[r].y : e == 2 ? w4[r].z : w4[r].w;
-          acc0[r] += wv * b0;
-          acc1[r] += wv * b1;
-        }
+      for (int k = 0; k < 16; ++k) {  // past the last split the (finite) repeat is added as exactly 0
+        const float keep = s0 + k < nsp ? 1.0f : 0.0f;
+        sum.x += v[k].x * keep;
+        sum.y += v[k].y * keep;
+        sum.z += v[k].z * keep;
+        sum.w += v[k].w * keep;
       }
     }
+    *(float4*)&W[rr][4 * k4] = sum;
+  }
+  __syncthreads();
+  // rows RH .. NR - 1 of W hold nothing; their sums are computed and never stored
+  float acc0[NR], acc1[NR];
 #pragma unroll
-    for (int r = 0; r < NR; ++r) {
-      red[part][r][2 * dp] = acc0[r];
-      red[part][r][2 * dp + 1] = acc1[r];
+  for (int r = 0; r < NR; ++r) acc0[r] = acc1[r] = 0.0f;
+#pragma unroll
+  for (int q = 0; q < kK3bComp / 4; ++q) {
+    float4 w4[NR];
+#pragma unroll
+    for (int r = 0; r < NR; ++r) w4[r] = *(const float4*)&W[r][part * kK3bComp + 4 * q];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const uint32_t bb = bw[4 * q + e];
+      const float b0 = half_bits_to_float((uint16_t)(bb & 0xffffu));
+      const float b1 = half_bits_to_float((uint16_t)(bb >> 16));
+#pragma unroll
+      for (int r = 0; r < NR; ++r) {
+        const float wv = e == 0 ? w4[r].x : e == 1 ? w4[r].y : e == 2 ? w4[r].z : w4[r].w;
+        acc0[r] += wv * b0;
+        acc1[r] += wv * b1;
+      }
+    }
+  }
+#pragma unroll
+  for (int r = 0; r < NR; ++r) {
+    red[part][r][2 * dp] = acc0[r];
+    red[part][r][2 * dp + 1] = acc1[r];
+  }
+  __syncthreads();
+  for (int e = tid; e < RH * kK3bDims; e += 256) {
+    const int r = e / kK3bDims, dd = e % kK3bDims;
+    float s = 0.0f;
+#pragma unroll
+    for (int p = 0; p < kK3bParts; ++p) s += red[p][r][dd];
+    a.out_part[(((long)c * a.batch + b) * a.R_total + (long)h * RH + r) * D + ds * kK3bDims + dd] = s;
+  }
+}
+
+// ---------------------------------------------------------------------------
+// K3b for many rows per KV head: one workgroup per (sequence, KV head, 32 rows, 128-component chunk).  The rows'
+// value partials are summed over the splits (each brought from its split's maximum to the row's by a power of two;
+// the loads of two splits in flight, which measured 31 us against 38 with four and 33 with one at 1,536 rows, rank
+// 2048 and 5 splits, a 63 MB read), split into two fp16 pieces per weight (22 bits; the basis is fp16 already) and
+// multiplied by the basis chunk on MFMA.  The basis chunk is turned in LDS: [dimension][component],
+// 16-byte pieces swizzled by dimension / 8.  The exact tail runs in the leading workgroups, one per output row,
+// a share of its tokens per wave.  The few-row kernel, a 64-dimension slice per workgroup in fp32, took 102 us there;
+// at 416 rows and rank 1024 9 us against 15.
+// ---------------------------------------------------------------------------
+struct K3bRowsArgs {
+  const int32_t* cu_seqlens;
+  const float* w_part;
+  const float* split_max;
+  const uint16_t* value_basis;
+  float* out_part;
+  int batch, n_total, layer, Hkv, RH, rank, R_total, nchunks, split_tok, row_blocks, n_exact_wg;
+};
+
+constexpr int kBasisRows = 32;  // rows per workgroup
+
+template <int D, int XT>
+__global__ __launch_bounds__(256) void basis_rows_kernel(K3bRowsArgs a, RowMergeArgs ex) {
+  constexpr int RB = kBasisRows;
+  constexpr int WSTR = kChunk + 8;    // halves per staged row
+  __shared__ __attribute__((aligned(16))) half_t Wl[2][RB][WSTR];  // the weights' hi and lo pieces
+  __shared__ __attribute__((aligned(16))) half_t BT[D][WSTR];
+  __shared__ int rshift[RB];
+  static_assert(sizeof(BT) >= 4 * kExactLds * sizeof(float), "the exact tail's staging");
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  if ((int)blockIdx.x < a.n_exact_wg) {
+    static_assert(kExactParts == 4, "one wave per share");
+    row_exact<XT>(ex, blockIdx.x, wave, (float*)&BT[0][0] + wave * kExactLds);
+    return;
+  }
+  const int bid = blockIdx.x - a.n_exact_wg;
+  const int c = bid % a.nchunks;
+  const int rb = (bid / a.nchunks) % a.row_blocks;
+  const int h = (bid / (a.nchunks * a.row_blocks)) % a.Hkv;
+  const int b = bid / (a.nchunks * a.row_blocks * a.Hkv);
+  const int l32 = lane & 31, lhi = lane >> 5;
+  const int sp0 = tiles_before(a.cu_seqlens, b, a.split_tok);
+  const int2 sr = seq_range(a.cu_seqlens, a.batch, a.n_total, b);
+  const int nsp = (sr.y - sr.x + a.split_tok - 1) / a.split_tok;
+  // the basis chunk: lane (o = lane % OCT, kp) holds dimensions 8 o .. of components 2 kp and 2 kp + 1
+  constexpr int OCT = D / 8;
+  constexpr int BI = kChunk / 2 * OCT / 256;  // 4 (D = 128) or 2
+  const uint16_t* bv = a.value_basis + (((long)a.layer * a.Hkv + h) * a.rank + (long)c * kChunk) * D;
+  uint4 b0[BI], b1[BI];
+#pragma unroll
+  for (int i = 0; i < BI; ++i) {
+    const int e = tid + 256 * i, o = e % OCT, kp = e / OCT;
+    b0[i] = *(const uint4*)(bv + (2 * kp) * D + 8 * o);
+    b1[i] = *(const uint4*)(bv + (2 * kp + 1) * D + 8 * o);
+  }
+  // this thread's weights: rows r8 + 8 p, components 4 k4 ..
+  constexpr int P = RB / 8;
+  const int r8 = tid >> 5, k4 = tid & 31;
+  const float* mp[P];
+  const float4* wp[P];
+  float M[P];
+  float4 w[P];
+#pragma unroll
+  for (int p = 0; p < P; ++p) {
+    const long row = (long)h * a.RH + min(rb * RB + r8 + 8 * p, a.RH - 1);  // rows past the end repeat the last; never stored
+    mp[p] = a.split_max + (long)sp0 * a.R_total + row;
+    wp[p] = (const float4*)(a.w_part + ((long)sp0 * a.R_total + row) * a.rank + (long)c * kChunk) + k4;
+    M[p] = -INFINITY;
+    w[p] = make_float4(0.f, 0.f, 0.f, 0.f);
+  }
+  const long wstep = (long)a.R_total * a.rank / 4;
+  constexpr int SB = 2;  // splits whose loads go out together
+  for (int s0 = 0; s0 < nsp; s0 += SB) {
+    float m[SB][P];
+    float4 v[SB][P];
+#pragma unroll
+    for (int k = 0; k < SB; ++k) {
+      const int s = min(s0 + k, nsp - 1);
+#pragma unroll
+      for (int p = 0; p < P; ++p) {
+        m[k][p] = mp[p][(long)s * a.R_total];
+        v[k][p] = wp[p][s * wstep];
+      }
+    }
+#pragma unroll
+    for (int p = 0; p < P; ++p) {
+      // powers of two: the running sum, then each split, to the larger maximum
+      float top = M[p];
+#pragma unroll
+      for (int k = 0; k < SB; ++k) top = fmaxf(top, m[k][p]);
+      auto scale = [&](float from) {
+        return from == -INFINITY ? 0.0f : __builtin_ldexpf(1.0f, (int)rintf((from - top) * 1.44269504f));
+      };
+      const float f0 = scale(M[p]);
+      w[p].x *= f0;
+      w[p].y *= f0;
+      w[p].z *= f0;
+      w[p].w *= f0;
+#pragma unroll
+      for (int k = 0; k < SB; ++k) {
+        const float f = s0 + k < nsp ? scale(m[k][p]) : 0.0f;
+        w[p].x += v[k][p].x * f;
+        w[p].y += v[k][p].y * f;
+        w[p].z += v[k][p].z * f;
+        w[p].w += v[k][p].w * f;
+      }
+      M[p] = top;
+    }
+  }
+#pragma unroll
+  for (int p = 0; p < P; ++p) {
+    // a power of two that takes the row's largest weight of the chunk to [2^14, 2^15), exactly undone at the end
+    const float top = max32(fmaxf(fmaxf(fabsf(w[p].x), fabsf(w[p].y)), fmaxf(fabsf(w[p].z), fabsf(w[p].w))));
+    int e = 0;
+    if (top > 0.0f && top < INFINITY) (void)frexpf(top, &e);
+    const int shift = 15 - e;
+    const float x[4] = {w[p].x, w[p].y, w[p].z, w[p].w};
+    half4 hi, lo;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const float v = __builtin_ldexpf(x[i], shift);
+      hi[i] = (half_t)v;
+      lo[i] = (half_t)(v - (float)hi[i]);
+    }
+    *(half4*)&Wl[0][r8 + 8 * p][4 * k4] = hi;
+    *(half4*)&Wl[1][r8 + 8 * p][4 * k4] = lo;
+    if (k4 == 0) rshift[r8 + 8 * p] = shift;
+  }
+#pragma unroll
+  for (int i = 0; i < BI; ++i) {
+    const int e = tid + 256 * i, o = e % OCT, kp = e / OCT;
+    const uint32_t w0[4] = {b0[i].x, b0[i].y, b0[i].z, b0[i].w}, w1[4] = {b1[i].x, b1[i].y, b1[i].z, b1[i].w};
+#pragma unroll
+    for (int d = 0; d < 8; ++d) {
+      const uint32_t lo = (w0[d >> 1] >> (16 * (d & 1))) & 0xffffu, hi = w1[d >> 1] >> (16 * (d & 1)) << 16;
+      *(uint32_t*)&BT[8 * o + d][(((kp >> 2) ^ (o & 15)) << 3) + 2 * (kp & 3)] = lo | hi;
+    }
+  }
+  __syncthreads();
+  // wave: 32 dimensions (block wd); at D = 64 the two waves of a block take half the components each
+  constexpr int DBLK = D / 32, KP = 4 / DBLK;
+  const int wd = wave % DBLK, kp = wave / DBLK;
+  floatx16 acc;
+#pragma unroll
+  for (int v = 0; v < 16; ++v) acc[v] = 0.0f;
+#pragma unroll
+  for (int i = 0; i < kChunk / 16 / KP; ++i) {
+    const int dim = wd * 32 + l32, oct = (kp * (kChunk / 16 / KP) + i) * 2 + lhi;
+    const half8 bt = *(const half8*)&BT[dim][(oct ^ ((dim >> 3) & 15)) << 3];
+    const half8 wlo = *(const half8*)&Wl[1][l32][oct * 8];
+    const half8 whi = *(const half8*)&Wl[0][l32][oct * 8];
+    acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(wlo, bt, acc, 0, 0, 0);
+    acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(whi, bt, acc, 0, 0, 0);
+  }
+  if constexpr (KP == 2) {
+    __syncthreads();  // every wave has read BT
+    float* half = (float*)&BT[0][0] + wd * 16 * 64 + lane;
+    if (kp == 1) {
+#pragma unroll
+      for (int v = 0; v < 16; ++v) half[v * 64] = acc[v];
     }
     __syncthreads();
-    for (int e = tid; e < nr * kK3bDims; e += 256) {
-      const int r = e / kK3bDims, dd = e % kK3bDims;
-      float s = 0.0f;
+    if (kp == 1) return;
 #pragma unroll
-      for (int p = 0; p < kK3bParts; ++p) s += red[p][r][dd];
-      a.out_part[(((long)c * a.batch + b) * a.R_total + (long)h * RH + r0 + r) * D + ds * kK3bDims + dd] = s;
-    }
-  };
-  pass(0);
-  for (int r0 = NR; r0 < RH; r0 += NR) {
-    __syncthreads();  // W and red are reused
-    pass(r0);
+    for (int v = 0; v < 16; ++v) acc[v] += half[v * 64];
+  }
+#pragma unroll
+  for (int v = 0; v < 16; ++v) {
+    const int rl = 8 * (v >> 2) + 4 * lhi + (v & 3);
+    if (rb * RB + rl >= a.RH) continue;
+    a.out_part[(((long)c * a.batch + b) * a.R_total + (long)h * a.RH + rb * RB + rl) * D + wd * 32 + l32] =
+        __builtin_ldexpf(acc[v], -rshift[rl]);
   }
 }
 
@@ -2211,8 +2769,10 @@ __global__ __launch_bounds__(kRowThreads) void finish_kernel(RowMergeArgs a) {
 // ---------------------------------------------------------------------------
 struct Layout {
   int ntiles, nsplits, split_tok, R_total, nchunks, n_total, n_slots;
-  int stat_tok, nstats;  // tokens per softmax-statistics entry (256, or 128 with K2's half-tile workgroups), entries per row
-  size_t coef, vcodes, vaff, probs, tile_max, tile_sum, w_part, out_part, exact, total;
+  int stat_tok, nstats;  // tokens per softmax-statistics entry (256, 128 with K2's half-tile workgroups, 64 with many rows), entries per row
+  int rows_mw;           // many-row decodes: value_rows_kernel's MW (64 rows each per workgroup); 0 otherwise
+  size_t noalloc_total;  // the size by which dkv_attend_layer_noalloc takes or refuses a context
+  size_t coef, vcodes, vaff, valid, vtop, lines, lines_exp, probs, tile_max, tile_sum, w_part, split_max, out_part, exact, total;
 };
 
 inline size_t align256(size_t x) { return (x + 255) & ~(size_t)255; }
@@ -2236,7 +2796,26 @@ inline int k2_head_tokens(const dkv_attend_args_t* a, int ntiles) {
   return k2_head_form(a, ntiles) && 2L * ntiles * a->kv_heads <= kCUs ? kTileTok / 2 : kTileTok;
 }
 
-// Workspace: [decoded key coefficients][decoded value codes][value affine][probabilities][tile statistics]
+// Waves (32 tokens each) per K2 workgroup of a many-row decode, 128 basis rows each, or 0 for the 256-row kernel.  A CU
+// holds one workgroup, so the smallest form that still runs in one round is taken: quarter tiles up to a quarter of
+// the CUs, half tiles up to half of them, whole tiles up to all of them, and past that the 256-row kernel, which reads
+// a third fewer bytes from LDS per product.  A layer, us, of quarter / half / whole tiles / 256 rows: 5 query
+// tokens (D = 128, rank 2048) at 1,500 tokens 40.8 / 42.3 / 52.2 / 72.3, at 3,900 (all 256 CUs with half
+// tiles) 50.5 / 47.8 / 56.9 / 76.1, at 6,000 74.6 / 70.8 / 62.4 / 81.3, at 8,300 98 / 97 / 100 / 87, and with 64 query
+// tokens at 6,000 142.7 / 140.1 / 127.2 / 149.2, at 8,300 186 / 185 / 183 / 164, at 16,384 272 / 267 / 245 / 230.
+inline int k2_rows_waves(const dkv_attend_args_t* a, int ntiles) {
+  const long tile_heads = (long)ntiles * a->kv_heads * a->head_dim / 128;  // workgroups of a whole tile
+  if (tile_heads > kCUs) return 0;
+  return 2 * tile_heads > kCUs ? 8 : 4 * tile_heads > kCUs ? 4 : 2;
+}
+
+// value_rows_kernel's cost, us: a tile (four stages) of 256, 128 and 64 rows, what a workgroup spends besides, and a
+// megabyte of partial sums (written here, read by basis_rows_kernel).  Fitted to sweeps of both heights' splits over
+// 48 to 3,200 rows and 1,100 to 16,400 tokens: the layer of the choice takes at most 3 % longer than the best one's.
+constexpr double kRowsTile4 = 6.0, kRowsTile2 = 3.2, kRowsTile1 = 2.4, kRowsFixed = 8.0, kRowsPartialMB = 0.1;
+
+// Workspace: [decoded key coefficients][decoded value codes][value affine][one word, and with many rows the value
+// lines][probabilities][tile statistics]
 // [split partials][chunk partials][exact-tail results].
 // The decoded areas are indexed by token slot (256 per tile, see slot_token).
 // `values` false: no value-decode areas (question scoring decodes and reads the keys alone), so
@@ -2262,7 +2841,35 @@ Layout make_layout(const dkv_attend_args_t* a, bool values = true) {
   L.n_slots = L.ntiles * kTileTok + kSplitTok;
   L.nchunks = a->rank / kChunk;
   L.stat_tok = k2_head_tokens(a, L.ntiles);
+  const int fixed_splits = L.nsplits;
+  int prob_rows = L.R_total, stat_rows = L.R_total;
+  if (values && L.R_total / a->kv_heads > kSmallRows) {
+    // many rows: the workgroup height and the splits (whole tiles, at least two) that take the least time by the
+    // measured stage costs: the rounds of one workgroup per CU, each its stages and a prologue
+    double least = 1e300;
+    for (int mw = 1; mw <= 4; mw *= 2) {
+      const long per_split = (long)((L.R_total + 64 * mw - 1) / (64 * mw)) * (a->rank / kRowsCols);
+      const double tile_us = mw == 4 ? kRowsTile4 : mw == 2 ? kRowsTile2 : kRowsTile1;
+      for (int st = 2; st <= std::max(2, L.ntiles); ++st) {
+        const int splits = count_splits(st * kTileTok);
+        const long rounds = (per_split * splits + kCUs - 1) / kCUs;
+        const double cost = rounds * (st * tile_us + kRowsFixed) + kRowsPartialMB * 4e-6 * splits * L.R_total * a->rank;
+        if (cost < least * 0.999) {
+          least = cost;
+          L.rows_mw = mw;
+          L.split_tok = st * kTileTok;
+        }
+      }
+    }
+    const int mt = (L.R_total + 64 * L.rows_mw - 1) / (64 * L.rows_mw);
+    L.nsplits = count_splits(L.split_tok);
+    L.stat_tok = kRowsStage;
+    prob_rows = mt * 64 * L.rows_mw;
+    stat_rows = (L.R_total + 7) / 8 * 8;
+  }
   L.nstats = L.ntiles * (kTileTok / L.stat_tok);
+  const size_t exact_bytes = align256((size_t)a->batch * L.R_total * kExactParts * (a->head_dim + 2) * 4);
+  const size_t out_part_bytes = align256((size_t)L.nchunks * a->batch * L.R_total * a->head_dim * 4);
   size_t off = 0;
   L.coef = off;
   off += align256((size_t)L.n_slots * a->rank * 2);
@@ -2270,19 +2877,37 @@ Layout make_layout(const dkv_attend_args_t* a, bool values = true) {
   if (values) off += align256((size_t)L.n_slots * a->rank);
   L.vaff = off;
   if (values) off += align256((size_t)L.n_slots * (a->rank / 64) * 8);
+  L.noalloc_total = off;
+  const size_t block_bytes = align256((size_t)(a->rank / 64) * (L.n_slots / 64) * 4);  // a word per (group, 64 slots)
+  L.valid = off;  // one word: the lines hold this decode's values
+  if (values) off += 256;
+  L.vtop = off;
+  if (values) off += block_bytes;
+  const size_t decode_bytes = off;
+  L.lines = off;
+  if (L.rows_mw) off += align256((size_t)L.n_slots * a->rank * 2);
+  L.lines_exp = off;
+  if (L.rows_mw) off += block_bytes;
   L.probs = off;
-  off += align256((size_t)L.R_total * L.n_slots * 2);
+  // a many-row decode is taken by its size without the lines, with one statistics entry per tile, unpadded rows and fixed splits
+  if (L.rows_mw)
+    L.noalloc_total += align256((size_t)L.R_total * L.n_slots * 2) + 2 * align256((size_t)L.R_total * L.ntiles * 4) +
+                    align256((size_t)fixed_splits * L.R_total * a->rank * 4) + out_part_bytes + exact_bytes;
+  off += align256((size_t)prob_rows * L.n_slots * 2);
   L.tile_max = off;
-  off += align256((size_t)L.R_total * L.nstats * 4);
+  off += align256((size_t)stat_rows * L.nstats * 4);
   L.tile_sum = off;
-  off += align256((size_t)L.R_total * L.nstats * 4);
+  off += align256((size_t)stat_rows * L.nstats * 4);
   L.w_part = off;
   off += align256((size_t)L.nsplits * L.R_total * a->rank * 4);
+  L.split_max = off;
+  if (L.rows_mw) off += align256((size_t)L.nsplits * L.R_total * 4);
   L.out_part = off;
-  off += align256((size_t)L.nchunks * a->batch * L.R_total * a->head_dim * 4);
+  off += out_part_bytes;
   L.exact = off;
-  off += align256((size_t)a->batch * L.R_total * kExactParts * (a->head_dim + 2) * 4);
+  off += exact_bytes;
   L.total = off;
+  if (!L.rows_mw) L.noalloc_total += off - decode_bytes;
   return L;
 }
 
@@ -2403,10 +3028,11 @@ int launch_keys_scores(const dkv_attend_args_t* a, const Layout& L, char* ws, hi
   k.ntiles = L.ntiles;
   k.nstats = L.nstats;
   k.query_dtype = a->query_dtype;
+  k.lines_valid = scoring ? nullptr : (uint32_t*)(ws + L.valid);
   const int HPW = 256 / a->head_dim;
   k.total_wg = L.ntiles * (a->kv_heads / HPW);
   k.per_xcd = (k.total_wg + 7) / 8;
-  const dim3 grid(8 * k.per_xcd);
+  dim3 grid(8 * k.per_xcd);
   // decoding (at most kSmallRows query rows per KV head) and question scoring are separate
   // instantiations, so neither epilogue's registers weigh on the other's main loop
   const bool small = (a->q_heads / a->kv_heads) * a->q_len <= kSmallRows;
@@ -2425,8 +3051,40 @@ int launch_keys_scores(const dkv_attend_args_t* a, const Layout& L, char* ws, hi
       hipLaunchKernelGGL((keys_scores_head_kernel<64, 8>), hgrid, dim3(512), 0, st, k);
     return dkv::check_launch("keys_scores (one head per workgroup)");
   }
-  // probabilities: the value side's blocked layout when decoding, row-major [R][ntiles * 256] for
-  // question scoring (read by the importance kernel)
+  if (!scoring && !small) {  // many rows: the statistics are the quarters'
+    k.sub_max = k.tile_max;
+    k.sub_sum = k.tile_sum;
+    k.vcodes = (const uint8_t*)(ws + L.vcodes);
+    k.vaff = (const float2*)(ws + L.vaff);
+    k.vtop = (const float*)(ws + L.vtop);
+    k.lines = (uint8_t*)(ws + L.lines);
+    k.lines_exp = (int*)(ws + L.lines_exp);
+    k.convert_wg = 2 * kCUs;
+    grid.x += k.convert_wg;
+    const int nw = k2_rows_waves(a, L.ntiles);
+    if (nw > 0) {
+      k.total_wg = L.ntiles * (8 / nw) * (a->kv_heads * a->head_dim / 128);
+      k.per_xcd = (k.total_wg + 7) / 8;
+      const dim3 rgrid(8 * k.per_xcd + k.convert_wg);
+      auto launch = [&](auto d, auto w) {
+        constexpr int Dv = decltype(d)::value, W = decltype(w)::value;
+        hipLaunchKernelGGL((keys_scores_head_kernel<Dv, W, true>), rgrid, dim3(W * 64), 0, st, k);
+      };
+      using D64 = std::integral_constant<int, 64>;
+      using D128 = std::integral_constant<int, 128>;
+      using W2 = std::integral_constant<int, 2>;
+      using W4 = std::integral_constant<int, 4>;
+      using W8 = std::integral_constant<int, 8>;
+      if (a->head_dim == 128) {
+        if (nw == 8) launch(D128{}, W8{}); else if (nw == 4) launch(D128{}, W4{}); else launch(D128{}, W2{});
+      } else {
+        if (nw == 8) launch(D64{}, W8{}); else if (nw == 4) launch(D64{}, W4{}); else launch(D64{}, W2{});
+      }
+      return dkv::check_launch("keys_scores (many rows)");
+    }
+  }
+  // probabilities: the value side's blocked layout when decoding (its operand lines with many rows), row-major
+  // [R][ntiles * 256] for question scoring (read by the importance kernel)
   if (a->head_dim == 128) {
     if (small && !scoring)
       hipLaunchKernelGGL((keys_scores_kernel<128, true>), grid, dim3(kK2Threads), 0, st, k);
@@ -2449,6 +3107,82 @@ int launch_keys_scores(const dkv_attend_args_t* a, const Layout& L, char* ws, hi
   return dkv::check_launch("keys_scores");
 }
 
+// The value side of a many-row decode: value_rows_kernel, basis_rows_kernel with the exact tail, the merge.
+int launch_rows_values(const dkv_attend_args_t* a, const Layout& L, char* ws, int E_total, hipStream_t st) {
+  int rc;
+  if (L.nsplits > 0) {
+    K3RowsArgs k{};
+    k.probs = (const uint8_t*)(ws + L.probs);
+    k.values = (const uint8_t*)(ws + L.lines);
+    k.lines_valid = (uint32_t*)(ws + L.valid);
+    k.lines_exp = (const int*)(ws + L.lines_exp);
+    k.sub_max = (const float*)(ws + L.tile_max);
+    k.cu_seqlens = a->cu_seqlens;
+    k.w_part = (float*)(ws + L.w_part);
+    k.split_max = (float*)(ws + L.split_max);
+    k.batch = a->batch;
+    k.n_total = L.n_total;
+    k.n_slots = L.n_slots;
+    k.R_total = L.R_total;
+    k.nsub = L.nstats;
+    k.rank = a->rank;
+    k.split_tok = L.split_tok;
+    k.mt = (L.R_total + 64 * L.rows_mw - 1) / (64 * L.rows_mw);
+    k.nt = a->rank / kRowsCols;
+    k.total_wg = k.mt * k.nt * L.nsplits;
+    k.per_xcd = (k.total_wg + 7) / 8;
+    const dim3 grid(8u * (unsigned)k.per_xcd);
+    if (L.rows_mw == 4)
+      hipLaunchKernelGGL(value_rows_kernel<4>, grid, dim3(512), 0, st, k);
+    else if (L.rows_mw == 2)
+      hipLaunchKernelGGL(value_rows_kernel<2>, grid, dim3(512), 0, st, k);
+    else
+      hipLaunchKernelGGL(value_rows_kernel<1>, grid, dim3(512), 0, st, k);
+    rc = dkv::check_launch("value_rows");
+    if (rc) return rc;
+  }
+  const RowMergeArgs m = row_merge_args(a, L, ws, E_total);
+  K3bRowsArgs kb{};
+  kb.cu_seqlens = a->cu_seqlens;
+  kb.w_part = (const float*)(ws + L.w_part);
+  kb.split_max = (const float*)(ws + L.split_max);
+  kb.value_basis = a->value_basis;
+  kb.out_part = (float*)(ws + L.out_part);
+  kb.batch = a->batch;
+  kb.n_total = L.n_total;
+  kb.layer = a->layer;
+  kb.Hkv = a->kv_heads;
+  kb.RH = L.R_total / a->kv_heads;
+  kb.rank = a->rank;
+  kb.R_total = L.R_total;
+  kb.nchunks = L.nchunks;
+  kb.split_tok = L.split_tok;
+  kb.row_blocks = (kb.RH + kBasisRows - 1) / kBasisRows;
+  kb.n_exact_wg = a->batch * L.R_total;
+  const long blocks = kb.n_exact_wg + (long)a->batch * a->kv_heads * kb.row_blocks * L.nchunks;
+  auto k3b = [&](auto d, auto xt) {
+    hipLaunchKernelGGL((basis_rows_kernel<decltype(d)::value, decltype(xt)::value>), dim3((unsigned)blocks), dim3(256), 0,
+                       st, kb, m);
+  };
+  using D64 = std::integral_constant<int, 64>;
+  using D128 = std::integral_constant<int, 128>;
+  using X32 = std::integral_constant<int, DKV_F32>;
+  using X16 = std::integral_constant<int, DKV_F16>;
+  using XB16 = std::integral_constant<int, DKV_BF16>;
+  const bool d128 = a->head_dim == 128;
+  if (a->exact_dtype == DKV_F16) {
+    if (d128) k3b(D128{}, X16{}); else k3b(D64{}, X16{});
+  } else if (a->exact_dtype == DKV_BF16) {
+    if (d128) k3b(D128{}, XB16{}); else k3b(D64{}, XB16{});
+  } else {
+    if (d128) k3b(D128{}, X32{}); else k3b(D64{}, X32{});
+  }
+  rc = dkv::check_launch("basis_rows");
+  if (rc) return rc;
+  hipLaunchKernelGGL(finish_kernel<4>, dim3((unsigned)((long)a->batch * L.R_total)), dim3(kRowThreads), 0, st, m);
+  return dkv::check_launch("finish");
+}
+
 }  // namespace
 
 extern "C" size_t dkv_attend_workspace_bytes(const dkv_attend_args_t* a) {
@@ -2467,8 +3201,8 @@ extern "C" int dkv_attend_prepare(const dkv_attend_args_t* a, int32_t plane_cap,
   // only the decoded areas at the head of the workspace are written (the value codes only with a
   // value stream), so an attend workspace, or a score workspace for the keys alone, will do
   const Layout L = make_layout(a, a->value.blob != nullptr);
-  DKV_REQUIRE(workspace && workspace_bytes >= L.probs, DKV_EWORKSPACE,
-              "dkv_attend_prepare: workspace %zu B < required %zu B", workspace_bytes, L.probs);
+  DKV_REQUIRE(workspace && workspace_bytes >= L.lines, DKV_EWORKSPACE,
+              "dkv_attend_prepare: workspace %zu B < required %zu B", workspace_bytes, L.lines);
   DecodeArgs d{};
   d.s = a->key;
   d.cu_seqlens = a->cu_seqlens;
@@ -2500,7 +3234,8 @@ extern "C" int dkv_attend_prepare(const dkv_attend_args_t* a, int32_t plane_cap,
   }
   hipLaunchKernelGGL(decode_codes_kernel, dim3((unsigned)(key_blocks + value_blocks)), dim3(kDecodeSlots),
                      rows * sizeof(int2), dkv::as_stream(stream), d, v, (uint8_t*)((char*)workspace + L.vcodes),
-                     (float2*)((char*)workspace + L.vaff), key_blocks);
+                     (float2*)((char*)workspace + L.vaff), (float*)((char*)workspace + L.vtop),
+                     a->value.blob ? (uint32_t*)((char*)workspace + L.valid) : nullptr, key_blocks);
   return dkv::check_launch("decode_codes");
 }
 
@@ -2535,6 +3270,7 @@ extern "C" int dkv_attend_values(const dkv_attend_args_t* a, void* workspace, si
   char* ws = (char*)workspace;
   hipStream_t st = dkv::as_stream(stream);
   const int G = dkv::stream_groups(a->key);
+  if (L.rows_mw) return launch_rows_values(a, L, ws, E_total, st);
   if (L.nsplits > 0) {  // K3a: one workgroup per (split, group, row block)
     K3aArgs k{};
     k.vcodes = (const uint8_t*)(ws + L.vcodes);
@@ -2588,23 +3324,13 @@ extern "C" int dkv_attend_values(const dkv_attend_args_t* a, void* workspace, si
   kb.split_tok = L.split_tok;
   kb.n_exact_wg = a->batch * L.R_total * kExactParts;
   const long k3b_blocks = kb.n_exact_wg + (long)a->batch * a->kv_heads * L.nchunks * (a->head_dim / kK3bDims);
-  const bool rows4 = (a->q_heads / a->kv_heads) * a->q_len <= 4;
-  auto k3b = [&](auto nr, auto xt) {
-    hipLaunchKernelGGL((basis_apply_kernel<decltype(nr)::value, decltype(xt)::value>), dim3((unsigned)k3b_blocks),
-                       dim3(kRowThreads), 0, st, kb, m);
-  };
-  using R4 = std::integral_constant<int, 4>;
-  using R8 = std::integral_constant<int, 8>;
-  using X32 = std::integral_constant<int, DKV_F32>;
-  using X16 = std::integral_constant<int, DKV_F16>;
-  using XB16 = std::integral_constant<int, DKV_BF16>;
-  if (a->exact_dtype == DKV_F16) {
-    if (rows4) k3b(R4{}, X16{}); else k3b(R8{}, X16{});
-  } else if (a->exact_dtype == DKV_BF16) {
-    if (rows4) k3b(R4{}, XB16{}); else k3b(R8{}, XB16{});
-  } else {
-    if (rows4) k3b(R4{}, X32{}); else k3b(R8{}, X32{});
-  }
+  const dim3 k3b_grid((unsigned)k3b_blocks);
+  if (a->exact_dtype == DKV_F16)
+    hipLaunchKernelGGL(basis_apply_kernel<DKV_F16>, k3b_grid, dim3(kRowThreads), 0, st, kb, m);
+  else if (a->exact_dtype == DKV_BF16)
+    hipLaunchKernelGGL(basis_apply_kernel<DKV_BF16>, k3b_grid, dim3(kRowThreads), 0, st, kb, m);
+  else
+    hipLaunchKernelGGL(basis_apply_kernel<DKV_F32>, k3b_grid, dim3(kRowThreads), 0, st, kb, m);
   rc = dkv::check_launch("basis_apply");
   if (rc) return rc;
   // K3c
@@ -3242,7 +3968,10 @@ extern "C" int dkv_topk(const float* scores, int32_t n, int32_t k, int32_t* idx_
 // ===========================================================================
 namespace {
 
-constexpr size_t kStaticScratchBytes = DKV_NOALLOC_MAX_BYTES;  // 64 MiB
+// 128 MiB: contexts are taken up to DKV_NOALLOC_MAX_BYTES of noalloc_total, and a many-row decode's layout stays
+// below twice that (its value lines add 2 bytes to 3.1 per component, and its probabilities' padding, statistics and
+// splits stay below twice theirs).
+constexpr size_t kStaticScratchBytes = 2 * DKV_NOALLOC_MAX_BYTES;
 constexpr int kMaxDevices = 64;
 
 }  // namespace
@@ -3282,10 +4011,10 @@ extern "C" int dkv_attend_layer_noalloc(const dkv_attend_args_t* a, void* stream
   rc = check_values(a, E_total);
   if (rc) return rc;
   const Layout L = make_layout(a);
-  DKV_REQUIRE(L.total <= kStaticScratchBytes, DKV_EWORKSPACE,
+  DKV_REQUIRE(L.noalloc_total <= DKV_NOALLOC_MAX_BYTES && L.total <= kStaticScratchBytes, DKV_EWORKSPACE,
               "dkv_attend_layer_noalloc: this context needs %zu B of scratch; the static maximum is %zu B "
               "(use dkv_attend_prepare + dkv_attend_layer with a caller workspace)",
-              L.total, kStaticScratchBytes);
+              L.noalloc_total, DKV_NOALLOC_MAX_BYTES);
   void* ws = nullptr;
   rc = scratch_address(&ws, "dkv_attend_layer_noalloc");
   if (rc) return rc;

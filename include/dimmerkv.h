@@ -346,10 +346,11 @@ int dkv_topk(const float* scores, int32_t n, int32_t k, int32_t* idx_out, void* 
  * memory (code under HIP graph capture, tight serving loops, harnesses that
  * forbid allocation).  Does what dkv_attend_prepare(a, 8, ...) followed by
  * dkv_attend_layer(a, ...) do, with the workspace in a file-scope device array
- * of DKV_NOALLOC_MAX_BYTES that every GPU the library runs on holds until the
- * process ends; calls nothing that allocates.  A context whose workspace
- * (dkv_attend_workspace_bytes) exceeds the maximum is rejected with
- * DKV_EWORKSPACE before anything is launched.  Every call decodes the codes
+ * of 2 * DKV_NOALLOC_MAX_BYTES that every GPU the library runs on holds until
+ * the process ends; calls nothing that allocates.  A context whose workspace
+ * (without the value lines and padding that more than 4 query rows per KV head
+ * add to dkv_attend_workspace_bytes) exceeds DKV_NOALLOC_MAX_BYTES is rejected
+ * with DKV_EWORKSPACE before anything is launched.  Every call decodes the codes
  * again (the array keeps only the last call's contents); calls in sequence are
  * independent, calls that overlap on one GPU race.  The first call on a device
  * looks up that device's address of the array (hipGetSymbolAddress) and must
