@@ -26,10 +26,32 @@ extern "C" int dkv_abi_version(void) { return DKV_ABI_VERSION; }
 extern "C" const char* dkv_last_error(void) { return dkv::g_error.c_str(); }
 
 // ---------------------------------------------------------------------------
-// Pack: one wave per (token, group).  Lane L owns bit position L of each
-// plane word; it fetches (by cross-lane shuffle) the code of the coefficient
-// that the layout puts at that position and the wave ballots the bit.
+// Pack: one thread per (token, group, half).  Byte i of the half's code word w is the coefficient of plane bit
+// w + 8 i (before the plane's rotation by 25 + p), so plane word p gathers bit 7 - p of all 32 bytes: an 8 x 8 bit
+// transpose of the eight words, byte by byte, in three rounds of masked swaps.  A plane's two words (halves) go
+// out side by side from neighbouring lanes.  8,155 tokens x 16 groups with the cold tier: 8.6 us (49 with one wave per
+// (token, group), eight shuffles and ballots each).
 // ---------------------------------------------------------------------------
+// Exchanges the bits of a under `mask << shift` with those of b under `mask`.
+DKV_DEVICE void swap_bits(uint32_t& a, uint32_t& b, int shift, uint32_t mask) {
+  const uint32_t d = ((a >> shift) ^ b) & mask;
+  b ^= d;
+  a ^= d << shift;
+}
+
+// In every byte lane: bit p of word w <-> bit w of word p.
+DKV_DEVICE void transpose_bits(uint32_t (&v)[8]) {
+#pragma unroll
+  for (int w = 0; w < 4; ++w) swap_bits(v[w], v[w + 4], 4, 0x0f0f0f0fu);
+#pragma unroll
+  for (int w = 0; w < 8; w += 4) {
+    swap_bits(v[w], v[w + 2], 2, 0x33333333u);
+    swap_bits(v[w + 1], v[w + 3], 2, 0x33333333u);
+  }
+#pragma unroll
+  for (int w = 0; w < 8; w += 2) swap_bits(v[w], v[w + 1], 1, 0x55555555u);
+}
+
 __global__ __launch_bounds__(256) void pack_kernel(const uint8_t* __restrict__ codes, const uint16_t* __restrict__ low,
                                                    const uint16_t* __restrict__ span,
                                                    const int16_t* __restrict__ pieces, int n, dkv_order_t order,
@@ -37,47 +59,37 @@ __global__ __launch_bounds__(256) void pack_kernel(const uint8_t* __restrict__ c
                                                    uint8_t* __restrict__ cold,
                                                    const int64_t* __restrict__ cold_tok_off) {
   const int G = order.groups;
-  const long gw = (long)blockIdx.x * 4 + (threadIdx.x >> 6);
-  const int lane = threadIdx.x & 63;
+  const long id = (long)blockIdx.x * 256 + threadIdx.x;
+  const long gw = id >> 1;
+  const int h = (int)(id & 1);
   if (gw >= (long)n * G) return;
   const int t = (int)(gw / G), g = (int)(gw % G);
+  uint32_t v[8];
+  __builtin_memcpy(v, codes + gw * 64 + h * 32, 32);  // (a caller's buffer may lie at any byte)
   const int k = pieces[t];
   const int m = order.planes[(long)k * G + g];
   const int m_full = order.planes[(long)order.pieces * G + g];
-  const uint32_t code = codes[gw * 64 + lane];
-  uint64_t words[8];
-#pragma unroll
-  for (int p = 0; p < 8; ++p) {
-    const int jj = ((lane & 31) + 25 + p) & 31;  // (q - 7 + p) mod 32
-    const int coef = (lane & 32) + 4 * (jj & 7) + (jj >> 3);
-    const uint32_t c = (uint32_t)__shfl((int)code, coef, 64);
-    words[p] = __ballot((c >> (7 - p)) & 1u);
-  }
   const uint32_t header = (uint32_t)low[gw] | ((uint32_t)span[gw] << 16);
+  transpose_bits(v);
+  uint32_t words[8];
+#pragma unroll
+  for (int p = 0; p < 8; ++p) words[p] = __builtin_rotateright32(v[7 - p], (25 + p) & 31);
   if (m > 0) {
     uint32_t* dst = (uint32_t*)(hot + hot_off[t] + order.seg_off[(long)k * G + g]);
-    if (lane == 0) dst[0] = header;
-    if (lane < m) {
-      uint64_t wv = 0;
+    if (h == 0) dst[0] = header;
 #pragma unroll
-      for (int p = 0; p < 8; ++p) wv = (p == lane) ? words[p] : wv;
-      dst[1 + 2 * lane] = (uint32_t)wv;
-      dst[2 + 2 * lane] = (uint32_t)(wv >> 32);
-    }
+    for (int p = 0; p < 8; ++p)
+      if (p < m) dst[1 + 2 * p + h] = words[p];
   }
   if (cold != nullptr && m < m_full) {
     uint32_t* dst = (uint32_t*)(cold + cold_tok_off[t] + order.cold_off[(long)k * G + g]);
     if (m == 0) {
-      if (lane == 0) dst[0] = header;
+      if (h == 0) dst[0] = header;
       dst += 1;
     }
-    if (lane >= m && lane < m_full) {
-      uint64_t wv = 0;
 #pragma unroll
-      for (int p = 0; p < 8; ++p) wv = (p == lane) ? words[p] : wv;
-      dst[2 * (lane - m)] = (uint32_t)wv;
-      dst[2 * (lane - m) + 1] = (uint32_t)(wv >> 32);
-    }
+    for (int p = 0; p < 8; ++p)
+      if (p >= m && p < m_full) dst[2 * (p - m) + h] = words[p];
   }
 }
 
@@ -90,8 +102,7 @@ extern "C" int dkv_pack_planes(const uint8_t* codes, const uint16_t* low, const 
   if (n == 0) return DKV_OK;
   DKV_REQUIRE(codes && low && span && pieces && hot && hot_off, DKV_EINVAL, "dkv_pack_planes: null pointer");
   DKV_REQUIRE(!cold || (cold_off && order.cold_off), DKV_EINVAL, "dkv_pack_planes: cold needs cold offsets");
-  const long waves = (long)n * order.groups;
-  const long blocks = (waves + 3) / 4;
+  const long blocks = ((long)n * order.groups * 2 + 255) / 256;
   DKV_REQUIRE(blocks < (1L << 31), DKV_ESHAPE, "dkv_pack_planes: too many tokens");
   hipLaunchKernelGGL(pack_kernel, dim3((unsigned)blocks), dim3(256), 0, dkv::as_stream(stream), codes, low, span,
                      pieces, n, order, hot, hot_off, cold, cold_off);
@@ -464,56 +475,169 @@ extern "C" int dkv_dequantize_codes(const uint8_t* codes, const uint16_t* low, c
 }
 
 // ---------------------------------------------------------------------------
-// Encoder: quantize8 (progressive.py:37-44) and the per-group squared error at
-// 0..8 planes (progressive.py:152-158) in one pass over the coefficients.  One
-// wave per (token, group), one lane per member: the group's min and max are
-// wave reductions; low = f16(min), span = f16(max(max - low, 1e-8)),
-// code = clamp(floor((x - low) / span * 256), 0, 255) with the division
-// correctly rounded (a NaN from a zero fp16 span gives code 0); then every
-// lane's squared error against the reference's dequantize at each plane count,
-// summed over the wave.
+// Encoder: quantize8 (progressive.py:37-44) and the squared error of the codes cut to 0..8 planes
+// (progressive.py:152-158) in one pass over the coefficients.  16 lanes per (token, group), four members
+// a lane (one 16-byte load, one word of codes): the group's min and max are reductions over the 16
+// lanes; low = f16(min), span = f16(max(max - low, 1e-8)), code = clamp(floor((x - low) / span * 256), 0, 255)
+// with the division correctly rounded (a NaN from a zero fp16 span gives code 0); then every lane's
+// squared errors against the reference's dequantize at each plane count, summed over the lanes.
+//
+// quantize8_kernel writes the codes and, asked for, the table of a group's nine errors; rung_errors_kernel writes
+// the codes and what the allocator takes instead of the table: a token's error at every rung of the order (the
+// sum over its groups of the table entry at the rung's planes) and its energy (the errors at no planes), a wave
+// per token.  8,155 tokens x 1,024, codes and errors at 7 rungs: 26 us, bound by the errors' arithmetic (its bytes take
+// 8; 53 us with the table at one wave per group before, and torch's gather and sums over it besides).
 // ---------------------------------------------------------------------------
+template <int CTRL>
+DKV_DEVICE float lanes_dpp(float v) {
+  return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), CTRL, 0xf, 0xf, true));
+}
+
+// Over the 16 lanes of a DPP row, in every lane: xor 1, xor 2, then the mirrored half row and row.
+DKV_DEVICE float row_sum(float v) {
+  v += lanes_dpp<0xB1>(v);
+  v += lanes_dpp<0x4E>(v);
+  v += lanes_dpp<0x141>(v);
+  return v + lanes_dpp<0x140>(v);
+}
+
+DKV_DEVICE float row_max(float v) {
+  v = fmaxf(v, lanes_dpp<0xB1>(v));
+  v = fmaxf(v, lanes_dpp<0x4E>(v));
+  v = fmaxf(v, lanes_dpp<0x141>(v));
+  return fmaxf(v, lanes_dpp<0x140>(v));
+}
+
+struct QuadCodes {
+  float lo, sp;
+  uint32_t codes;  // byte i: member 4 * (lane & 15) + i
+};
+
+DKV_DEVICE uint16_t half_bits(float v) {
+  const half_t h = (half_t)v;
+  uint16_t b;
+  __builtin_memcpy(&b, &h, 2);
+  return b;
+}
+
+DKV_DEVICE QuadCodes quantize_quad(const float (&x)[4]) {
+  QuadCodes q;
+  const float amin = -row_max(fmaxf(fmaxf(-x[0], -x[1]), fmaxf(-x[2], -x[3])));
+  const float amax = row_max(fmaxf(fmaxf(x[0], x[1]), fmaxf(x[2], x[3])));
+  q.lo = (float)(half_t)amin;
+  q.sp = (float)(half_t)fmaxf(amax - q.lo, 1e-8f);
+  q.codes = 0;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    float v;
+    {
+#pragma clang fp contract(off)
+      v = floorf(((x[i] - q.lo) / q.sp) * 256.0f);
+    }
+    v = (v != v) ? 0.0f : fminf(fmaxf(v, 0.0f), 255.0f);
+    q.codes |= (uint32_t)v << (8 * i);
+  }
+  return q;
+}
+
+// The group's squared error at `lane & 15` planes (0 in lanes past 8).  dequant_exact's value at m planes,
+// low + ((code >> (8 - m)) + 0.5) * span / 2^m, with the code's low bits cleared instead of shifted out: the factor
+// has at most 9 bits and the fp16 span 11, so their product is exact and one fma rounds the sum as the separate
+// operations do.
+DKV_DEVICE float quad_error(const float (&x)[4], const QuadCodes& q) {
+  const int j = threadIdx.x & 15;
+  const float step = q.sp * (1.0f / 256.0f);
+  float mine = 0.0f;
+#pragma unroll
+  for (int m = 0; m <= 8; ++m) {
+    const uint32_t cut = q.codes & (0x01010101u * (0xffu & (0xff00u >> m)));
+    float s = 0.0f;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const float c = (float)((cut >> (8 * i)) & 0xffu) + __builtin_ldexpf(0.5f, 8 - m);
+      const float d = m == 0 ? x[i] : x[i] - __builtin_fmaf(c, step, q.lo);
+      s = __builtin_fmaf(d, d, s);
+    }
+    s = row_sum(s);
+    mine = j == m ? s : mine;
+  }
+  return mine;
+}
+
 __global__ __launch_bounds__(256) void quantize8_kernel(const float* __restrict__ coef, long ngroups,
                                                         uint8_t* __restrict__ codes, uint16_t* __restrict__ low,
                                                         uint16_t* __restrict__ span, float* __restrict__ errors) {
-  const long tg = (long)blockIdx.x * 4 + (threadIdx.x >> 6);
-  const int lane = threadIdx.x & 63;
-  if (tg >= ngroups) return;
-  const float x = coef[tg * 64 + lane];
-  const float amin = -wave_max(-x), amax = wave_max(x);
-  const half_t lo_h = (half_t)amin;
-  const float lo = (float)lo_h;
-  const half_t sp_h = (half_t)fmaxf(amax - lo, 1e-8f);
-  const float sp = (float)sp_h;
-  float q;
-  {
-#pragma clang fp contract(off)
-    q = floorf(((x - lo) / sp) * 256.0f);
-  }
-  q = (q != q) ? 0.0f : fminf(fmaxf(q, 0.0f), 255.0f);
-  const uint32_t code = (uint32_t)q;
-  codes[tg * 64 + lane] = (uint8_t)code;
-  if (lane == 0) {
-    uint16_t lb, sb;
-    __builtin_memcpy(&lb, &lo_h, 2);
-    __builtin_memcpy(&sb, &sp_h, 2);
-    low[tg] = lb;
-    span[tg] = sb;
+  const long tg = (long)blockIdx.x * 16 + (threadIdx.x >> 4);
+  const int j = threadIdx.x & 15;
+  if (tg >= ngroups) return;  // whole rows of 16 lanes
+  float x[4];
+  __builtin_memcpy(x, coef + tg * 64 + 4 * j, 16);  // (callers' buffers may lie at any element)
+  const QuadCodes q = quantize_quad(x);
+  __builtin_memcpy(codes + tg * 64 + 4 * j, &q.codes, 4);
+  if (j == 0) {
+    low[tg] = half_bits(q.lo);
+    span[tg] = half_bits(q.sp);
   }
   if (!errors) return;
-  float mine = 0.0f;  // this lane ends up holding the error at (lane) planes, lane < 9
+  const float e = quad_error(x, q);
+  if (j <= 8) errors[tg * 9 + j] = e;
+}
+
+constexpr int kRungChunks = 8;  // 16 rungs each
+
+template <int CHUNKS>
+__global__ __launch_bounds__(256) void rung_errors_kernel(const float* __restrict__ coef, int n, int G,
+                                                          const uint8_t* __restrict__ planes, int rungs,
+                                                          uint8_t* __restrict__ codes, uint16_t* __restrict__ low,
+                                                          uint16_t* __restrict__ span, float* __restrict__ errors,
+                                                          float* __restrict__ energy) {
+  extern __shared__ uint8_t at_rung[];  // [rungs][G]
+  for (int e = threadIdx.x; e < rungs * G; e += 256) at_rung[e] = min((int)planes[e], 8);
+  __syncthreads();
+  const int t = blockIdx.x * 4 + (threadIdx.x >> 6);
+  if (t >= n) return;
+  const int lane = threadIdx.x & 63, j = lane & 15, row = lane >> 4;
+  float sum[CHUNKS], total = 0.0f;
 #pragma unroll
-  for (int m = 0; m <= 8; ++m) {
-    float d;
-    {
-#pragma clang fp contract(off)
-      d = x - dequant_exact(code, m, lo, sp, __builtin_ldexpf(1.0f, -m));
-      d = d * d;
+  for (int c = 0; c < CHUNKS; ++c) sum[c] = 0.0f;
+  const float* src = coef + (long)t * G * 64 + lane * 4;
+  float next[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+  if (row < G) __builtin_memcpy(next, src, 16);
+  for (int g0 = 0; g0 < G; g0 += 4) {
+    const int g = g0 + row;  // past the last group: zeros, not stored, not summed
+    float x[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) x[i] = g < G ? next[i] : 0.0f;
+    if (g + 4 < G) __builtin_memcpy(next, src + (long)(g0 + 4) * 64, 16);
+    const QuadCodes q = quantize_quad(x);
+    const float e = quad_error(x, q);
+    const long tg = (long)t * G + g;
+    if (g < G) {
+      __builtin_memcpy(codes + tg * 64 + 4 * j, &q.codes, 4);
+      if (j == 0) {
+        low[tg] = half_bits(q.lo);
+        span[tg] = half_bits(q.sp);
+        total += e;  // lane 0 of the row holds the error at no planes
+      }
     }
-    const float e = wave_sum(d);
-    mine = lane == m ? e : mine;
+#pragma unroll
+    for (int c = 0; c < CHUNKS; ++c) {
+      const int r = min(c * 16 + j, rungs - 1);
+      const float v = __shfl(e, (lane & 48) + at_rung[r * G + min(g, G - 1)], 64);
+      sum[c] += g < G ? v : 0.0f;
+    }
   }
-  if (lane <= 8) errors[tg * 9 + lane] = mine;
+  // the four rows' groups
+#pragma unroll
+  for (int c = 0; c < CHUNKS; ++c) {
+    float v = sum[c];
+    v += __shfl_xor(v, 16, 64);
+    v += __shfl_xor(v, 32, 64);
+    if (row == 0 && c * 16 + j < rungs) errors[(long)t * rungs + c * 16 + j] = v;
+  }
+  total += __shfl_xor(total, 16, 64);
+  total += __shfl_xor(total, 32, 64);
+  if (lane == 0) energy[t] = total;
 }
 
 extern "C" int dkv_quantize8(const float* coef, int32_t n, int32_t groups, uint8_t* codes, uint16_t* low,
@@ -522,9 +646,27 @@ extern "C" int dkv_quantize8(const float* coef, int32_t n, int32_t groups, uint8
   DKV_REQUIRE(n >= 0 && groups > 0, DKV_ESHAPE, "dkv_quantize8: bad shape (n=%d groups=%d)", n, groups);
   if (n == 0) return DKV_OK;
   const long ngroups = (long)n * groups;
-  hipLaunchKernelGGL(quantize8_kernel, dim3((unsigned)((ngroups + 3) / 4)), dim3(256), 0, dkv::as_stream(stream),
+  hipLaunchKernelGGL(quantize8_kernel, dim3((unsigned)((ngroups + 15) / 16)), dim3(256), 0, dkv::as_stream(stream),
                      coef, ngroups, codes, low, span, errors);
   return dkv::check_launch("dkv_quantize8");
+}
+
+extern "C" int dkv_quantize8_rungs(const float* coef, int32_t n, int32_t groups, const uint8_t* planes, int32_t rungs,
+                                   uint8_t* codes, uint16_t* low, uint16_t* span, float* errors, float* energy,
+                                   void* stream) {
+  DKV_REQUIRE(n >= 0 && groups > 0 && rungs > 0 && rungs <= 16 * kRungChunks && (long)rungs * groups <= 65536, DKV_ESHAPE,
+              "dkv_quantize8_rungs: bad shape (n=%d groups=%d rungs=%d)", n, groups, rungs);
+  if (n == 0) return DKV_OK;
+  DKV_REQUIRE(coef && planes && codes && low && span && errors && energy, DKV_EINVAL, "dkv_quantize8_rungs: null pointer");
+  const dim3 grid((unsigned)((n + 3) / 4));
+  const size_t lds = (size_t)rungs * groups;
+  if (rungs <= 16)
+    hipLaunchKernelGGL(rung_errors_kernel<1>, grid, dim3(256), lds, dkv::as_stream(stream), coef, n, groups, planes, rungs,
+                       codes, low, span, errors, energy);
+  else
+    hipLaunchKernelGGL(rung_errors_kernel<kRungChunks>, grid, dim3(256), lds, dkv::as_stream(stream), coef, n, groups, planes,
+                       rungs, codes, low, span, errors, energy);
+  return dkv::check_launch("dkv_quantize8_rungs");
 }
 
 // ---------------------------------------------------------------------------

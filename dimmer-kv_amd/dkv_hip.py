@@ -29,7 +29,7 @@ EXPORTS = [
     "dkv_attend_scores", "dkv_attend_values",
     "dkv_score_workspace_bytes", "dkv_score_begin", "dkv_score_layer", "dkv_topk_workspace_bytes", "dkv_topk",
     "dkv_gather_cold", "dkv_refine_rows", "dkv_wire_pack", "dkv_wire_unpack", "dkv_attend_layer_noalloc",
-    "dkv_quantize8", "dkv_centered_rows", "dkv_matmul_f32_workspace_bytes", "dkv_matmul_f32",
+    "dkv_quantize8", "dkv_quantize8_rungs", "dkv_centered_rows", "dkv_matmul_f32_workspace_bytes", "dkv_matmul_f32",
     "dkv_ladder_errors", "dkv_ladder_code", "dkv_rows_to_caches", "dkv_copy_tokens",
 ]
 NOALLOC_MAX_BYTES = 64 << 20  # DKV_NOALLOC_MAX_BYTES: the static workspace of dkv_attend_layer_noalloc
@@ -305,6 +305,14 @@ def quantize8(coef, codes, low, span, errors=None) -> None:
     n, groups = codes.shape[0], codes.shape[1]
     _check(lib().dkv_quantize8(c_vp(ptr(coef)), c_i32(n), c_i32(groups), c_vp(ptr(codes)), c_vp(ptr(low)),
                                c_vp(ptr(span)), c_vp(ptr(errors)), c_vp(stream_handle())), "dkv_quantize8")
+
+
+def quantize8_rungs(coef, planes, codes, low, span, errors, energy) -> None:
+    """coef f32 [n, 64G], planes u8 [R, G] -> codes, low, span as quantize8's, errors f32 [n, R], energy f32 [n]."""
+    n, groups = codes.shape[0], codes.shape[1]
+    _check(lib().dkv_quantize8_rungs(c_vp(ptr(coef)), c_i32(n), c_i32(groups), c_vp(ptr(planes)), c_i32(planes.shape[0]),
+                                     c_vp(ptr(codes)), c_vp(ptr(low)), c_vp(ptr(span)), c_vp(ptr(errors)),
+                                     c_vp(ptr(energy)), c_vp(stream_handle())), "dkv_quantize8_rungs")
 
 
 def dequantize_codes(codes, low, span, planes, out) -> None:

@@ -176,6 +176,12 @@ int dkv_unpack_dequant(const dkv_stream_t* s, int32_t t0, int32_t nt, void* out,
 int dkv_quantize8(const float* coef, int32_t n, int32_t groups, uint8_t* codes, uint16_t* low, uint16_t* span,
                   float* errors, void* stream);
 
+/* The same codes with what the allocator needs of the errors (scripts/progressive.py:144-163): planes u8
+ * [rungs][G], each rung's planes per group (rungs <= 128, rungs * G <= 65536) -> errors f32 [n][rungs], the
+ * squared error of the token cut to each rung, and energy f32 [n], the sum of its squared coefficients. */
+int dkv_quantize8_rungs(const float* coef, int32_t n, int32_t groups, const uint8_t* planes, int32_t rungs,
+                        uint8_t* codes, uint16_t* low, uint16_t* span, float* errors, float* energy, void* stream);
+
 /* Centred token-matrix rows, the encoders' input to the PCA projection
  * (scripts/kvtc.py:137-140 to_matrix with :40-43 derotate and :50-53
  * token_matrix, then (matrix[start:end] - mean) as at :189 and
