@@ -30,7 +30,7 @@ EXPORTS = [
     "dkv_score_workspace_bytes", "dkv_score_begin", "dkv_score_layer", "dkv_topk_workspace_bytes", "dkv_topk",
     "dkv_gather_cold", "dkv_refine_rows", "dkv_wire_pack", "dkv_wire_unpack", "dkv_attend_layer_noalloc",
     "dkv_quantize8", "dkv_quantize8_rungs", "dkv_centered_rows", "dkv_matmul_f32_workspace_bytes", "dkv_matmul_f32",
-    "dkv_ladder_errors", "dkv_ladder_code", "dkv_rows_to_caches", "dkv_copy_tokens",
+    "dkv_ladder_errors", "dkv_ladder_code", "dkv_rows_to_caches", "dkv_copy_tokens", "dkv_outside_tokens",
 ]
 NOALLOC_MAX_BYTES = 64 << 20  # DKV_NOALLOC_MAX_BYTES: the static workspace of dkv_attend_layer_noalloc
 
@@ -268,6 +268,18 @@ def copy_tokens(src, dst, skip: int, skip_len: int) -> None:
     _check(lib().dkv_copy_tokens(c_vp(ptr(a)), c_vp(ptr(b)), c_i32(dtype_code(src[0].dtype)), c_i32(len(src)), c_i32(heads),
                                  c_i32(tokens), c_i32(dim), c_i32(skip), c_i32(skip_len), c_vp(stream_handle())),
            "dkv_copy_tokens")
+
+
+def outside_tokens(src, skip: int, skip_len: int) -> torch.Tensor:
+    """Every token outside [skip, skip + skip_len) of per-layer caches [1, H, T, D] (contiguous, one dtype):
+    [L, 1, H, T - skip_len, D]."""
+    _, heads, tokens, dim = src[0].shape
+    out = torch.empty(len(src), 1, heads, tokens - skip_len, dim, dtype=src[0].dtype, device=src[0].device)
+    table = (c_i64 * len(src))(*[ptr(t) for t in src])
+    _check(lib().dkv_outside_tokens(table, c_vp(ptr(out)), c_i32(dtype_code(out.dtype)), c_i32(len(src)), c_i32(heads),
+                                    c_i32(tokens), c_i32(dim), c_i32(skip), c_i32(skip_len), c_vp(stream_handle())),
+           "dkv_outside_tokens")
+    return out
 
 
 def matmul_f32(a: torch.Tensor, b: torch.Tensor, bias: torch.Tensor | None = None) -> torch.Tensor:

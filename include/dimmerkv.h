@@ -218,12 +218,16 @@ int dkv_ladder_code(const float* coef, int32_t n, int32_t groups, const uint8_t*
  * device pointers): row i is token first + i, plus gap_len from token
  * gap_start on; with cos / sin (f32 [tokens][head_dim]) x cos + rotate_half(x) sin
  * at that token (scripts/kvtc.py:46-47).  dkv_copy_tokens copies every token
- * outside [skip, skip + skip_len) between two such sets of caches. */
+ * outside [skip, skip + skip_len) between two such sets of caches;
+ * dkv_outside_tokens gathers them into one buffer [layers][heads][tokens - skip_len][head_dim]
+ * (layer_ptrs: a host array of device pointers; buffers 16-byte aligned). */
 int dkv_rows_to_caches(const float* rows, int32_t n, int32_t first, int32_t gap_start, int32_t gap_len,
                        const uint64_t* layer_ptrs, int32_t dtype, int32_t layers, int32_t heads, int32_t tokens,
                        int32_t head_dim, const float* cos, const float* sin, void* stream);
 int dkv_copy_tokens(const uint64_t* src_ptrs, const uint64_t* dst_ptrs, int32_t dtype, int32_t layers, int32_t heads,
                     int32_t tokens, int32_t head_dim, int32_t skip, int32_t skip_len, void* stream);
+int dkv_outside_tokens(const uint64_t* layer_ptrs, void* out, int32_t dtype, int32_t layers, int32_t heads,
+                       int32_t tokens, int32_t head_dim, int32_t skip, int32_t skip_len, void* stream);
 
 /* ---- float32 products on the fp16 matrix cores -----------------------------
  * C[m][n] = sum_k A[m][k] B[n][k] + bias[n] (bias may be NULL), all float32:

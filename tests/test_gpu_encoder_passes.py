@@ -61,3 +61,16 @@ def test_pack_any_alignment(groups, tokens, shift):
     assert torch.equal(packed.dequantize(), progressive.dequantize(codes, low, span, planes))
     packed.refine(torch.arange(tokens, device=DEV))
     assert torch.equal(packed.dequantize(), progressive.dequantize(codes, low, span, torch.full((1, groups), 8, device=DEV)))
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.float32])
+@pytest.mark.parametrize("layers,heads,tokens,dim,start,end", [(2, 3, 50, 64, 4, 18), (130, 1, 9, 8, 0, 8), (1, 8, 40, 128, 5, 40)])
+def test_outside_tokens_match_cat(layers, heads, tokens, dim, start, end, dtype):
+    """More layers than one launch takes, no sinks, no recent window."""
+    import dkv_hip
+
+    print(f"[case] outside tokens L={layers} H={heads} T={tokens} D={dim} {start}..{end} {dtype}", flush=True)
+    g = torch.Generator(DEV).manual_seed(layers)
+    caches = [torch.randn(1, heads, tokens, dim, generator=g, device=DEV).to(dtype) for _ in range(layers)]
+    got = dkv_hip.outside_tokens(caches, start, end - start)
+    assert torch.equal(got, torch.stack([torch.cat([t[..., :start, :], t[..., end:, :]], dim=2) for t in caches]))
