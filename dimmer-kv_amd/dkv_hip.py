@@ -245,8 +245,17 @@ def ladder_code(coef, bits, level):
     return decoded, codes, low, scale
 
 
+def to_device(values, dtype, device) -> torch.Tensor:
+    """A small host list (or tensor) on ``device`` without waiting for the GPU's earlier work: from pinned memory,
+    as a pageable copy synchronizes the stream."""
+    host = torch.as_tensor(values, dtype=dtype)
+    if torch.device(device).type != "cuda" or host.is_cuda or host.numel() == 0:
+        return host.to(device)
+    return host.pin_memory().to(device, non_blocking=True)
+
+
 def _pointer_table(tensors) -> torch.Tensor:
-    return torch.tensor([ptr(t) for t in tensors], dtype=torch.int64).to(tensors[0].device)
+    return to_device([ptr(t) for t in tensors], torch.int64, tensors[0].device)
 
 
 def rows_to_caches(rows, caches, first: int, gap_start: int, gap_len: int, cos=None, sin=None) -> None:

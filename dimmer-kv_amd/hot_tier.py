@@ -77,18 +77,22 @@ def _nbytes(*tensors) -> int:
     return sum(t.numel() * t.element_size() for t in tensors if t is not None and t.is_cuda)
 
 
-def _exclusive_cumsum(sizes: torch.Tensor) -> tuple[torch.Tensor, int]:
+def _offsets(sizes: torch.Tensor) -> torch.Tensor:
     off = _nonnull(torch.zeros(sizes.numel(), dtype=torch.int64, device=sizes.device))
     if sizes.numel() > 1:
         off[1:] = torch.cumsum(sizes[:-1], 0)
-    total = int(sizes.sum()) if sizes.numel() else 0
-    return off, total
+    return off
+
+
+def _exclusive_cumsum(sizes: torch.Tensor) -> tuple[torch.Tensor, int]:
+    return _offsets(sizes), int(sizes.sum()) if sizes.numel() else 0
 
 
 class PackedStream:
     """Hot + cold tiers of one stream (keys or values) for n tokens."""
 
-    def __init__(self, tables: OrderTables, blob, tok_off, pieces, cold, cold_off, hot_used: int, refine_capacity: int):
+    def __init__(self, tables: OrderTables, blob, tok_off, pieces, cold, cold_off, hot_used: int, refine_capacity: int,
+                 pieces_host: np.ndarray | None = None):
         self.tables = tables
         self.blob, self.tok_off, self.pieces = blob, tok_off, pieces
         self.cold, self.cold_off = cold, cold_off
@@ -99,8 +103,8 @@ class PackedStream:
         self.initial_pieces = pieces.clone()
         # host mirrors of each token's piece count and of the prefix sizes, for the host cold tier's
         # refine (it needs the rows on the host anyway); the device tier counts bytes on the device
-        self._pieces_h = pieces.cpu().numpy().astype(np.int64)
-        self._prefix_h = tables.prefix64.cpu().numpy()
+        self._pieces_h = pieces.cpu().numpy().astype(np.int64) if pieces_host is None else pieces_host
+        self._prefix_h = tables.prefix_np
         self._owner = None  # device tier: per-token first-entry tags of dkv_refine_rows (never cleared)
         self._refine_calls = 0
         self._stage_off = None  # host cold tier: device offsets of the staged cold blobs, by token
@@ -145,19 +149,21 @@ class PackedStream:
         pieces = _nonnull(pieces.to(device=device, dtype=torch.int16).contiguous())
         p64 = pieces.long()
         hot_sizes = tables.prefix64[p64] if n else torch.zeros(0, dtype=torch.int64, device=device)
-        tok_off, hot_total = _exclusive_cumsum(hot_sizes)
+        tok_off = _offsets(hot_sizes)
+        pieces_host = pieces.cpu().numpy().astype(np.int64)  # the one host read: the totals follow from it
+        hot_total = int(tables.prefix_np[pieces_host].sum())
         capacity = hot_total + refine_capacity * tables.full_bytes
         blob = torch.zeros(max(capacity, 16), dtype=torch.uint8, device=device)
         cold = cold_off = None
         if with_cold:
             cold_sizes = tables.full_bytes - hot_sizes
-            cold_off, cold_total = _exclusive_cumsum(cold_sizes)
+            cold_off, cold_total = _offsets(cold_sizes), n * tables.full_bytes - hot_total
             cold = torch.zeros(max(cold_total, 16), dtype=torch.uint8, device=device)
         if n:
             dkv_hip.pack_planes(codes.contiguous(), low.contiguous().view(torch.int16),
                                 span.contiguous().view(torch.int16), pieces, tables.c_order(), blob, tok_off,
                                 cold, cold_off)
-        stream = cls(tables, blob, tok_off, pieces, cold, cold_off, hot_total, refine_capacity)
+        stream = cls(tables, blob, tok_off, pieces, cold, cold_off, hot_total, refine_capacity, pieces_host)
         if cold_tier == "host":
             stream.move_cold_to_host()
         return stream
