@@ -315,6 +315,15 @@ DKV_DEVICE int2 find_tile(const int32_t* cu, int batch, int n_total, int tile, i
   return make_int2(-1, 0);
 }
 
+// De-rotation of one element (x cos - rotate_half(x) sin) / (cos^2 + sin^2), minus the mean.
+DKV_DEVICE float derotated(float x, float rh, float c, float s, float mu) {
+#pragma clang fp contract(off)
+  const float num = x * c - rh * s;
+  const float den = c * c + s * s;
+  const float v = num / den;
+  return v - mu;
+}
+
 // First and one-past-last token of sequence b.  With one sequence they are 0
 // and n_total from the kernel arguments, so the first data loads do not wait
 // on a load of cu_seqlens.

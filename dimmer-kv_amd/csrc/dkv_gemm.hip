@@ -12,7 +12,8 @@
 //
 // Three fp16 products run at a third of the fp16 rate (about 1.4 PFLOP/s here), against 0.15 PFLOP/s of
 // the float32 matrix instructions.  16,348 x 2,048 x 28,672 (the projection of a 16K-token 3B cache): 5,190 us
-// with the splitting, 1.11 PFLOP/s of fp16 products, against 12,440 us of the library's float32 product;
+// with the splitting, 1.11 PFLOP/s of fp16 products, against 12,440 us of the library's float32 product (5,030
+// straight from the caches, with the 627 us of their centred rows in it);
 // 4,061 x 28,672 x 2,048 (back): 1,295 against 3,500 us.  Error against float64 2.0e-6 and 5.0e-7, against the
 // library's 3.0e-6 and 8.1e-7.
 #include <hip/hip_runtime.h>
@@ -383,8 +384,164 @@ __global__ __launch_bounds__(256) void sum_splits_kernel(const float* __restrict
   c[(e / N) * ldc + n] = s + (bias ? bias[n] : 0.0f);
 }
 
+// A's rows as special_rows_kernel reads them: as they lie, or a token's centred row from the caches.
+struct PlainRows {
+  const float* a;
+  long lda;
+  DKV_DEVICE float at(long m, int k) const { return a[m * lda + k]; }
+};
+
+template <int T>
+DKV_DEVICE float load_elem(const void* base, long idx) {
+  if constexpr (T == DKV_F32) return ((const float*)base)[idx];
+  const uint16_t b = ((const uint16_t*)base)[idx];
+  return T == DKV_BF16 ? bf16_bits_to_float(b) : half_bits_to_float(b);
+}
+
+template <int T>
+DKV_DEVICE void load_elem8(const void* base, long idx, float (&x)[8]) {
+  if constexpr (T == DKV_F32) {
+    const float4 a = *(const float4*)((const float*)base + idx), b = *(const float4*)((const float*)base + idx + 4);
+    x[0] = a.x; x[1] = a.y; x[2] = a.z; x[3] = a.w; x[4] = b.x; x[5] = b.y; x[6] = b.z; x[7] = b.w;
+  } else {
+    const uint4 w = *(const uint4*)((const uint16_t*)base + idx);
+    const uint32_t e[4] = {w.x, w.y, w.z, w.w};
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const uint16_t lo = (uint16_t)(e[i] & 0xffffu), hi = (uint16_t)(e[i] >> 16);
+      x[2 * i] = T == DKV_BF16 ? bf16_bits_to_float(lo) : half_bits_to_float(lo);
+      x[2 * i + 1] = T == DKV_BF16 ? bf16_bits_to_float(hi) : half_bits_to_float(hi);
+    }
+  }
+}
+
+struct CacheArgs {
+  const uint64_t* layer_ptrs;
+  const float* cos;  // with sin: keys, de-rotated
+  const float* sin;
+  const float* mean;
+  int H, tokens, D, start, K;
+};
+
+template <int T, bool ROTATE>
+struct CacheRows {
+  CacheArgs c;
+  DKV_DEVICE float at(long m, int f) const {
+    const int lh = f / c.D, d = f % c.D, half = c.D / 2;
+    const long t = c.start + m, row = ((long)(lh % c.H) * c.tokens + t) * c.D;
+    const void* base = (const void*)c.layer_ptrs[lh / c.H];
+    const float x = load_elem<T>(base, row + d);
+    if constexpr (!ROTATE) return x - c.mean[f];
+    const float y = load_elem<T>(base, row + (d < half ? d + half : d - half));
+    return derotated(x, d < half ? -y : y, c.cos[t * c.D + d], c.sin[t * c.D + d], c.mean[f]);
+  }
+};
+
+// The split form of the middle tokens' centred rows (centered_rows_kernel's arithmetic, then split_rows_kernel's)
+// straight from the caches: a workgroup keeps a token's whole row in registers, 16 elements a unit (8 at d and the 8
+// at d + D / 2 that rotate with them), so neither the rows nor a second read of them exist.  `energy`, when given,
+// gets the row's sum of squares.  Bound by the lines it writes (4 bytes an element) beside the 2 it reads: 16,348 keys
+// of 28,672 columns take 793 us, 3.5 TB/s (the two kernels 627 and 715; 878 with 1,024 threads, a single workgroup on a
+// CU), 8,155 of 8,192 columns 116 against 84 and 95.
+template <int T, bool ROTATE, int NT, int U>
+__global__ __launch_bounds__(NT, NT == 512 ? 4 : 1) void split_caches_kernel(CacheArgs c, int rows, int KB, uint8_t* __restrict__ out,
+                                                          int* __restrict__ shifts, float* __restrict__ energy) {
+  __shared__ uint32_t wtop[NT / 64];
+  __shared__ float wsum[NT / 64];
+  const int tid = threadIdx.x;
+  const long row = blockIdx.x;
+  const bool live = row < rows;
+  const long t = c.start + (live ? row : 0);
+  const int per_head = c.D / 16, half = c.D / 2, units = c.K / 16;
+  float x[U][2][8];
+#pragma unroll
+  for (int u = 0; u < U; ++u) {
+    const int unit = min(tid + u * NT, units - 1);
+    const int lh = unit / per_head, d = 8 * (unit % per_head);
+    const void* base = (const void*)c.layer_ptrs[lh / c.H];
+    const long at = ((long)(lh % c.H) * c.tokens + t) * c.D + d;
+    load_elem8<T>(base, at, x[u][0]);
+    load_elem8<T>(base, at + half, x[u][1]);
+  }
+  uint32_t top = 0;
+  float sum = 0.0f;
+#pragma unroll
+  for (int u = 0; u < U; ++u) {
+    const int unit = min(tid + u * NT, units - 1);
+    const int f = unit / per_head * c.D + 8 * (unit % per_head), d = 8 * (unit % per_head);
+    float m0[8], m1[8];
+    load_elem8<DKV_F32>(c.mean, f, m0);
+    load_elem8<DKV_F32>(c.mean, f + half, m1);
+    if constexpr (ROTATE) {
+      float c0[8], s0[8], c1[8], s1[8];
+      load_elem8<DKV_F32>(c.cos, t * c.D + d, c0);
+      load_elem8<DKV_F32>(c.sin, t * c.D + d, s0);
+      load_elem8<DKV_F32>(c.cos, t * c.D + d + half, c1);
+      load_elem8<DKV_F32>(c.sin, t * c.D + d + half, s1);
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        const float a = x[u][0][i], b = x[u][1][i];
+        x[u][0][i] = derotated(a, -b, c0[i], s0[i], m0[i]);
+        x[u][1][i] = derotated(b, a, c1[i], s1[i], m1[i]);
+      }
+    } else {
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        x[u][0][i] -= m0[i];
+        x[u][1][i] -= m1[i];
+      }
+    }
+    const bool mine = live && tid + u * NT < units;
+#pragma unroll
+    for (int e = 0; e < 2; ++e)
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        x[u][e][i] = mine ? x[u][e][i] : 0.0f;
+        top = max(top, abs_bits(x[u][e][i]));
+        sum = __builtin_fmaf(x[u][e][i], x[u][e][i], sum);
+      }
+  }
+#pragma unroll
+  for (int o = 1; o < 64; o <<= 1) {
+    top = max(top, (uint32_t)__shfl_xor((int)top, o));
+    sum += __shfl_xor(sum, o);
+  }
+  if ((tid & 63) == 0) {
+    wtop[tid >> 6] = top;
+    wsum[tid >> 6] = sum;
+  }
+  __syncthreads();
+#pragma unroll
+  for (int w = 0; w < NT / 64; ++w) top = max(top, wtop[w]);
+  const int shift = row_shift(top);
+  if (tid == 0) {
+    shifts[row] = shift;
+    if (energy && live) {
+      float s = 0.0f;
+#pragma unroll
+      for (int w = 0; w < NT / 64; ++w) s += wsum[w];
+      energy[row] = s;
+    }
+  }
+  half8 hi, lo;
+#pragma unroll
+  for (int u = 0; u < U; ++u) {
+    const int unit = tid + u * NT;
+    if (unit >= units) break;
+    const int oct = unit / per_head * (c.D / 8) + unit % per_head;
+#pragma unroll
+    for (int e = 0; e < 2; ++e) {
+      split8(x[u][e], shift, hi, lo);
+      store_octet(out, row, oct + e * (half / 8), KB, hi, lo);
+    }
+  }
+  const half8 zero = {0, 0, 0, 0, 0, 0, 0, 0};
+  for (int o = c.K / 8 + tid; o < KB * 4; o += NT) store_octet(out, row, o, KB, zero, zero);
+}
+
 // Rows of A or B that hold an infinity or a NaN have no split form: their products in plain fp32.
-__global__ __launch_bounds__(256) void special_rows_kernel(const float* __restrict__ a, long lda, const float* __restrict__ b,
+template <class Rows>
+__global__ __launch_bounds__(256) void special_rows_kernel(Rows a, const float* __restrict__ b,
                                                            long ldb, int b_kn, const float* __restrict__ bias, int M,
                                                            int N, int K, const int* __restrict__ sa,
                                                            const int* __restrict__ sb, const uint32_t* __restrict__ flag,
@@ -403,7 +560,7 @@ __global__ __launch_bounds__(256) void special_rows_kernel(const float* __restri
     for (int n = threadIdx.x; n < N; n += 256) {
       if (!row && sb[n] != kFlagged) continue;
       float s = 0.0f;
-      for (int k = 0; k < K; ++k) s += a[m * lda + k] * (b_kn ? b[k * ldb + n] : b[n * ldb + k]);
+      for (int k = 0; k < K; ++k) s += a.at(m, k) * (b_kn ? b[k * ldb + n] : b[n * ldb + k]);
       c[m * ldc + n] = s + (bias ? bias[n] : 0.0f);
     }
   }
@@ -479,15 +636,17 @@ extern "C" size_t dkv_matmul_f32_workspace_bytes(int64_t M, int64_t N, int64_t K
   return gemm_layout(M, N, K).total;
 }
 
-extern "C" int dkv_matmul_f32(const float* a, int64_t lda, const float* b, int64_t ldb, int32_t b_is_kn,
-                              const float* bias, int64_t M, int64_t N, int64_t K, float* c, int64_t ldc,
-                              void* workspace, size_t workspace_bytes, void* stream) {
-  int rc = check_gemm(M, N, K, "dkv_matmul_f32");
+namespace {
+
+// The product of A's split rows, once `split_a` has launched their split into the workspace.
+template <class Rows, class SplitA>
+int launch_product(const char* what, Rows rows, SplitA&& split_a, const float* b, long ldb, int b_is_kn, const float* bias, long M,
+                   long N, long K, float* c, long ldc, void* workspace, size_t workspace_bytes, void* stream) {
+  int rc = check_gemm(M, N, K, what);
   if (rc) return rc;
-  DKV_REQUIRE(a && b && c, DKV_EINVAL, "dkv_matmul_f32: null pointer");
-  DKV_REQUIRE(lda >= K && ldb >= (b_is_kn ? N : K) && ldc >= N, DKV_ESHAPE, "dkv_matmul_f32: bad row strides");
+  DKV_REQUIRE(ldb >= (b_is_kn ? N : K) && ldc >= N, DKV_ESHAPE, "%s: bad row strides", what);
   const GemmLayout L = gemm_layout(M, N, K);
-  DKV_REQUIRE(workspace && workspace_bytes >= L.total, DKV_EWORKSPACE, "dkv_matmul_f32: workspace %zu B < required %zu B",
+  DKV_REQUIRE(workspace && workspace_bytes >= L.total, DKV_EWORKSPACE, "%s: workspace %zu B < required %zu B", what,
               workspace_bytes, L.total);
   uint8_t* ws = (uint8_t*)workspace;
   hipStream_t st = dkv::as_stream(stream);
@@ -495,7 +654,7 @@ extern "C" int dkv_matmul_f32(const float* a, int64_t lda, const float* b, int64
   uint32_t* top = (uint32_t*)(ws + L.top);
   uint32_t* flag = top + N;
   hipLaunchKernelGGL(clear_kernel, dim3((unsigned)((N + 1 + 255) / 256)), dim3(256), 0, st, top, (int)N + 1);
-  launch_split_rows(a, lda, M, (long)L.mt * kTile, (int)K, L.KB, ws + L.a, sa, nullptr, st);
+  split_a(L, ws + L.a, sa, st);
   if (b_is_kn) {
     hipLaunchKernelGGL(column_top_kernel, dim3((unsigned)((N + 63) / 64 * ((K + 127) / 128))), dim3(256), 0, st, b,
                        ldb, (int)K, (int)N, top);
@@ -504,7 +663,7 @@ extern "C" int dkv_matmul_f32(const float* a, int64_t lda, const float* b, int64
   } else {
     launch_split_rows(b, ldb, N, (long)L.nt * kTile, (int)K, L.KB, ws + L.b, sb, flag, st);
   }
-  rc = dkv::check_launch("dkv_matmul_f32 (split)");
+  rc = dkv::check_launch(what);
   if (rc) return rc;
   GemmArgs g{};
   g.a = ws + L.a;
@@ -524,12 +683,69 @@ extern "C" int dkv_matmul_f32(const float* a, int64_t lda, const float* b, int64
   g.total = L.mt * L.nt * L.splits;
   g.per_xcd = (g.total + 7) / 8;
   hipLaunchKernelGGL(gemm_split_kernel, dim3(8u * (unsigned)g.per_xcd), dim3(512), 0, st, g);
-  rc = dkv::check_launch("dkv_matmul_f32");
+  rc = dkv::check_launch(what);
   if (rc) return rc;
   if (L.splits > 1)
     hipLaunchKernelGGL(sum_splits_kernel, dim3((unsigned)((M * N + 255) / 256)), dim3(256), 0, st,
-                       (const float*)(ws + L.part), L.splits, (int)M, (int)N, bias, c, (long)ldc);
-  hipLaunchKernelGGL(special_rows_kernel, dim3((unsigned)((M + 63) / 64)), dim3(256), 0, st, a, (long)lda, b, (long)ldb, b_is_kn, bias,
-                     (int)M, (int)N, (int)K, sa, sb, flag, c, (long)ldc);
-  return dkv::check_launch("dkv_matmul_f32 (sums)");
+                       (const float*)(ws + L.part), L.splits, (int)M, (int)N, bias, c, ldc);
+  hipLaunchKernelGGL(special_rows_kernel<Rows>, dim3((unsigned)((M + 63) / 64)), dim3(256), 0, st, rows, b, ldb, b_is_kn, bias,
+                     (int)M, (int)N, (int)K, sa, sb, flag, c, ldc);
+  return dkv::check_launch(what);
+}
+
+template <int T, bool ROTATE>
+int launch_project(const CacheArgs& c, const float* b, long ldb, int b_is_kn, long M, long N, float* out, long ldo, float* energy,
+                   void* workspace, size_t workspace_bytes, void* stream) {
+  auto split = [&](const GemmLayout& L, uint8_t* lines, int* sa, hipStream_t st) {
+    const dim3 grid((unsigned)(L.mt * kTile));
+    if (c.K <= 8192)
+      hipLaunchKernelGGL((split_caches_kernel<T, ROTATE, 256, 2>), grid, dim3(256), 0, st, c, (int)M, L.KB, lines, sa, energy);
+    else
+      hipLaunchKernelGGL((split_caches_kernel<T, ROTATE, 512, 4>), grid, dim3(512), 0, st, c, (int)M, L.KB, lines, sa, energy);
+  };
+  return launch_product("dkv_project_caches", CacheRows<T, ROTATE>{c}, split, b, ldb, b_is_kn, nullptr, M, N, c.K, out, ldo,
+                        workspace, workspace_bytes, stream);
+}
+
+}  // namespace
+
+extern "C" int dkv_project_caches(const uint64_t* layer_ptrs, int32_t dtype, int32_t layers, int32_t heads, int32_t tokens,
+                                  int32_t head_dim, const float* cos, const float* sin, const float* mean, int32_t start,
+                                  int32_t end, const float* basis, int64_t ldb, int32_t b_is_kn, int64_t rank, float* out,
+                                  int64_t ldo, float* energy, void* workspace, size_t workspace_bytes, void* stream) {
+  DKV_REQUIRE(layer_ptrs && mean && basis && out, DKV_EINVAL, "dkv_project_caches: null pointer");
+  DKV_REQUIRE((cos == nullptr) == (sin == nullptr), DKV_EINVAL, "dkv_project_caches: cos and sin go together");
+  DKV_REQUIRE(dtype == DKV_F32 || dtype == DKV_F16 || dtype == DKV_BF16, DKV_EINVAL,
+              "dkv_project_caches: dtype %d not supported", dtype);
+  DKV_REQUIRE(layers > 0 && heads > 0 && tokens >= 0 && head_dim > 0 && head_dim % 16 == 0 &&
+                  (long)layers * heads * head_dim <= 32768,
+              DKV_ESHAPE, "dkv_project_caches: bad shape (layers=%d heads=%d tokens=%d head_dim=%d)", layers, heads, tokens,
+              head_dim);
+  DKV_REQUIRE(0 <= start && start < end && end <= tokens, DKV_ESHAPE, "dkv_project_caches: rows %d..%d outside 0..%d", start,
+              end, tokens);
+  const CacheArgs c{layer_ptrs, cos, sin, mean, heads, tokens, head_dim, start, layers * heads * head_dim};
+#define DKV_PROJECT(T_, R_) \
+  return launch_project<T_, R_>(c, basis, ldb, b_is_kn, end - start, rank, out, ldo, energy, workspace, workspace_bytes, stream)
+  if (dtype == DKV_F32) {
+    if (cos) DKV_PROJECT(DKV_F32, true);
+    DKV_PROJECT(DKV_F32, false);
+  } else if (dtype == DKV_F16) {
+    if (cos) DKV_PROJECT(DKV_F16, true);
+    DKV_PROJECT(DKV_F16, false);
+  }
+  if (cos) DKV_PROJECT(DKV_BF16, true);
+  DKV_PROJECT(DKV_BF16, false);
+#undef DKV_PROJECT
+}
+
+extern "C" int dkv_matmul_f32(const float* a, int64_t lda, const float* b, int64_t ldb, int32_t b_is_kn,
+                              const float* bias, int64_t M, int64_t N, int64_t K, float* c, int64_t ldc,
+                              void* workspace, size_t workspace_bytes, void* stream) {
+  DKV_REQUIRE(a && b && c, DKV_EINVAL, "dkv_matmul_f32: null pointer");
+  DKV_REQUIRE(lda >= K, DKV_ESHAPE, "dkv_matmul_f32: bad row strides");
+  auto split = [&](const GemmLayout& L, uint8_t* lines, int* sa, hipStream_t st) {
+    launch_split_rows(a, lda, M, (long)L.mt * kTile, (int)K, L.KB, lines, sa, nullptr, st);
+  };
+  return launch_product("dkv_matmul_f32", PlainRows{a, lda}, split, b, ldb, b_is_kn, bias, M, N, K, c, ldc, workspace,
+                        workspace_bytes, stream);
 }

@@ -702,15 +702,6 @@ DKV_DEVICE float4 load_elem4(const void* base, long idx) {
 
 constexpr int kRowTok = 4;  // tokens per thread
 
-// De-rotation of one element (x cos - rotate_half(x) sin) / (cos^2 + sin^2), minus the mean.
-DKV_DEVICE float derotated(float x, float rh, float c, float s, float mu) {
-#pragma clang fp contract(off)
-  const float num = x * c - rh * s;
-  const float den = c * c + s * s;
-  const float v = num / den;
-  return v - mu;
-}
-
 template <int T, bool ROTATE>
 __global__ __launch_bounds__(256) void centered_rows_kernel(const uint64_t* __restrict__ layer_ptrs, int L, int H,
                                                             int tokens, int D, const float* __restrict__ cos,

@@ -30,7 +30,7 @@ EXPORTS = [
     "dkv_score_workspace_bytes", "dkv_score_begin", "dkv_score_layer", "dkv_topk_workspace_bytes", "dkv_topk",
     "dkv_gather_cold", "dkv_refine_rows", "dkv_wire_pack", "dkv_wire_unpack", "dkv_attend_layer_noalloc",
     "dkv_quantize8", "dkv_quantize8_rungs", "dkv_centered_rows", "dkv_matmul_f32_workspace_bytes", "dkv_matmul_f32",
-    "dkv_ladder_errors", "dkv_ladder_code", "dkv_rows_to_caches", "dkv_copy_tokens", "dkv_outside_tokens",
+    "dkv_ladder_errors", "dkv_ladder_code", "dkv_rows_to_caches", "dkv_copy_tokens", "dkv_outside_tokens", "dkv_project_caches",
 ]
 NOALLOC_MAX_BYTES = 64 << 20  # DKV_NOALLOC_MAX_BYTES: the static workspace of dkv_attend_layer_noalloc
 
@@ -319,6 +319,32 @@ def matmul_f32(a: torch.Tensor, b: torch.Tensor, bias: torch.Tensor | None = Non
                                     c_vp(ptr(bias)), c_i64(m), c_i64(n), c_i64(k), c_vp(ptr(out)), c_i64(n),
                                     c_vp(ptr(workspace)), c_sz(need), c_vp(stream_handle())), "dkv_matmul_f32")
     return out
+
+
+def project_caches(tensors, cos, sin, mean, start: int, end: int, basis, with_energy: bool):
+    """Centred rows of per-layer caches [1, H, T, D] times basis f32 [L*H*D, rank]: f32 [end - start, rank], and the rows'
+    energies [end - start] or None (dkv_project_caches; contiguous 16-byte aligned tensors, cos and sin for keys)."""
+    first = tensors[0]
+    _, heads, tokens, dim = first.shape
+    (k, n), m = basis.shape, end - start
+    kn = basis.stride(1) == 1 and basis.stride(0) >= n
+    if not kn and not (basis.stride(0) == 1 and basis.stride(1) >= k):
+        basis, kn = basis.contiguous(), True
+    out = torch.empty(m, n, dtype=torch.float32, device=first.device)
+    energy = torch.empty(m, dtype=torch.float32, device=first.device) if with_energy else None
+    need = lib().dkv_matmul_f32_workspace_bytes(c_i64(m), c_i64(n), c_i64(k))
+    if need == 0:
+        _check(-2, "dkv_matmul_f32_workspace_bytes")
+    workspace = torch.empty(need, dtype=torch.uint8, device=first.device)
+    table = _pointer_table(tensors)
+    with torch.cuda.device(first.device):
+        _check(lib().dkv_project_caches(c_vp(ptr(table)), c_i32(dtype_code(first.dtype)), c_i32(len(tensors)), c_i32(heads),
+                                        c_i32(tokens), c_i32(dim), c_vp(ptr(cos)), c_vp(ptr(sin)), c_vp(ptr(mean)),
+                                        c_i32(start), c_i32(end), c_vp(basis.data_ptr()),
+                                        c_i64(basis.stride(0) if kn else basis.stride(1)), c_i32(kn), c_i64(n), c_vp(ptr(out)),
+                                        c_i64(n), c_vp(ptr(energy)), c_vp(ptr(workspace)), c_sz(need), c_vp(stream_handle())),
+               "dkv_project_caches")
+    return out, energy
 
 
 def quantize8(coef, codes, low, span, errors=None) -> None:

@@ -136,7 +136,7 @@ def _fp16_rows(wire: torch.Tensor, at: int, rows: int, features: int) -> torch.T
 
 def encode_bytes(codec, keys, values, choice: dict, exact_recent: int) -> bytes:
     """Serialize a compressed cache; ``choice`` is ``codec.last_choice`` (scripts/kvtc_storage.py:42-79)."""
-    from kvtc import float_product, quantize_groups_codes, rope_tables, token_matrix
+    from kvtc import quantize_groups_codes, rope_tables, token_matrix
 
     device = codec.device
     tokens = keys[0].shape[2]
@@ -159,7 +159,7 @@ def encode_bytes(codec, keys, values, choice: dict, exact_recent: int) -> bytes:
     for kind, tensors, rungs, layout in prepared:
         stream = codec.streams[kind]
         # compress's arithmetic
-        coefficients = float_product(codec.centered(tensors, kind, cos, sin, start, end), stream.basis)
+        coefficients = codec.project(tensors, kind, cos, sin, start, end)
         wire[layout.rung_ids:layout.rung_ids + middle] = rungs.to(torch.uint8)
         groups = coefficients.shape[1] // codec.group
         codes = torch.zeros(middle, groups, codec.group, dtype=torch.uint8, device=device)

@@ -229,6 +229,16 @@ int dkv_copy_tokens(const uint64_t* src_ptrs, const uint64_t* dst_ptrs, int32_t 
 int dkv_outside_tokens(const uint64_t* layer_ptrs, void* out, int32_t dtype, int32_t layers, int32_t heads,
                        int32_t tokens, int32_t head_dim, int32_t skip, int32_t skip_len, void* stream);
 
+/* The encoders' projection straight from the caches: dkv_centered_rows' rows (its arguments and arithmetic; caches,
+ * cos, sin and mean 16-byte aligned, head_dim a multiple of 16, layers * heads * head_dim at most 32,768, at least one row)
+ * times basis [layers*heads*head_dim][rank] (b_is_kn and ldb as dkv_matmul_f32's) -> out f32 [end - start][rank]
+ * of row stride ldo, with dkv_matmul_f32's arithmetic and no rows in memory; energy, unless NULL, f32
+ * [end - start]: each row's sum of squares.  Workspace: dkv_matmul_f32_workspace_bytes(end - start, rank, columns). */
+int dkv_project_caches(const uint64_t* layer_ptrs, int32_t dtype, int32_t layers, int32_t heads, int32_t tokens,
+                       int32_t head_dim, const float* cos, const float* sin, const float* mean, int32_t start,
+                       int32_t end, const float* basis, int64_t ldb, int32_t b_is_kn, int64_t rank, float* out,
+                       int64_t ldo, float* energy, void* workspace, size_t workspace_bytes, void* stream);
+
 /* ---- float32 products on the fp16 matrix cores -----------------------------
  * C[m][n] = sum_k A[m][k] B[n][k] + bias[n] (bias may be NULL), all float32:
  * the projections onto a PCA basis and back (scripts/kvtc.py:88-97, :189;

@@ -84,3 +84,30 @@ def test_float_product_route():
     assert kvtc.float_product(a.half(), b.half()).dtype == torch.float16
     out, tangent = torch.func.jvp(lambda x: kvtc.float_product(x, b), (a,), (a,))
     assert torch.equal(out, a @ b) and torch.equal(tangent, a @ b)
+
+
+@pytest.mark.parametrize("layers,heads,dim,rank,dtype,start,end,kind", [
+    (2, 8, 64, 256, torch.float16, 4, 269, "key"),       # 1,024 columns: idle threads, a row tile and a remainder
+    (28, 8, 128, 192, torch.bfloat16, 0, 33, "key"),     # 28,672 columns, no sinks, 192 of 256 basis columns
+    (16, 8, 64, 1024, torch.float32, 4, 260, "value"),   # 8,192 columns: every thread of the small workgroup
+    (3, 5, 48, 130, torch.float16, 2, 300, "value"),     # 720 columns: no whole block of 64
+])
+def test_projection_from_caches_matches_rows(layers, heads, dim, rank, dtype, start, end, kind):
+    """dkv_project_caches equals dkv_matmul_f32 of dkv_centered_rows' rows bit for bit (same pieces, same sums), also
+    in a row with an infinity, and its energies are the rows' (at most `columns` roundings of a positive sum)."""
+    import dkv_hip
+
+    tokens, width = end + 7, layers * heads * dim
+    print(f"[case] projection from caches {layers}x{heads}x{dim} rank {rank} {dtype} {start}..{end} {kind}", flush=True)
+    g = torch.Generator(DEV).manual_seed(rank)
+    caches = [torch.randn(1, heads, tokens, dim, generator=g, device=DEV).to(dtype) for _ in range(layers)]
+    caches[1][0, 1, start + 5, 3] = float("inf")
+    mean = torch.randn(width, generator=g, device=DEV)
+    cos, sin = (torch.randn(tokens, dim, generator=g, device=DEV) for _ in range(2)) if kind == "key" else (None, None)
+    basis = torch.randn(width, rank, generator=g, device=DEV) / width ** 0.5
+    rows = torch.empty(end - start, width, device=DEV)
+    dkv_hip.centered_rows(caches, cos, sin, mean, start, end, rows)
+    for b in (basis, basis.T.contiguous().T):
+        got, energy = dkv_hip.project_caches(caches, cos, sin, mean, start, end, b, True)
+        assert torch.equal(torch.nan_to_num(got), torch.nan_to_num(dkv_hip.matmul_f32(rows, b)))
+    assert torch.allclose(energy.double(), rows.double().square().sum(1), rtol=width * 2.0 ** -24, atol=0.0)
