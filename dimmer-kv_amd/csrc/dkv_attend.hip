@@ -303,15 +303,6 @@ constexpr float kLn2 = 0.693147180559945309f;
 DKV_DEVICE long sub_index(long row, int t, int nsub) { return ((row >> 3) * nsub + t) * 8 + (row & 7); }
 
 
-// ---------------------------------------------------------------------------
-// Softmax statistics of the compressed part of sequence b, row `row`.
-// ---------------------------------------------------------------------------
-DKV_DEVICE int tiles_before(const int32_t* cu, int b, int tile) {
-  int base = 0;
-  for (int i = 0; i < b; ++i) base += (cu[i + 1] - cu[i] + tile - 1) / tile;
-  return base;
-}
-
 // Part `part` of `parts` of the values as operand lines (many-row decodes): a wave takes one group's 64 components
 // (a lane each) over a 64-slot block: 64 codes and 64 (scale, offset) pairs, the pairs through its LDS area.  The
 // values of a sequence's group are scaled by the power of two that brings their bound into [2^14, 2^15), so a group

@@ -299,20 +299,55 @@ DKV_DEVICE void ladder_half_f16(const uint32_t (&cw)[8], uint32_t header, uint32
   }
 }
 
+// Inclusive sum over a wave's lanes (all active): within rows of 16 lanes, then rows 1 and 3, then the upper half.
+template <int CTRL, int ROWS>
+DKV_DEVICE int scan_step(int v) {
+  return v + __builtin_amdgcn_update_dpp(0, v, CTRL, ROWS, 0xf, false);
+}
+
+DKV_DEVICE int wave_scan(int v) {
+  v = scan_step<0x111, 0xf>(v);  // row_shr 1, 2, 4, 8
+  v = scan_step<0x112, 0xf>(v);
+  v = scan_step<0x114, 0xf>(v);
+  v = scan_step<0x118, 0xf>(v);
+  v = scan_step<0x142, 0xa>(v);  // lane 15 of rows 0 and 2 to the next row
+  return scan_step<0x143, 0xc>(v);  // lane 31 to the upper half
+}
+
+// Tiles of `tile` tokens in the sequence of this lane among b0 .. b0 + 63 (none at `end` and past it).
+DKV_DEVICE int lane_tiles(const int32_t* cu, int b0, int end, int tile) {
+  const int b = b0 + (int)__lane_id();
+  const int lo = cu[min(b, end - 1)], hi = cu[min(b, end - 1) + 1];
+  return b < end ? (hi - lo + tile - 1) / tile : 0;
+}
+
 // Sequence/tile lookup from cu_seqlens without a host-built table: returns
-// the sequence b and the tile index inside it for a global tile id, where
-// sequence b has ceil(len_b / tile) tiles.  One sequence (n_total tokens)
-// needs no load.
+// the sequence b and the tile index inside it for a global tile id (the same in
+// every lane of a wave, all of them active), where sequence b has ceil(len_b / tile)
+// tiles.  One sequence (n_total tokens) needs no load.  A wave takes 64 sequences at
+// once, a lane each: a loop over them is a chain of loads and divisions, 3 us for 32
+// sequences at the head of every workgroup.
 DKV_DEVICE int2 find_tile(const int32_t* cu, int batch, int n_total, int tile, int gid) {
   if (batch == 1) return make_int2(gid < (n_total + tile - 1) / tile ? 0 : -1, gid);
-  int base = 0;
-  for (int b = 0; b < batch; ++b) {
-    const int len = cu[b + 1] - cu[b];
-    const int nt = (len + tile - 1) / tile;
-    if (gid < base + nt) return make_int2(b, gid - base);
-    base += nt;
+  int left = __builtin_amdgcn_readfirstlane(gid);
+  for (int b0 = 0; b0 < batch; b0 += 64) {
+    const int nt = lane_tiles(cu, b0, batch, tile), upto = wave_scan(nt);
+    const unsigned long long past = __ballot(upto > left);
+    if (past != 0) {
+      const int k = __builtin_ctzll(past);
+      return make_int2(b0 + k, left - __builtin_amdgcn_readlane(upto - nt, k));
+    }
+    left -= __builtin_amdgcn_readlane(upto, 63);
   }
   return make_int2(-1, 0);
+}
+
+// Tiles of the sequences before b (the same in every lane of a wave, all of them active).
+DKV_DEVICE int tiles_before(const int32_t* cu, int b, int tile) {
+  const int end = __builtin_amdgcn_readfirstlane(b);
+  int base = 0;
+  for (int b0 = 0; b0 < end; b0 += 64) base += __builtin_amdgcn_readlane(wave_scan(lane_tiles(cu, b0, end, tile)), 63);
+  return base;
 }
 
 // De-rotation of one element (x cos - rotate_half(x) sin) / (cos^2 + sin^2), minus the mean.
