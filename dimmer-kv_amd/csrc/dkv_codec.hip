@@ -241,6 +241,41 @@ __global__ __launch_bounds__(256) void copy_tokens_kernel(const uint64_t* __rest
   ((uint4*)dst[l])[at] = ((const uint4*)src[l])[at];
 }
 
+// Which groups some row uses (scripts/kvtc.py:88-97): live[g] = 1 where any row's 64 coefficients of group g are not all
+// 0 (a NaN is not 0); live starts at 0.  CODES: the coefficients are code * scale + low of ladder codes, each operation
+// rounded on its own (scripts/kvtc_storage.py:119), and are written on the way.  16 lanes per (row, group), four
+// members each.  Bound by its bytes: 5,964 x 2,048 from codes 14 us, 4,061 x 2,048 of coefficients 8 (4.2 TB/s); torch took
+// 56 us for the latter's reduction alone, and three passes more for the former's coefficients.
+template <bool CODES>
+__global__ __launch_bounds__(256) void live_groups_kernel(const uint8_t* __restrict__ codes, const uint16_t* __restrict__ low,
+                                                          const uint16_t* __restrict__ scale, float* __restrict__ coef,
+                                                          long ngroups, int G, int32_t* __restrict__ live) {
+  const long tg = (long)blockIdx.x * 16 + (threadIdx.x >> 4);
+  const int j = threadIdx.x & 15;
+  const bool ok = tg < ngroups;
+  const long at = (ok ? tg : 0) * 64 + 4 * j;
+  float4 v;
+  if constexpr (CODES) {
+    uint32_t c;
+    __builtin_memcpy(&c, codes + at, 4);
+    const float s = half_bits_to_float(scale[ok ? tg : 0]), l = half_bits_to_float(low[ok ? tg : 0]);
+    {
+#pragma clang fp contract(off)
+      v.x = (float)(c & 0xffu) * s + l;
+      v.y = (float)((c >> 8) & 0xffu) * s + l;
+      v.z = (float)((c >> 16) & 0xffu) * s + l;
+      v.w = (float)(c >> 24) * s + l;
+    }
+    if (ok) *(float4*)(coef + at) = v;
+  } else {
+    v = *(const float4*)(coef + at);
+  }
+  const bool any = ok && (v.x != 0.0f || v.y != 0.0f || v.z != 0.0f || v.w != 0.0f);
+  const unsigned long long row = __ballot(any) >> (threadIdx.x & 48) & 0xffffull;
+  // one lane a group, and only until the flag is seen: every writer stores the same 1
+  if (j == 0 && row != 0 && live[(int)(tg % G)] == 0) live[(int)(tg % G)] = 1;
+}
+
 // The same tokens gathered into one buffer [layers][H][tokens - skip_len][row], the layers' addresses in the launch's
 // arguments.  A progressive encode's sinks and recent window (16 layers x 8 heads x 36 tokens of 128 bytes): one launch
 // a stream in place of a concatenation a layer, 16 launches of 7.4 us.
@@ -262,6 +297,22 @@ __global__ __launch_bounds__(256) void outside_tokens_kernel(LayerPtrs src, uint
 }
 
 }  // namespace
+
+extern "C" int dkv_live_groups(const uint8_t* codes, const uint16_t* low, const uint16_t* scale, float* coef, int64_t n,
+                               int32_t groups, int32_t* live, void* stream) {
+  DKV_REQUIRE(n >= 0 && groups > 0 && n < (1L << 31), DKV_ESHAPE, "dkv_live_groups: bad shape (n=%ld groups=%d)", (long)n, groups);
+  if (n == 0) return DKV_OK;
+  DKV_REQUIRE(coef && live && (!codes || (low && scale)), DKV_EINVAL, "dkv_live_groups: null pointer");
+  const long ngroups = (long)n * groups, blocks = (ngroups + 15) / 16;
+  DKV_REQUIRE(blocks < (1L << 31), DKV_ESHAPE, "dkv_live_groups: too many rows");
+  if (codes)
+    hipLaunchKernelGGL(live_groups_kernel<true>, dim3((unsigned)blocks), dim3(256), 0, dkv::as_stream(stream), codes, low, scale,
+                       coef, ngroups, groups, live);
+  else
+    hipLaunchKernelGGL(live_groups_kernel<false>, dim3((unsigned)blocks), dim3(256), 0, dkv::as_stream(stream), codes, low, scale,
+                       coef, ngroups, groups, live);
+  return dkv::check_launch("dkv_live_groups");
+}
 
 extern "C" int dkv_outside_tokens(const uint64_t* layer_ptrs, void* out, int32_t dtype, int32_t layers, int32_t heads,
                                   int32_t tokens, int32_t head_dim, int32_t skip, int32_t skip_len, void* stream) {

@@ -30,7 +30,7 @@ EXPORTS = [
     "dkv_score_workspace_bytes", "dkv_score_begin", "dkv_score_layer", "dkv_topk_workspace_bytes", "dkv_topk",
     "dkv_gather_cold", "dkv_refine_rows", "dkv_wire_pack", "dkv_wire_unpack", "dkv_attend_layer_noalloc",
     "dkv_quantize8", "dkv_quantize8_rungs", "dkv_centered_rows", "dkv_matmul_f32_workspace_bytes", "dkv_matmul_f32",
-    "dkv_ladder_errors", "dkv_ladder_code", "dkv_rows_to_caches", "dkv_copy_tokens", "dkv_outside_tokens", "dkv_project_caches",
+    "dkv_ladder_errors", "dkv_ladder_code", "dkv_rows_to_caches", "dkv_copy_tokens", "dkv_outside_tokens", "dkv_project_caches", "dkv_live_groups",
 ]
 NOALLOC_MAX_BYTES = 64 << 20  # DKV_NOALLOC_MAX_BYTES: the static workspace of dkv_attend_layer_noalloc
 
@@ -319,6 +319,16 @@ def matmul_f32(a: torch.Tensor, b: torch.Tensor, bias: torch.Tensor | None = Non
                                     c_vp(ptr(bias)), c_i64(m), c_i64(n), c_i64(k), c_vp(ptr(out)), c_i64(n),
                                     c_vp(ptr(workspace)), c_sz(need), c_vp(stream_handle())), "dkv_matmul_f32")
     return out
+
+
+def live_groups(coef, codes=None, low=None, scale=None) -> torch.Tensor:
+    """bool [G]: the 64-wide groups of coef f32 [n, 64G] that some row uses.  With ladder codes u8 [n, G, 64], low and scale
+    f16 [n, G], coef is written first: code * scale + low."""
+    n, groups = coef.shape[0], coef.shape[1] // 64
+    live = torch.zeros(groups, dtype=torch.int32, device=coef.device)
+    _check(lib().dkv_live_groups(c_vp(ptr(codes)), c_vp(ptr(low)), c_vp(ptr(scale)), c_vp(ptr(coef)), c_i64(n), c_i32(groups),
+                                 c_vp(ptr(live)), c_vp(stream_handle())), "dkv_live_groups")
+    return live.bool()
 
 
 def project_caches(tensors, cos, sin, mean, start: int, end: int, basis, with_energy: bool):

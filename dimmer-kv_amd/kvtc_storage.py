@@ -243,9 +243,18 @@ class _Parsed:
 
     def coefficients(self, kind: str) -> torch.Tensor:
         """code * scale + shift in float32 (scripts/kvtc_storage.py:119), zeros where nothing is stored."""
+        return self.coefficients_and_live(kind)[0]
+
+    def coefficients_and_live(self, kind: str):
+        """``coefficients(kind)`` and, from the same HIP pass where there is one, the groups some token uses (else None)."""
+        from kvtc import _plain_gpu
+
         codes, low, scale = self.codes[kind]
+        if codes.shape[0] > 0 and codes.shape[2] == 64 and _plain_gpu(codes, low, scale):
+            values = torch.empty(codes.shape[0], codes.shape[1] * 64, dtype=torch.float32, device=codes.device)
+            return values, dkv_hip.live_groups(values, codes, low, scale)
         values = codes.float() * scale.float().unsqueeze(2) + low.float().unsqueeze(2)
-        return values.reshape(codes.shape[0], -1)
+        return values.reshape(codes.shape[0], -1), None
 
 
 def decode_bytes(codec, data: bytes, dtype=torch.float16):
@@ -259,7 +268,8 @@ def decode_bytes(codec, data: bytes, dtype=torch.float16):
     in_kernel = dtype in (torch.float16, torch.bfloat16, torch.float32) and codec.head_dim % 8 == 0
     out = {}
     for kind in ("key", "value"):
-        rows = inverse_transform(p.coefficients(kind), codec.streams[kind], codec.group)
+        coefficients, live = p.coefficients_and_live(kind)
+        rows = inverse_transform(coefficients, codec.streams[kind], codec.group, live)
         idx, stored = p.exact_rows[kind]
         if stored is not None:
             rows[idx] = stored

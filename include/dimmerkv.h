@@ -229,6 +229,12 @@ int dkv_copy_tokens(const uint64_t* src_ptrs, const uint64_t* dst_ptrs, int32_t 
 int dkv_outside_tokens(const uint64_t* layer_ptrs, void* out, int32_t dtype, int32_t layers, int32_t heads,
                        int32_t tokens, int32_t head_dim, int32_t skip, int32_t skip_len, void* stream);
 
+/* live i32 [groups] (zero at entry): 1 where some of the n rows of coef f32 [n][64*groups] (16-byte aligned) uses the
+ * group, i.e. has a coefficient other than 0 in it.  With codes u8 [n][groups][64], low and scale f16 [n][groups], coef
+ * is first written: code * scale + low (scripts/kvtc_storage.py:119). */
+int dkv_live_groups(const uint8_t* codes, const uint16_t* low, const uint16_t* scale, float* coef, int64_t n,
+                    int32_t groups, int32_t* live, void* stream);
+
 /* The encoders' projection straight from the caches: dkv_centered_rows' rows (its arguments and arithmetic; caches,
  * cos, sin and mean 16-byte aligned, head_dim a multiple of 16, layers * heads * head_dim at most 32,768, at least one row)
  * times basis [layers*heads*head_dim][rank] (b_is_kn and ldb as dkv_matmul_f32's) -> out f32 [end - start][rank]

@@ -84,3 +84,28 @@ def test_rebuilt_caches_match_from_matrix(shape, tokens, span, dtype, monkeypatc
             want = codec._rebuilt_caches(kind, None, originals, span, cos, sin)
         for a, b in zip(got, want):
             assert a.dtype == b.dtype == dtype and torch.equal(a, b)
+
+
+@pytest.mark.parametrize("groups,tokens", [(1, 1), (7, 33), (32, 130)])
+def test_live_groups_match_torch(groups, tokens):
+    """Unused groups, one whose only entry is the last row's last, one of negative zeros, a NaN; and the coefficients of
+    ladder codes bit for bit."""
+    import dkv_hip
+
+    print(f"[case] live groups G={groups} n={tokens}", flush=True)
+    g = torch.Generator(DEV).manual_seed(groups)
+    coef = torch.randn(tokens, groups * 64, generator=g, device=DEV)
+    for k in range(groups):
+        if k % 3 != 1:
+            coef[:, k * 64:(k + 1) * 64] = -0.0 if k % 2 else 0.0
+    coef[-1, -1] = float("nan") if groups == 7 else 2.0
+    want = coef.reshape(tokens, -1, 64).ne(0).any(dim=2).any(dim=0)
+    assert torch.equal(dkv_hip.live_groups(coef), want)
+    codes = torch.randint(0, 256, (tokens, groups, 64), generator=g, device=DEV, dtype=torch.uint8)
+    low, scale = (torch.randn(tokens, groups, generator=g, device=DEV).half() for _ in range(2))
+    codes[:, 0], low[:, 0] = 0, 0.0
+    values = codes.float() * scale.float().unsqueeze(2) + low.float().unsqueeze(2)
+    got = torch.empty(tokens, groups * 64, device=DEV)
+    live = dkv_hip.live_groups(got, codes, low, scale)
+    assert torch.equal(got.view(torch.int32), values.reshape(tokens, -1).view(torch.int32))
+    assert torch.equal(live, values.ne(0).any(dim=2).any(dim=0))
