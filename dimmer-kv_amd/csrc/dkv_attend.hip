@@ -2008,10 +2008,10 @@ __global__ __launch_bounds__(kDecodeSlots) void decode_codes_kernel(DecodeArgs k
                                                                     float2* vaff, float* vtop, uint32_t* lines_valid,
                                                                     int key_blocks) {
   extern __shared__ int2 tab[];
-  if (blockIdx.x == gridDim.x - 1 && threadIdx.x == 0 && lines_valid) *lines_valid = 0u;
-  if ((int)blockIdx.x < key_blocks)
+  if ((int)blockIdx.x < key_blocks) {
     decode_keys_block(k, tab, blockIdx.x);
-  else
+    if (blockIdx.x == 0 && threadIdx.x == 0 && lines_valid) *lines_valid = 0u;
+  } else
     decode_values_block(v, vcodes, vaff, vtop, tab, blockIdx.x - key_blocks);
 }
 

@@ -328,7 +328,8 @@ DKV_DEVICE int lane_tiles(const int32_t* cu, int b0, int end, int tile) {
 // once, a lane each: a loop over them is a chain of loads and divisions, 3 us for 32
 // sequences at the head of every workgroup.
 DKV_DEVICE int2 find_tile(const int32_t* cu, int batch, int n_total, int tile, int gid) {
-  if (batch == 1) return make_int2(gid < (n_total + tile - 1) / tile ? 0 : -1, gid);
+  // (one sequence is the latency-bound case: the lookup's code lies out of its way)
+  if (__builtin_expect(batch == 1, 1)) return make_int2(gid < (n_total + tile - 1) / tile ? 0 : -1, gid);
   int left = __builtin_amdgcn_readfirstlane(gid);
   for (int b0 = 0; b0 < batch; b0 += 64) {
     const int nt = lane_tiles(cu, b0, batch, tile), upto = wave_scan(nt);
@@ -346,7 +347,7 @@ DKV_DEVICE int2 find_tile(const int32_t* cu, int batch, int n_total, int tile, i
 DKV_DEVICE int tiles_before(const int32_t* cu, int b, int tile) {
   const int end = __builtin_amdgcn_readfirstlane(b);
   int base = 0;
-  for (int b0 = 0; b0 < end; b0 += 64) base += __builtin_amdgcn_readlane(wave_scan(lane_tiles(cu, b0, end, tile)), 63);
+  for (int b0 = 0; __builtin_expect(b0 < end, 0); b0 += 64) base += __builtin_amdgcn_readlane(wave_scan(lane_tiles(cu, b0, end, tile)), 63);
   return base;
 }
 
