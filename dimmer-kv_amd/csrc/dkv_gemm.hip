@@ -12,7 +12,7 @@
 //
 // Three fp16 products run at a third of the fp16 rate (about 1.4 PFLOP/s here), against 0.15 PFLOP/s of
 // the float32 matrix instructions.  16,348 x 2,048 x 28,672 (the projection of a 16K-token 3B cache): 5,190 us
-// with the splitting, 1.11 PFLOP/s of fp16 products, against 12,440 us of the library's float32 product (5,030
+// with the splitting, 1.11 PFLOP/s of fp16 products, against 12,440 us of the library's float32 product (5,090 to 5,230
 // straight from the caches, with the 627 us of their centred rows in it);
 // 4,061 x 28,672 x 2,048 (back): 1,295 against 3,500 us.  Error against float64 2.0e-6 and 5.0e-7, against the
 // library's 3.0e-6 and 8.1e-7.
