@@ -143,6 +143,11 @@ def stream_handle() -> int:
     return torch.cuda.current_stream().cuda_stream
 
 
+def _on_device_of(t: torch.Tensor):
+    """``t``'s GPU as the current device: ``stream_handle`` is then the stream that orders the work on its memory."""
+    return torch.cuda.device(t.device)
+
+
 def dtype_code(dtype: torch.dtype) -> int:
     if dtype not in _DTYPE:
         raise ValueError(f"unsupported dtype {dtype}")
@@ -216,18 +221,20 @@ def centered_rows(tensors, cos, sin, mean, start: int, end: int, out) -> None:
     need(mean, "mean", lambda sh: sh == (width,), f"[{width}]")
     need(out, "out", lambda sh: sh == (end - start, width), f"[{end - start}, {width}]")
     ptrs = torch.tensor([ptr(t) for t in tensors], dtype=torch.int64).to(first.device)
-    _check(lib().dkv_centered_rows(c_vp(ptr(ptrs)), c_i32(_DTYPE[first.dtype]), c_i32(len(tensors)), c_i32(heads),
-                                   c_i32(tokens), c_i32(head_dim), c_vp(ptr(cos)), c_vp(ptr(sin)), c_vp(ptr(mean)),
-                                   c_i32(start), c_i32(end), c_vp(ptr(out)), c_vp(stream_handle())),
-           "dkv_centered_rows")
+    with _on_device_of(first):
+        _check(lib().dkv_centered_rows(c_vp(ptr(ptrs)), c_i32(_DTYPE[first.dtype]), c_i32(len(tensors)), c_i32(heads),
+                                       c_i32(tokens), c_i32(head_dim), c_vp(ptr(cos)), c_vp(ptr(sin)), c_vp(ptr(mean)),
+                                       c_i32(start), c_i32(end), c_vp(ptr(out)), c_vp(stream_handle())),
+               "dkv_centered_rows")
 
 
 def ladder_errors(coef, bits) -> torch.Tensor:
     """coef f32 [n, 64G], bits u8 [R, G] -> squared quantization error of every token at every rung [n, R]."""
     rungs, groups = bits.shape
     errors = torch.empty(coef.shape[0], rungs, dtype=torch.float32, device=coef.device)
-    _check(lib().dkv_ladder_errors(c_vp(ptr(coef)), c_i32(coef.shape[0]), c_i32(groups), c_vp(ptr(bits)), c_i32(rungs),
-                                   c_vp(ptr(errors)), c_vp(stream_handle())), "dkv_ladder_errors")
+    with _on_device_of(coef):
+        _check(lib().dkv_ladder_errors(c_vp(ptr(coef)), c_i32(coef.shape[0]), c_i32(groups), c_vp(ptr(bits)), c_i32(rungs),
+                                       c_vp(ptr(errors)), c_vp(stream_handle())), "dkv_ladder_errors")
     return errors
 
 
@@ -239,9 +246,10 @@ def ladder_code(coef, bits, level):
     codes = torch.empty(n, groups, features // groups, dtype=torch.uint8, device=coef.device)
     low = torch.empty(n, groups, dtype=torch.float16, device=coef.device)
     scale = torch.empty_like(low)
-    _check(lib().dkv_ladder_code(c_vp(ptr(coef)), c_i32(n), c_i32(groups), c_vp(ptr(bits)), c_i32(rungs), c_vp(ptr(level)),
-                                 c_vp(ptr(decoded)), c_vp(ptr(codes)), c_vp(ptr(low)), c_vp(ptr(scale)),
-                                 c_vp(stream_handle())), "dkv_ladder_code")
+    with _on_device_of(coef):
+        _check(lib().dkv_ladder_code(c_vp(ptr(coef)), c_i32(n), c_i32(groups), c_vp(ptr(bits)), c_i32(rungs), c_vp(ptr(level)),
+                                     c_vp(ptr(decoded)), c_vp(ptr(codes)), c_vp(ptr(low)), c_vp(ptr(scale)),
+                                     c_vp(stream_handle())), "dkv_ladder_code")
     return decoded, codes, low, scale
 
 
@@ -264,19 +272,21 @@ def rows_to_caches(rows, caches, first: int, gap_start: int, gap_len: int, cos=N
     head = caches[0]
     _, heads, tokens, dim = head.shape
     table = _pointer_table(caches)
-    _check(lib().dkv_rows_to_caches(c_vp(ptr(rows)), c_i32(rows.shape[0]), c_i32(first), c_i32(gap_start), c_i32(gap_len),
-                                    c_vp(ptr(table)), c_i32(dtype_code(head.dtype)), c_i32(len(caches)), c_i32(heads),
-                                    c_i32(tokens), c_i32(dim), c_vp(ptr(cos)), c_vp(ptr(sin)), c_vp(stream_handle())),
-           "dkv_rows_to_caches")
+    with _on_device_of(head):
+        _check(lib().dkv_rows_to_caches(c_vp(ptr(rows)), c_i32(rows.shape[0]), c_i32(first), c_i32(gap_start), c_i32(gap_len),
+                                        c_vp(ptr(table)), c_i32(dtype_code(head.dtype)), c_i32(len(caches)), c_i32(heads),
+                                        c_i32(tokens), c_i32(dim), c_vp(ptr(cos)), c_vp(ptr(sin)), c_vp(stream_handle())),
+               "dkv_rows_to_caches")
 
 
 def copy_tokens(src, dst, skip: int, skip_len: int) -> None:
     """Every token outside [skip, skip + skip_len) of per-layer caches [1, H, T, D] (contiguous, one dtype) into others."""
     _, heads, tokens, dim = src[0].shape
     a, b = _pointer_table(src), _pointer_table(dst)
-    _check(lib().dkv_copy_tokens(c_vp(ptr(a)), c_vp(ptr(b)), c_i32(dtype_code(src[0].dtype)), c_i32(len(src)), c_i32(heads),
-                                 c_i32(tokens), c_i32(dim), c_i32(skip), c_i32(skip_len), c_vp(stream_handle())),
-           "dkv_copy_tokens")
+    with _on_device_of(src[0]):
+        _check(lib().dkv_copy_tokens(c_vp(ptr(a)), c_vp(ptr(b)), c_i32(dtype_code(src[0].dtype)), c_i32(len(src)), c_i32(heads),
+                                     c_i32(tokens), c_i32(dim), c_i32(skip), c_i32(skip_len), c_vp(stream_handle())),
+               "dkv_copy_tokens")
 
 
 def outside_tokens(src, skip: int, skip_len: int) -> torch.Tensor:
@@ -285,9 +295,10 @@ def outside_tokens(src, skip: int, skip_len: int) -> torch.Tensor:
     _, heads, tokens, dim = src[0].shape
     out = torch.empty(len(src), 1, heads, tokens - skip_len, dim, dtype=src[0].dtype, device=src[0].device)
     table = (c_i64 * len(src))(*[ptr(t) for t in src])
-    _check(lib().dkv_outside_tokens(table, c_vp(ptr(out)), c_i32(dtype_code(out.dtype)), c_i32(len(src)), c_i32(heads),
-                                    c_i32(tokens), c_i32(dim), c_i32(skip), c_i32(skip_len), c_vp(stream_handle())),
-           "dkv_outside_tokens")
+    with _on_device_of(out):
+        _check(lib().dkv_outside_tokens(table, c_vp(ptr(out)), c_i32(dtype_code(out.dtype)), c_i32(len(src)), c_i32(heads),
+                                        c_i32(tokens), c_i32(dim), c_i32(skip), c_i32(skip_len), c_vp(stream_handle())),
+               "dkv_outside_tokens")
     return out
 
 
@@ -314,7 +325,7 @@ def matmul_f32(a: torch.Tensor, b: torch.Tensor, bias: torch.Tensor | None = Non
     if need == 0:
         _check(-2, "dkv_matmul_f32_workspace_bytes")
     workspace = torch.empty(need, dtype=torch.uint8, device=a.device)
-    with torch.cuda.device(a.device):
+    with _on_device_of(a):
         _check(lib().dkv_matmul_f32(c_vp(a.data_ptr()), c_i64(a.stride(0)), c_vp(b.data_ptr()), c_i64(ldb), c_i32(kn),
                                     c_vp(ptr(bias)), c_i64(m), c_i64(n), c_i64(k), c_vp(ptr(out)), c_i64(n),
                                     c_vp(ptr(workspace)), c_sz(need), c_vp(stream_handle())), "dkv_matmul_f32")
@@ -326,8 +337,9 @@ def live_groups(coef, codes=None, low=None, scale=None) -> torch.Tensor:
     f16 [n, G], coef is written first: code * scale + low."""
     n, groups = coef.shape[0], coef.shape[1] // 64
     live = torch.zeros(groups, dtype=torch.int32, device=coef.device)
-    _check(lib().dkv_live_groups(c_vp(ptr(codes)), c_vp(ptr(low)), c_vp(ptr(scale)), c_vp(ptr(coef)), c_i64(n), c_i32(groups),
-                                 c_vp(ptr(live)), c_vp(stream_handle())), "dkv_live_groups")
+    with _on_device_of(coef):
+        _check(lib().dkv_live_groups(c_vp(ptr(codes)), c_vp(ptr(low)), c_vp(ptr(scale)), c_vp(ptr(coef)), c_i64(n), c_i32(groups),
+                                     c_vp(ptr(live)), c_vp(stream_handle())), "dkv_live_groups")
     return live.bool()
 
 
@@ -347,7 +359,7 @@ def project_caches(tensors, cos, sin, mean, start: int, end: int, basis, with_en
         _check(-2, "dkv_matmul_f32_workspace_bytes")
     workspace = torch.empty(need, dtype=torch.uint8, device=first.device)
     table = _pointer_table(tensors)
-    with torch.cuda.device(first.device):
+    with _on_device_of(first):
         _check(lib().dkv_project_caches(c_vp(ptr(table)), c_i32(dtype_code(first.dtype)), c_i32(len(tensors)), c_i32(heads),
                                         c_i32(tokens), c_i32(dim), c_vp(ptr(cos)), c_vp(ptr(sin)), c_vp(ptr(mean)),
                                         c_i32(start), c_i32(end), c_vp(basis.data_ptr()),
@@ -360,16 +372,18 @@ def project_caches(tensors, cos, sin, mean, start: int, end: int, basis, with_en
 def quantize8(coef, codes, low, span, errors=None) -> None:
     """coef f32 [n, 64G] -> codes u8 [n, G, 64], low/span f16 bits [n, G], errors f32 [n, G, 9] or None."""
     n, groups = codes.shape[0], codes.shape[1]
-    _check(lib().dkv_quantize8(c_vp(ptr(coef)), c_i32(n), c_i32(groups), c_vp(ptr(codes)), c_vp(ptr(low)),
-                               c_vp(ptr(span)), c_vp(ptr(errors)), c_vp(stream_handle())), "dkv_quantize8")
+    with _on_device_of(codes):
+        _check(lib().dkv_quantize8(c_vp(ptr(coef)), c_i32(n), c_i32(groups), c_vp(ptr(codes)), c_vp(ptr(low)),
+                                   c_vp(ptr(span)), c_vp(ptr(errors)), c_vp(stream_handle())), "dkv_quantize8")
 
 
 def quantize8_rungs(coef, planes, codes, low, span, errors, energy) -> None:
     """coef f32 [n, 64G], planes u8 [R, G] -> codes, low, span as quantize8's, errors f32 [n, R], energy f32 [n]."""
     n, groups = codes.shape[0], codes.shape[1]
-    _check(lib().dkv_quantize8_rungs(c_vp(ptr(coef)), c_i32(n), c_i32(groups), c_vp(ptr(planes)), c_i32(planes.shape[0]),
-                                     c_vp(ptr(codes)), c_vp(ptr(low)), c_vp(ptr(span)), c_vp(ptr(errors)),
-                                     c_vp(ptr(energy)), c_vp(stream_handle())), "dkv_quantize8_rungs")
+    with _on_device_of(codes):
+        _check(lib().dkv_quantize8_rungs(c_vp(ptr(coef)), c_i32(n), c_i32(groups), c_vp(ptr(planes)), c_i32(planes.shape[0]),
+                                         c_vp(ptr(codes)), c_vp(ptr(low)), c_vp(ptr(span)), c_vp(ptr(errors)),
+                                         c_vp(ptr(energy)), c_vp(stream_handle())), "dkv_quantize8_rungs")
 
 
 def dequantize_codes(codes, low, span, planes, out) -> None:
