@@ -154,6 +154,26 @@ def dtype_code(dtype: torch.dtype) -> int:
     return _DTYPE[dtype]
 
 
+def _expect(what: str, device, *expected) -> None:
+    """Refuse tensors that a kernel would read or write past: each (tensor, name, dtype, shape), None in a shape for
+    any length."""
+    for t, name, dtype, shape in expected:
+        if (t.dtype != dtype or t.device != device or t.dim() != len(shape)
+                or any(want is not None and have != want for have, want in zip(t.shape, shape))):
+            raise ValueError(f"{what}: {name} must be {dtype} {list(shape)} on {device} "
+                             f"(got {t.dtype} {list(t.shape)} on {t.device})")
+
+
+def _expect_caches(what: str, *lists) -> None:
+    """Per-layer caches [1, H, T, D] of one shape, type and device, over every list of them."""
+    first = lists[0][0]
+    if first.dim() != 4 or first.shape[0] != 1 or any(len(caches) != len(lists[0]) for caches in lists):
+        raise ValueError(f"{what}: caches must be [1, heads, tokens, head_dim], one per layer (got {list(first.shape)})")
+    for caches in lists:
+        for t in caches:
+            _expect(what, first.device, (t, "every cache", first.dtype, first.shape))
+
+
 # ----------------------------------------------------------------- wrappers
 
 def pack_planes(codes, low, span, pieces, order: Order, hot, hot_off, cold=None, cold_off=None) -> None:
@@ -231,6 +251,8 @@ def centered_rows(tensors, cos, sin, mean, start: int, end: int, out) -> None:
 def ladder_errors(coef, bits) -> torch.Tensor:
     """coef f32 [n, 64G], bits u8 [R, G] -> squared quantization error of every token at every rung [n, R]."""
     rungs, groups = bits.shape
+    _expect("ladder_errors", coef.device, (coef, "coef", torch.float32, (None, 64 * groups)),
+            (bits, "bits", torch.uint8, (rungs, groups)))
     errors = torch.empty(coef.shape[0], rungs, dtype=torch.float32, device=coef.device)
     with _on_device_of(coef):
         _check(lib().dkv_ladder_errors(c_vp(ptr(coef)), c_i32(coef.shape[0]), c_i32(groups), c_vp(ptr(bits)), c_i32(rungs),
@@ -242,6 +264,8 @@ def ladder_code(coef, bits, level):
     """coef f32 [n, 64G] at each token's level (int64 [n]: a rung of bits u8 [R, G], R as it is, -1 dropped) ->
     decoded f32 [n, 64G], codes u8 [n, G, 64], low and scale f16 [n, G]."""
     (n, features), (rungs, groups) = coef.shape, bits.shape
+    _expect("ladder_code", coef.device, (coef, "coef", torch.float32, (n, 64 * groups)),
+            (bits, "bits", torch.uint8, (rungs, groups)), (level, "level", torch.int64, (n,)))
     decoded = torch.empty_like(coef)
     codes = torch.empty(n, groups, features // groups, dtype=torch.uint8, device=coef.device)
     low = torch.empty(n, groups, dtype=torch.float16, device=coef.device)
@@ -270,7 +294,10 @@ def rows_to_caches(rows, caches, first: int, gap_start: int, gap_len: int, cos=N
     """Token-matrix rows f32 [n, L*H*D] into per-layer caches [1, H, T, D] (contiguous, one dtype): row i is token
     first + i, plus gap_len from token gap_start on; keys are rotated when cos / sin [T, D] are given."""
     head = caches[0]
+    _expect_caches("rows_to_caches", caches)
     _, heads, tokens, dim = head.shape
+    _expect("rows_to_caches", head.device, (rows, "rows", torch.float32, (None, len(caches) * heads * dim)),
+            *((t, "cos and sin", torch.float32, (tokens, dim)) for t in (cos, sin) if t is not None))
     table = _pointer_table(caches)
     with _on_device_of(head):
         _check(lib().dkv_rows_to_caches(c_vp(ptr(rows)), c_i32(rows.shape[0]), c_i32(first), c_i32(gap_start), c_i32(gap_len),
@@ -281,6 +308,7 @@ def rows_to_caches(rows, caches, first: int, gap_start: int, gap_len: int, cos=N
 
 def copy_tokens(src, dst, skip: int, skip_len: int) -> None:
     """Every token outside [skip, skip + skip_len) of per-layer caches [1, H, T, D] (contiguous, one dtype) into others."""
+    _expect_caches("copy_tokens", src, dst)
     _, heads, tokens, dim = src[0].shape
     a, b = _pointer_table(src), _pointer_table(dst)
     with _on_device_of(src[0]):
@@ -292,6 +320,7 @@ def copy_tokens(src, dst, skip: int, skip_len: int) -> None:
 def outside_tokens(src, skip: int, skip_len: int) -> torch.Tensor:
     """Every token outside [skip, skip + skip_len) of per-layer caches [1, H, T, D] (contiguous, one dtype):
     [L, 1, H, T - skip_len, D]."""
+    _expect_caches("outside_tokens", src)
     _, heads, tokens, dim = src[0].shape
     out = torch.empty(len(src), 1, heads, tokens - skip_len, dim, dtype=src[0].dtype, device=src[0].device)
     table = (c_i64 * len(src))(*[ptr(t) for t in src])
@@ -336,6 +365,10 @@ def live_groups(coef, codes=None, low=None, scale=None) -> torch.Tensor:
     """bool [G]: the 64-wide groups of coef f32 [n, 64G] that some row uses.  With ladder codes u8 [n, G, 64], low and scale
     f16 [n, G], coef is written first: code * scale + low."""
     n, groups = coef.shape[0], coef.shape[1] // 64
+    _expect("live_groups", coef.device, (coef, "coef", torch.float32, (n, 64 * groups)))
+    if codes is not None:
+        _expect("live_groups", coef.device, (codes, "codes", torch.uint8, (n, groups, 64)),
+                *((t, "low and scale", torch.float16, (n, groups)) for t in (low, scale)))
     live = torch.zeros(groups, dtype=torch.int32, device=coef.device)
     with _on_device_of(coef):
         _check(lib().dkv_live_groups(c_vp(ptr(codes)), c_vp(ptr(low)), c_vp(ptr(scale)), c_vp(ptr(coef)), c_i64(n), c_i32(groups),
@@ -347,8 +380,14 @@ def project_caches(tensors, cos, sin, mean, start: int, end: int, basis, with_en
     """Centred rows of per-layer caches [1, H, T, D] times basis f32 [L*H*D, rank]: f32 [end - start, rank], and the rows'
     energies [end - start] or None (dkv_project_caches; contiguous 16-byte aligned tensors, cos and sin for keys)."""
     first = tensors[0]
+    _expect_caches("project_caches", tensors)
     _, heads, tokens, dim = first.shape
     (k, n), m = basis.shape, end - start
+    _expect("project_caches", first.device, (basis, "basis", torch.float32, (len(tensors) * heads * dim, n)),
+            (mean, "mean", torch.float32, (k,)))
+    for t in (cos, sin):
+        if t is not None:
+            _expect("project_caches", first.device, (t, "cos and sin", torch.float32, (max(end, t.shape[0]), dim)))
     kn = basis.stride(1) == 1 and basis.stride(0) >= n
     if not kn and not (basis.stride(0) == 1 and basis.stride(1) >= k):
         basis, kn = basis.contiguous(), True
@@ -380,6 +419,9 @@ def quantize8(coef, codes, low, span, errors=None) -> None:
 def quantize8_rungs(coef, planes, codes, low, span, errors, energy) -> None:
     """coef f32 [n, 64G], planes u8 [R, G] -> codes, low, span as quantize8's, errors f32 [n, R], energy f32 [n]."""
     n, groups = codes.shape[0], codes.shape[1]
+    _expect("quantize8_rungs", coef.device, (coef, "coef", torch.float32, (n, 64 * groups)),
+            (planes, "planes", torch.uint8, (None, groups)), (codes, "codes", torch.uint8, (n, groups, 64)),
+            (errors, "errors", torch.float32, (n, planes.shape[0])), (energy, "energy", torch.float32, (n,)))
     with _on_device_of(codes):
         _check(lib().dkv_quantize8_rungs(c_vp(ptr(coef)), c_i32(n), c_i32(groups), c_vp(ptr(planes)), c_i32(planes.shape[0]),
                                          c_vp(ptr(codes)), c_vp(ptr(low)), c_vp(ptr(span)), c_vp(ptr(errors)),

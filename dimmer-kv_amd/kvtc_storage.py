@@ -260,7 +260,7 @@ class _Parsed:
 def decode_bytes(codec, data: bytes, dtype=torch.float16):
     """Rebuild per-layer keys and values [1, heads, tokens, dim] from ``encode_bytes`` output
     (scripts/kvtc_storage.py:82-135)."""
-    from kvtc import _plain_gpu, inverse_transform, rope_tables, rows_to_caches, split_token_matrix
+    from kvtc import fit_caches, inverse_transform, rope_tables, rows_to_caches, split_token_matrix
 
     p = _Parsed(codec, data)
     features = codec.layers * codec.heads * codec.head_dim
@@ -273,8 +273,8 @@ def decode_bytes(codec, data: bytes, dtype=torch.float16):
         idx, stored = p.exact_rows[kind]
         if stored is not None:
             rows[idx] = stored
-        if in_kernel and _plain_gpu(rows, cos, sin):
-            like = torch.empty(1, codec.heads, p.tokens, codec.head_dim, dtype=dtype, device=rows.device)
+        like = torch.empty(1, codec.heads, p.tokens, codec.head_dim, dtype=dtype, device=rows.device)
+        if in_kernel and fit_caches(rows, like, codec.layers, (p.start, p.end), (cos, sin) if kind == "key" else ()):
             out[kind] = rows_to_caches(rows, like, codec.layers, (p.start, p.end), cos, sin, kind == "key")
             if p.middle < p.tokens:
                 dkv_hip.rows_to_caches(p.exact_tokens[kind].float(), out[kind], 0, p.start, p.middle)

@@ -72,3 +72,67 @@ def test_kernels_launch_on_their_tensors_device(name, monkeypatch):
     _wrapped_calls()[name]()
     assert launches.log == [(name, "cpu", hash("cpu") & 0xFFFF)]
     assert launches.current == "elsewhere"
+
+
+def _codec(layers=2, heads=2, dim=64, rank=64):
+    import kvtc
+    import synth
+
+    shape = synth.ModelShape(layers, heads, dim, heads, rank)
+    return kvtc.KVTCCodec(synth.kvtc_checkpoint(synth.make_context(shape, 60, seed=2)), "cpu", synth.RopeModel(shape))
+
+
+@pytest.mark.parametrize("change", ["wide rows", "narrow rows", "narrow tables", "short tables", "heads", "short span"])
+def test_rebuilt_caches_of_other_shapes_are_left_to_torch(change, monkeypatch):
+    """rows_to_caches takes its strides from the caches: rows or tables of another width would be read out of range."""
+    import kvtc
+
+    launches = Launches(monkeypatch)
+    monkeypatch.setattr(kvtc, "_plain_gpu", lambda *t: True)
+    codec, tokens, span = _codec(), 20, (4, 12)
+    features = 256 + 64 * (change == "wide rows") - 64 * (change == "narrow rows")
+    rows = torch.zeros(span[1] - span[0] - (change == "short span"), features)
+    cos = torch.ones(tokens - (change == "short tables"), 32 if change == "narrow tables" else 64)
+    caches = [torch.zeros(1, 4 if change == "heads" else 2, tokens, 64) for _ in range(2)]
+    monkeypatch.setattr(kvtc, "inverse_transform", lambda *a: rows)
+    with pytest.raises(RuntimeError):
+        codec._rebuilt_caches("key", None, caches, span, cos, cos)
+    assert launches.log == []
+
+
+def test_compress_of_other_shapes_raises_as_torch_does(monkeypatch):
+    """Caches of other heads than the calibration's: torch's broadcast error, not the binding's."""
+    import kvtc
+
+    monkeypatch.setattr(kvtc, "_plain_gpu", lambda *t: True)
+    codec = _codec()
+    monkeypatch.setattr(codec, "centered", lambda *a: pytest.fail("the kernel's route"))
+    caches = [torch.randn(1, 4, 40, 64) for _ in range(2)]
+    with pytest.raises(RuntimeError):
+        codec.compress(caches, caches, 0.3, 8, True)
+
+
+def test_bindings_refuse_shapes_they_would_read_past():
+    """On the host, before a pointer is taken (CPU tensors pass the shape checks and are refused as host memory)."""
+    f, u8, f16, i64 = torch.float32, torch.uint8, torch.float16, torch.int64
+    z = lambda *shape, dtype=f: torch.zeros(*shape, dtype=dtype)  # noqa: E731
+    caches, other = [z(1, 2, 5, 64) for _ in range(2)], [z(1, 2, 5, 64), z(1, 2, 4, 64)]
+    for call in (
+        lambda: dkv_hip.ladder_errors(z(3, 192), z(4, 2, dtype=u8)),
+        lambda: dkv_hip.ladder_errors(z(3, 128), z(4, 2)),
+        lambda: dkv_hip.ladder_code(z(3, 128), z(4, 2, dtype=u8), z(2, dtype=i64)),
+        lambda: dkv_hip.rows_to_caches(z(3, 255), caches, 1, 5, 0),
+        lambda: dkv_hip.rows_to_caches(z(3, 256), other, 1, 5, 0),
+        lambda: dkv_hip.rows_to_caches(z(3, 256), caches, 1, 5, 0, z(5, 32), z(5, 32)),
+        lambda: dkv_hip.copy_tokens(caches, other, 1, 3),
+        lambda: dkv_hip.copy_tokens(caches, caches[:1], 1, 3),
+        lambda: dkv_hip.outside_tokens(other, 1, 3),
+        lambda: dkv_hip.live_groups(z(3, 100)),
+        lambda: dkv_hip.live_groups(z(3, 128), z(2, 2, 64, dtype=u8), z(3, 2, dtype=f16), z(3, 2, dtype=f16)),
+        lambda: dkv_hip.quantize8_rungs(z(3, 128), z(4, 3, dtype=u8), z(3, 2, 64, dtype=u8), z(3, 2), z(3, 2), z(3, 4), z(3)),
+        lambda: dkv_hip.project_caches(caches, None, None, z(256), 1, 4, z(255, 8), False),
+        lambda: dkv_hip.project_caches(caches, None, None, z(255), 1, 4, z(256, 8), False),
+        lambda: dkv_hip.project_caches(caches, z(5, 32), z(5, 32), z(256), 1, 4, z(256, 8), False),
+    ):
+        with pytest.raises(ValueError, match="must be"):
+            call()
