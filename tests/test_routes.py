@@ -136,3 +136,15 @@ def test_bindings_refuse_shapes_they_would_read_past():
     ):
         with pytest.raises(ValueError, match="must be"):
             call()
+
+
+def test_ladder_kernels_need_a_size_for_every_rung(monkeypatch):
+    """The exact level follows the last sized rung; the kernels take it to follow the last row of widths."""
+    import kvtc
+
+    monkeypatch.setattr(kvtc, "_plain_gpu", lambda *t: True)
+    codec = _codec()
+    coef = torch.zeros(3, 64)
+    assert codec._ladder_on_gpu(coef, "key")
+    codec.streams["key"].rung_bytes = codec.streams["key"].rung_bytes[:-1]
+    assert not codec._ladder_on_gpu(coef, "key")
