@@ -148,3 +148,28 @@ def test_ladder_kernels_need_a_size_for_every_rung(monkeypatch):
     assert codec._ladder_on_gpu(coef, "key")
     codec.streams["key"].rung_bytes = codec.streams["key"].rung_bytes[:-1]
     assert not codec._ladder_on_gpu(coef, "key")
+
+
+def test_recorded_calls_are_left_to_torch():
+    """A trace of a call must hold its operations: a kernel's output would be a constant in it."""
+    import kvtc
+    from torch.fx.experimental.proxy_tensor import make_fx
+    from torch.utils.flop_counter import FlopCounterMode
+
+    seen = []
+
+    def watched(x):
+        seen.append(kvtc._watched())
+        return x + 1
+
+    x = torch.ones(2)
+    watched(x)
+    torch.jit.trace(watched, x, check_trace=False)
+    make_fx(watched)(x)
+    with FlopCounterMode(display=False):
+        watched(x)
+    torch.func.vmap(watched)(x)
+    torch.func.jvp(watched, (x,), (x,))
+    torch.compile(watched, backend="eager")(x)
+    watched(x)
+    assert seen[0] is False and seen[-1] is False and len(seen) >= 8 and all(seen[1:-1])
