@@ -296,6 +296,9 @@ DKV_DEVICE long operand_line(long row, int t, int n_slots) {
 }
 
 constexpr float kLn2 = 0.693147180559945309f;
+// A scale of 0 (every token weighs the same) as many-row decodes take it: the -inf of slots past the tokens times 0 would
+// be NaN; times this it stays -inf, and every finite score still comes to about 0.
+constexpr float kLeastScale = 1.17549435e-38f;
 
 // Question scoring's and many-row decodes' per-quarter statistics, [R/8][nsub][8]: eight consecutive rows sit together for
 // each 64-token quarter t, so a wave's 32 rows store four 32-byte pieces and the row-statistics
@@ -1036,6 +1039,7 @@ __global__ __launch_bounds__(kK2Threads) void keys_scores_kernel(K2Args a) {
           }
           float c2 = a.scaling * 1.44269504088896341f;
           if constexpr (!ROWMAJOR) {
+            if (c2 == 0.0f) c2 = kLeastScale;
             if (c2 < 0.0f) {  // (uniform) the maximum below is over the raw products
               c2 = -c2;
 #pragma unroll
@@ -1268,7 +1272,7 @@ DKV_DEVICE void many_rows_epilogue(const K2Args& a, floatx16 (&acc)[DB], float4 
     }
   };
   const float c2s = a.scaling * 1.44269504088896341f;
-  const float c2 = fabsf(c2s);
+  const float c2 = c2s == 0.0f ? kLeastScale : fabsf(c2s);
   load_queries(0);
   __syncthreads();  // the main loop's basis blocks are read
   store_queries(0);

@@ -112,3 +112,25 @@ def test_value_lines_follow_decodes_and_few_row_layers():
     fresh, _, again = gpu_context(case, refine_capacity=200)
     again["value"].refine(torch.arange(0, 1400, 7, device=DEV)[:200])
     assert np.array_equal(changed, gpu_attend(case, fresh, 1))
+
+
+@pytest.mark.parametrize("name,tokens", [("1b", 300), ("3b", 13000)])  # 128-row and 256-row workgroups, a ragged last tile
+def test_many_rows_with_zero_scale(name, tokens):
+    """A scale of 0: every token weighs the same, as zero queries make it (the same kernels, finite scores of 0)."""
+    print(f"[case] many rows, scale 0, {name} T={tokens}", flush=True)
+    case = build_case(SHAPES[name], tokens, seed=8, query_scale=50.0, q_len=5)
+    ctx, _, _ = gpu_context(case)
+    case.mask = None
+    ke, ve = (getattr(case, f)[0].to(DEV).contiguous() for f in ("key_exact", "value_exact"))
+
+    def run(query, scaling):
+        out = torch.empty(1, 5, case.shape.q_heads, case.shape.head_dim, device=DEV)
+        ctx.run_layer(ctx.layer_args(0, query, out, ke, ve, None, None, scaling))
+        torch.cuda.synchronize()
+        return out
+
+    query = case.queries[0].to(DEV).contiguous()
+    got, want = run(query, 0.0), run(torch.zeros_like(query), case.shape.head_dim ** -0.5)
+    assert torch.isfinite(got).all()
+    # the weights are equal in both; their common power of two may differ
+    assert torch.allclose(got, want, rtol=1e-5, atol=1e-6 * float(want.abs().max()))
