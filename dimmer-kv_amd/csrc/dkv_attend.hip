@@ -2336,6 +2336,13 @@ __global__ __launch_bounds__(512, 2) void value_rows_kernel(K3RowsArgs a) {
 #pragma unroll
       for (int v = 0; v < 16; ++v) acc[i][j][v] = 0.0f;
 
+  auto meet = [&]() {
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_waitcnt(0x0070);  // vmcnt(0) lgkmcnt(0)
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+  };
+
   // first round: two stages (a split has at least four), and the rows' maxima over the split by 512 / MT threads each
   copy(0, S0);
   copy(1, S1);
@@ -2354,7 +2361,7 @@ __global__ __launch_bounds__(512, 2) void value_rows_kernel(K3RowsArgs a) {
     for (int e = part; e < stages; e += PARTS) m = fmaxf(m, src[8 * e]);
     rmax[part][r] = m;
   }
-  __syncthreads();  // drains the copies too
+  meet();  // every wave's copies have landed, the maxima are in
   float M[2];
 #pragma unroll
   for (int i = 0; i < 2; ++i) {
@@ -2389,12 +2396,6 @@ __global__ __launch_bounds__(512, 2) void value_rows_kernel(K3RowsArgs a) {
     for (int i = 0; i < 2; ++i)
 #pragma unroll
       for (int j = 0; j < JB; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(pa[i], f.b[j], acc[i][j], 0, 0, 0);
-  };
-  auto meet = [&]() {
-    asm volatile("" ::: "memory");
-    __builtin_amdgcn_s_waitcnt(0x0070);  // vmcnt(0) lgkmcnt(0)
-    __builtin_amdgcn_s_barrier();
-    asm volatile("" ::: "memory");
   };
   // one step per scheduling region: the next step's reads (and the copies) between the products
   auto spread = [&](auto reads_t, auto copies_t) {
