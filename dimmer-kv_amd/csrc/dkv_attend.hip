@@ -2810,6 +2810,42 @@ inline int k2_rows_waves(const dkv_attend_args_t* a, int ntiles) {
 // 48 to 3,200 rows and 1,100 to 16,400 tokens: the layer of the choice takes at most 3 % longer than the best one's.
 constexpr double kRowsTile4 = 6.0, kRowsTile2 = 3.2, kRowsTile1 = 2.4, kRowsFixed = 8.0, kRowsPartialMB = 0.1;
 
+// fn(st, splits) for every split length of st >= 2 whole tiles at which the batch's number of splits changes, shortest
+// first.  Every layer of a step asks, so it is counted from how many sequences reach each tile (a few adds per length:
+// 3 us for 64 sequences of 16K tokens, where a division per sequence and length up to the batch's tiles took 2 ms).
+template <class Fn>
+void each_split_count(const dkv_attend_args_t* a, Fn&& fn) {
+  constexpr int kMost = 4096;  // tiles of a sequence (a million tokens) up to which they are counted
+  auto tiles_of = [&](int b) { return (a->cu_seqlens_host[b + 1] - a->cu_seqlens_host[b] + kTileTok - 1) / kTileTok; };
+  int longest = 0;
+  for (int b = 0; b < a->batch; ++b) longest = std::max(longest, tiles_of(b));
+  int reach[kMost + 1];  // sequences of more than x tiles
+  const bool counted = a->batch > 1 && longest <= kMost;
+  if (counted) {
+    std::fill(reach, reach + longest + 1, 0);
+    for (int b = 0; b < a->batch; ++b) ++reach[tiles_of(b)];
+    for (int x = longest, more = 0; x >= 0; --x) {
+      const int exactly = reach[x];
+      reach[x] = more;
+      more += exactly;
+    }
+  }
+  long last = -1;
+  for (int st = 2; st <= std::max(2, longest); ++st) {
+    long splits = 0;
+    if (counted) {
+      for (int x = 0; x < longest; x += st) splits += reach[x];
+    } else {
+      for (int b = 0; b < a->batch; ++b) splits += (tiles_of(b) + st - 1) / st;
+    }
+    if (splits != last) fn(st, splits);
+    last = splits;
+    // one sequence: straight to the next length with fewer splits
+    if (a->batch == 1 && splits > 1) st = std::max(st, (int)((longest + splits - 2) / (splits - 1)) - 1);
+    if (a->batch == 1 && splits <= 1) break;
+  }
+}
+
 // Workspace: [decoded key coefficients][decoded value codes][value affine][one word, and with many rows the value
 // lines][probabilities][tile statistics]
 // [split partials][chunk partials][exact-tail results].
@@ -2841,13 +2877,13 @@ Layout make_layout(const dkv_attend_args_t* a, bool values = true) {
   int prob_rows = L.R_total, stat_rows = L.R_total;
   if (values && L.R_total / a->kv_heads > kSmallRows) {
     // many rows: the workgroup height and the splits (whole tiles, at least two) that take the least time by the
-    // measured stage costs: the rounds of one workgroup per CU, each its stages and a prologue
+    // measured stage costs: the rounds of one workgroup per CU, each its stages and a prologue.  Of the split lengths
+    // that give as many splits only the shortest can be the best.
     double least = 1e300;
     for (int mw = 1; mw <= 4; mw *= 2) {
       const long per_split = (long)((L.R_total + 64 * mw - 1) / (64 * mw)) * (a->rank / kRowsCols);
       const double tile_us = mw == 4 ? kRowsTile4 : mw == 2 ? kRowsTile2 : kRowsTile1;
-      for (int st = 2; st <= std::max(2, L.ntiles); ++st) {
-        const int splits = count_splits(st * kTileTok);
+      each_split_count(a, [&](int st, long splits) {
         const long rounds = (per_split * splits + kCUs - 1) / kCUs;
         const double cost = rounds * (st * tile_us + kRowsFixed) + kRowsPartialMB * 4e-6 * splits * L.R_total * a->rank;
         if (cost < least * 0.999) {
@@ -2855,7 +2891,7 @@ Layout make_layout(const dkv_attend_args_t* a, bool values = true) {
           L.rows_mw = mw;
           L.split_tok = st * kTileTok;
         }
-      }
+      });
     }
     const int mt = (L.R_total + 64 * L.rows_mw - 1) / (64 * L.rows_mw);
     L.nsplits = count_splits(L.split_tok);
