@@ -39,7 +39,14 @@ constexpr int kTile = 256;         // rows of A, and of B, per workgroup
 constexpr int kLine = 128;         // bytes of one (row, 32-component block)
 constexpr int kBlock = 32 * kLine; // bytes of one (32 rows, 32 components)
 constexpr int kStage = 2 * 8 * kBlock;  // bytes of one stage: 256 rows of A and of B, 32 components
-constexpr int kFlagged = INT_MIN;  // exponent of a row that holds an infinity or a NaN
+constexpr int kFlagged = INT_MIN;  // in place of the exponent of a row that holds an infinity or a NaN: its pieces are zeros
+
+// Such rows of an operand, in any order: special_kernel's work.
+struct Flagged {
+  int* count;
+  int* list;
+  DKV_DEVICE void add(int row) const { list[atomicAdd(count, 1)] = row; }
+};
 
 inline long pad_to(long x, long m) { return (x + m - 1) / m * m; }
 
@@ -55,10 +62,13 @@ DKV_DEVICE int row_shift(uint32_t top) {
 
 // Eight scaled floats -> their hi and lo pieces.
 DKV_DEVICE void split8(const float (&x)[8], int shift, half8& hi, half8& lo) {
-  const int s = shift == kFlagged ? 0 : shift;
+  if (shift == kFlagged) {
+    hi = lo = half8{0, 0, 0, 0, 0, 0, 0, 0};
+    return;
+  }
 #pragma unroll
   for (int i = 0; i < 8; ++i) {
-    const float v = __builtin_ldexpf(x[i], s);
+    const float v = __builtin_ldexpf(x[i], shift);
     const half_t h = (half_t)v;
     hi[i] = h;
     lo[i] = (half_t)(v - (float)h);
@@ -84,7 +94,7 @@ __global__ __launch_bounds__(256) void clear_kernel(uint32_t* __restrict__ p, in
 template <int NT, int OCT, bool VEC>
 __global__ __launch_bounds__(NT) void split_rows_kernel(const float* __restrict__ src, long ld, int rows, int K, int KB,
                                                         uint8_t* __restrict__ out, int* __restrict__ shifts,
-                                                        uint32_t* __restrict__ flag) {
+                                                        Flagged flagged) {
   __shared__ uint32_t wtop[NT / 64];
   const int tid = threadIdx.x;
   const long row = blockIdx.x;
@@ -123,8 +133,8 @@ __global__ __launch_bounds__(NT) void split_rows_kernel(const float* __restrict_
   for (int w = 0; w < NT / 64; ++w) top = max(top, wtop[w]);
   const int shift = row_shift(top);
   if (tid == 0) {
-    shifts[row] = shift;
-    if (shift == kFlagged && flag) atomicOr(flag, 1u);
+    shifts[row] = shift == kFlagged ? 0 : shift;
+    if (shift == kFlagged) flagged.add((int)row);
   }
   half8 hi, lo;
 #pragma unroll
@@ -161,7 +171,7 @@ __global__ __launch_bounds__(256) void column_top_kernel(const float* __restrict
 // The columns of a row-major [K][N] source as split rows: a workgroup turns 64 columns x 32 components.
 __global__ __launch_bounds__(256) void split_columns_kernel(const float* __restrict__ src, long ld, int K, int N, int KB,
                                                             const uint32_t* __restrict__ top, uint8_t* __restrict__ out,
-                                                            int* __restrict__ shifts, uint32_t* __restrict__ flag) {
+                                                            int* __restrict__ shifts, Flagged flagged) {
   __shared__ float t[32][65];
   const int tid = threadIdx.x;
   const int nb = gridDim.x / KB;  // column blocks, fastest in the grid
@@ -183,8 +193,8 @@ __global__ __launch_bounds__(256) void split_columns_kernel(const float* __restr
   split8(x, shift, hi, lo);
   store_octet(out, n, 4 * kb + o, KB, hi, lo);
   if (kb == 0 && o == 0) {
-    shifts[n] = shift;
-    if (shift == kFlagged) atomicOr(flag, 1u);
+    shifts[n] = shift == kFlagged ? 0 : shift;
+    if (shift == kFlagged) flagged.add((int)n);
   }
 }
 
@@ -384,7 +394,7 @@ __global__ __launch_bounds__(256) void sum_splits_kernel(const float* __restrict
   c[(e / N) * ldc + n] = s + (bias ? bias[n] : 0.0f);
 }
 
-// A's rows as special_rows_kernel reads them: as they lie, or a token's centred row from the caches.
+// A's rows as special_kernel reads them: as they lie, or a token's centred row from the caches.
 struct PlainRows {
   const float* a;
   long lda;
@@ -445,7 +455,8 @@ struct CacheRows {
 // CU), 8,155 of 8,192 columns 116 against 84 and 95.
 template <int T, bool ROTATE, int NT, int U>
 __global__ __launch_bounds__(NT, NT == 512 ? 4 : 1) void split_caches_kernel(CacheArgs c, int rows, int KB, uint8_t* __restrict__ out,
-                                                          int* __restrict__ shifts, float* __restrict__ energy) {
+                                                          int* __restrict__ shifts, Flagged flagged,
+                                                          float* __restrict__ energy) {
   __shared__ uint32_t wtop[NT / 64];
   __shared__ float wsum[NT / 64];
   const int tid = threadIdx.x;
@@ -515,7 +526,8 @@ __global__ __launch_bounds__(NT, NT == 512 ? 4 : 1) void split_caches_kernel(Cac
   for (int w = 0; w < NT / 64; ++w) top = max(top, wtop[w]);
   const int shift = row_shift(top);
   if (tid == 0) {
-    shifts[row] = shift;
+    shifts[row] = shift == kFlagged ? 0 : shift;
+    if (shift == kFlagged) flagged.add((int)row);
     if (energy && live) {
       float s = 0.0f;
 #pragma unroll
@@ -539,36 +551,66 @@ __global__ __launch_bounds__(NT, NT == 512 ? 4 : 1) void split_caches_kernel(Cac
   for (int o = c.K / 8 + tid; o < KB * 4; o += NT) store_octet(out, row, o, KB, zero, zero);
 }
 
-// Rows of A or B that hold an infinity or a NaN have no split form: their products in plain fp32.
+// Outputs of flagged rows.  One element that is not finite makes every output of its row infinite or NaN, whatever the
+// finite terms are, so those are left out (zeros in the product above): a workgroup takes a flagged row of A (or of B),
+// lists its elements that are not finite, 2,048 components at a time, and adds their products with every row of B (of A).
+// A term of two such elements may be added from both sides, which changes nothing.  With nothing flagged every workgroup
+// ends at once.  16,348 x 2,048 x 28,672, 4,945 us with nothing flagged: 4,961 with a flagged row, 5,060 with a flagged
+// column, 4,376 with a NaN in every row (zeros are faster to multiply); from the caches, 5,054 us: 6,388 with an infinite
+// channel of every token.
+constexpr int kSpecialList = 2048;
+constexpr int kSpecialGrid = 1024;  // workgroups at most
+
 template <class Rows>
-__global__ __launch_bounds__(256) void special_rows_kernel(Rows a, const float* __restrict__ b,
-                                                           long ldb, int b_kn, const float* __restrict__ bias, int M,
-                                                           int N, int K, const int* __restrict__ sa,
-                                                           const int* __restrict__ sb, const uint32_t* __restrict__ flag,
-                                                           float* __restrict__ c, long ldc) {
-  __shared__ unsigned long long marked;
-  const int m0 = blockIdx.x * 64, lane = threadIdx.x;
-  const bool columns = *flag != 0;
-  if (lane < 64) {
-    const unsigned long long w = __ballot(m0 + lane < M && (columns || sa[min(m0 + lane, M - 1)] == kFlagged));
-    if (lane == 0) marked = w;
-  }
-  __syncthreads();
-  for (unsigned long long w = marked; w != 0; w &= w - 1) {
-    const long m = m0 + __builtin_ctzll(w);
-    const bool row = sa[m] == kFlagged;
-    for (int n = threadIdx.x; n < N; n += 256) {
-      if (!row && sb[n] != kFlagged) continue;
-      float s = 0.0f;
-      for (int k = 0; k < K; ++k) s += a.at(m, k) * (b_kn ? b[k * ldb + n] : b[n * ldb + k]);
-      c[m * ldc + n] = s + (bias ? bias[n] : 0.0f);
+__global__ __launch_bounds__(256) void special_kernel(Rows a, const float* __restrict__ b, long ldb, int b_kn, int M, int N,
+                                                      int K, const int* __restrict__ counts, const int* __restrict__ listed_a,
+                                                      const int* __restrict__ listed_b, float* __restrict__ c, long ldc) {
+  __shared__ int at[kSpecialList];
+  __shared__ float value[kSpecialList];
+  __shared__ int found;
+  const int tid = threadIdx.x, na = counts[0], nb = counts[1];
+  auto b_at = [&](int n, int k) { return b_kn ? b[(long)k * ldb + n] : b[(long)n * ldb + k]; };
+  for (int it = blockIdx.x; it < na + nb; it += gridDim.x) {
+    const bool of_a = it < na;
+    const int row = of_a ? listed_a[it] : listed_b[it - na], others = of_a ? N : M;
+    bool open = true;  // some output of this row is not NaN yet, as far as this workgroup knows
+    for (int k0 = 0; k0 < K && open; k0 += kSpecialList) {
+      float x[kSpecialList / 256];
+#pragma unroll
+      for (int i = 0; i < kSpecialList / 256; ++i) {
+        const int k = min(k0 + tid + 256 * i, K - 1);
+        x[i] = of_a ? a.at(row, k) : b_at(row, k);
+      }
+      __syncthreads();  // the segment before is added
+      if (tid == 0) found = 0;
+      __syncthreads();
+#pragma unroll
+      for (int i = 0; i < kSpecialList / 256; ++i) {
+        const int k = k0 + tid + 256 * i;
+        if (k < K && abs_bits(x[i]) >= 0x7f800000u) {
+          const int j = atomicAdd(&found, 1);
+          at[j] = k;
+          value[j] = x[i];
+        }
+      }
+      __syncthreads();
+      const int count = found;
+      if (count == 0) continue;
+      bool mine = false;
+      for (int o = tid; o < others; o += 256) {
+        float s = 0.0f;
+        for (int j = 0; j < count && s == s; ++j) s += value[j] * (of_a ? b_at(o, at[j]) : a.at(o, at[j]));
+        atomicAdd(&c[of_a ? row * ldc + o : o * ldc + row], s);
+        mine |= s == s;
+      }
+      open = __syncthreads_or(mine);
     }
   }
 }
 
 struct GemmLayout {
   int KB, mt, nt, splits, per_split;
-  size_t a, b, sa, sb, top, part, total;  // top: the column maxima and, after them, the flag word
+  size_t a, b, sa, sb, top, listed, part, total;  // top: the column maxima and, after them, the flagged rows' counts
 };
 
 constexpr int kGemmCUs = 256;
@@ -594,24 +636,25 @@ GemmLayout gemm_layout(long M, long N, long K) {
   L.b = take((size_t)L.nt * kTile * L.KB * kLine);
   L.sa = take((size_t)L.mt * kTile * 4);
   L.sb = take((size_t)L.nt * kTile * 4);
-  L.top = take((size_t)(N + 1) * 4);
+  L.top = take((size_t)(N + 2) * 4);
+  L.listed = take((size_t)(M + N) * 4);  // the flagged rows of A, then of B
   L.part = take(L.splits > 1 ? (size_t)L.splits * M * N * 4 : 0);
   L.total = off;
   return L;
 }
 
 void launch_split_rows(const float* src, long ld, long rows, long rows_pad, int K, int KB, uint8_t* out, int* shifts,
-                       uint32_t* flag, hipStream_t st) {
+                       Flagged flagged, hipStream_t st) {
   const bool vec = ld % 4 == 0 && (uintptr_t)src % 16 == 0;
   const dim3 grid((unsigned)rows_pad);
 #define DKV_SPLIT(NT_, OCT_)                                                                                        \
   do {                                                                                                              \
     if (vec)                                                                                                        \
       hipLaunchKernelGGL((split_rows_kernel<NT_, OCT_, true>), grid, dim3(NT_), 0, st, src, ld, (int)rows, K, KB,   \
-                         out, shifts, flag);                                                                        \
+                         out, shifts, flagged);                                                                     \
     else                                                                                                            \
       hipLaunchKernelGGL((split_rows_kernel<NT_, OCT_, false>), grid, dim3(NT_), 0, st, src, ld, (int)rows, K, KB,  \
-                         out, shifts, flag);                                                                        \
+                         out, shifts, flagged);                                                                     \
   } while (0)
   if (KB * 4 <= 256)
     DKV_SPLIT(256, 1);
@@ -652,16 +695,17 @@ int launch_product(const char* what, Rows rows, SplitA&& split_a, const float* b
   hipStream_t st = dkv::as_stream(stream);
   int *sa = (int*)(ws + L.sa), *sb = (int*)(ws + L.sb);
   uint32_t* top = (uint32_t*)(ws + L.top);
-  uint32_t* flag = top + N;
-  hipLaunchKernelGGL(clear_kernel, dim3((unsigned)((N + 1 + 255) / 256)), dim3(256), 0, st, top, (int)N + 1);
-  split_a(L, ws + L.a, sa, st);
+  int *counts = (int*)(top + N), *listed = (int*)(ws + L.listed);
+  hipLaunchKernelGGL(clear_kernel, dim3((unsigned)((N + 2 + 255) / 256)), dim3(256), 0, st, top, (int)N + 2);
+  split_a(L, ws + L.a, sa, Flagged{counts, listed}, st);
+  const Flagged flagged{counts + 1, listed + M};
   if (b_is_kn) {
     hipLaunchKernelGGL(column_top_kernel, dim3((unsigned)((N + 63) / 64 * ((K + 127) / 128))), dim3(256), 0, st, b,
                        ldb, (int)K, (int)N, top);
     hipLaunchKernelGGL(split_columns_kernel, dim3((unsigned)((long)L.nt * (kTile / 64) * L.KB)), dim3(256), 0, st, b, ldb,
-                       (int)K, (int)N, L.KB, top, ws + L.b, sb, flag);
+                       (int)K, (int)N, L.KB, top, ws + L.b, sb, flagged);
   } else {
-    launch_split_rows(b, ldb, N, (long)L.nt * kTile, (int)K, L.KB, ws + L.b, sb, flag, st);
+    launch_split_rows(b, ldb, N, (long)L.nt * kTile, (int)K, L.KB, ws + L.b, sb, flagged, st);
   }
   rc = dkv::check_launch(what);
   if (rc) return rc;
@@ -688,20 +732,22 @@ int launch_product(const char* what, Rows rows, SplitA&& split_a, const float* b
   if (L.splits > 1)
     hipLaunchKernelGGL(sum_splits_kernel, dim3((unsigned)((M * N + 255) / 256)), dim3(256), 0, st,
                        (const float*)(ws + L.part), L.splits, (int)M, (int)N, bias, c, ldc);
-  hipLaunchKernelGGL(special_rows_kernel<Rows>, dim3((unsigned)((M + 63) / 64)), dim3(256), 0, st, rows, b, ldb, b_is_kn, bias,
-                     (int)M, (int)N, (int)K, sa, sb, flag, c, ldc);
+  hipLaunchKernelGGL(special_kernel<Rows>, dim3((unsigned)std::min(M + N, (long)kSpecialGrid)), dim3(256), 0, st, rows, b,
+                     ldb, b_is_kn, (int)M, (int)N, (int)K, counts, listed, listed + M, c, ldc);
   return dkv::check_launch(what);
 }
 
 template <int T, bool ROTATE>
 int launch_project(const CacheArgs& c, const float* b, long ldb, int b_is_kn, long M, long N, float* out, long ldo, float* energy,
                    void* workspace, size_t workspace_bytes, void* stream) {
-  auto split = [&](const GemmLayout& L, uint8_t* lines, int* sa, hipStream_t st) {
+  auto split = [&](const GemmLayout& L, uint8_t* lines, int* sa, Flagged flagged, hipStream_t st) {
     const dim3 grid((unsigned)(L.mt * kTile));
     if (c.K <= 8192)
-      hipLaunchKernelGGL((split_caches_kernel<T, ROTATE, 256, 2>), grid, dim3(256), 0, st, c, (int)M, L.KB, lines, sa, energy);
+      hipLaunchKernelGGL((split_caches_kernel<T, ROTATE, 256, 2>), grid, dim3(256), 0, st, c, (int)M, L.KB, lines, sa, flagged,
+                         energy);
     else
-      hipLaunchKernelGGL((split_caches_kernel<T, ROTATE, 512, 4>), grid, dim3(512), 0, st, c, (int)M, L.KB, lines, sa, energy);
+      hipLaunchKernelGGL((split_caches_kernel<T, ROTATE, 512, 4>), grid, dim3(512), 0, st, c, (int)M, L.KB, lines, sa, flagged,
+                         energy);
   };
   return launch_product("dkv_project_caches", CacheRows<T, ROTATE>{c}, split, b, ldb, b_is_kn, nullptr, M, N, c.K, out, ldo,
                         workspace, workspace_bytes, stream);
@@ -743,8 +789,8 @@ extern "C" int dkv_matmul_f32(const float* a, int64_t lda, const float* b, int64
                               void* workspace, size_t workspace_bytes, void* stream) {
   DKV_REQUIRE(a && b && c, DKV_EINVAL, "dkv_matmul_f32: null pointer");
   DKV_REQUIRE(lda >= K, DKV_ESHAPE, "dkv_matmul_f32: bad row strides");
-  auto split = [&](const GemmLayout& L, uint8_t* lines, int* sa, hipStream_t st) {
-    launch_split_rows(a, lda, M, (long)L.mt * kTile, (int)K, L.KB, lines, sa, nullptr, st);
+  auto split = [&](const GemmLayout& L, uint8_t* lines, int* sa, Flagged flagged, hipStream_t st) {
+    launch_split_rows(a, lda, M, (long)L.mt * kTile, (int)K, L.KB, lines, sa, flagged, st);
   };
   return launch_product("dkv_matmul_f32", PlainRows{a, lda}, split, b, ldb, b_is_kn, bias, M, N, K, c, ldc, workspace,
                         workspace_bytes, stream);

@@ -252,7 +252,8 @@ int dkv_project_caches(const uint64_t* layer_ptrs, int32_t dtype, int32_t layers
  * b_is_kn [K][ldb]; C is [M][ldc].  Operands are split into two fp16 pieces per
  * element in the workspace (4 bytes per element of each padded operand, and
  * partial sums where a product has few tiles); errors against float64 are below a float32
- * product's.  Rows with infinities or NaN are multiplied in plain float32. */
+ * product's.  Outputs of rows with infinities or NaN are where float32 puts
+ * them. */
 size_t dkv_matmul_f32_workspace_bytes(int64_t M, int64_t N, int64_t K);
 int dkv_matmul_f32(const float* a, int64_t lda, const float* b, int64_t ldb, int32_t b_is_kn, const float* bias,
                    int64_t M, int64_t N, int64_t K, float* c, int64_t ldc, void* workspace, size_t workspace_bytes,

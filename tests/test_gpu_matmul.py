@@ -111,3 +111,60 @@ def test_projection_from_caches_matches_rows(layers, heads, dim, rank, dtype, st
         got, energy = dkv_hip.project_caches(caches, cos, sin, mean, start, end, b, True)
         assert torch.equal(torch.nan_to_num(got), torch.nan_to_num(dkv_hip.matmul_f32(rows, b)))
     assert torch.allclose(energy.double(), rows.double().square().sum(1), rtol=width * 2.0 ** -24, atol=0.0)
+
+
+def _same_specials(got, want):
+    for same in (torch.isnan, torch.isposinf, torch.isneginf):
+        assert torch.equal(same(got), same(want))
+    fine = torch.isfinite(want)
+    assert torch.allclose(got[fine], want[fine], rtol=1e-4, atol=1e-4)
+
+
+@pytest.mark.parametrize("kn", [True, False])
+@pytest.mark.parametrize("rows,columns", [("all", 0), (0, "all"), (65, 129), (1, 0), (0, 1)])
+def test_matmul_flagged_rows_and_columns(rows, columns, kn):
+    """Rows of A and columns of B with infinities or NaN, from one (a tile of one row) to all of them, with a bias:
+    where torch puts them, the other outputs untouched."""
+    import dkv_hip
+
+    m, n, k = 200, 300, 1100
+    print(f"[case] matmul flagged rows {rows}, columns {columns} kn={kn}", flush=True)
+    a, b, bias = _pair(m, n, k, kn, 11)
+    specials = torch.tensor([float("inf"), float("-inf"), float("nan")], device=DEV)
+    for i in range(m if rows == "all" else rows):
+        a[i if rows == "all" else 3 * i, (7 * i) % k] = specials[i % 3]
+    for i in range(n if columns == "all" else columns):
+        b[(5 * i) % k, i if columns == "all" else 2 * i] = specials[(i + 1) % 3]
+    _same_specials(dkv_hip.matmul_f32(a, b, bias), torch.matmul(a, b) + bias)
+
+
+def test_projection_from_caches_with_every_row_flagged():
+    """A NaN in the mean reaches every row: all outputs NaN, and no slower than a few of the product (by one workgroup per 64
+    rows, a thread per output and all of K in turn, it was hundreds of them)."""
+    import dkv_hip
+
+    layers, heads, dim, rank, end = 16, 8, 64, 1024, 2052
+    print("[case] projection from caches, every row flagged", flush=True)
+    g = torch.Generator(DEV).manual_seed(3)
+    caches = [torch.randn(1, heads, end + 3, dim, generator=g, device=DEV).half() for _ in range(layers)]
+    mean = torch.zeros(layers * heads * dim, device=DEV)
+    cos, sin = (torch.randn(end + 3, dim, generator=g, device=DEV) for _ in range(2))
+    basis = torch.randn(layers * heads * dim, rank, generator=g, device=DEV)
+
+    def timed():
+        best = 1e9
+        for _ in range(3):
+            t0, t1 = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+            t0.record()
+            out, _ = dkv_hip.project_caches(caches, cos, sin, mean, 4, end, basis, False)
+            t1.record()
+            t1.synchronize()
+            best = min(best, t0.elapsed_time(t1))
+        return out, best
+
+    out, plain = timed()
+    assert torch.isfinite(out).all()
+    mean[77] = float("nan")
+    out, flagged = timed()
+    print(f"  {1e3 * plain:.0f} us, every row flagged {1e3 * flagged:.0f} us", flush=True)
+    assert torch.isnan(out).all() and flagged < 4 * plain
