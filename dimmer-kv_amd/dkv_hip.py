@@ -155,23 +155,15 @@ def dtype_code(dtype: torch.dtype) -> int:
 
 
 def _expect(what: str, device, *expected) -> None:
-    """Refuse tensors that a kernel would read or write past: each (tensor, name, dtype, shape), None in a shape for
-    any length."""
+    """Refuse tensors that a kernel would read or write past: each (tensor, name, dtype, shape), a first length of None
+    for any.  Lists of caches are their callers' to compare (kvtc._plain_caches, or made alike)."""
     for t, name, dtype, shape in expected:
-        if (t.dtype != dtype or t.device != device or t.dim() != len(shape)
-                or any(want is not None and have != want for have, want in zip(t.shape, shape))):
+        have, want = t.shape, shape
+        if want[0] is None and len(have) == len(want):
+            have, want = have[1:], want[1:]
+        if have != want or t.dtype != dtype or t.device != device:
             raise ValueError(f"{what}: {name} must be {dtype} {list(shape)} on {device} "
                              f"(got {t.dtype} {list(t.shape)} on {t.device})")
-
-
-def _expect_caches(what: str, *lists) -> None:
-    """Per-layer caches [1, H, T, D] of one shape, type and device, over every list of them."""
-    first = lists[0][0]
-    if first.dim() != 4 or first.shape[0] != 1 or any(len(caches) != len(lists[0]) for caches in lists):
-        raise ValueError(f"{what}: caches must be [1, heads, tokens, head_dim], one per layer (got {list(first.shape)})")
-    for caches in lists:
-        for t in caches:
-            _expect(what, first.device, (t, "every cache", first.dtype, first.shape))
 
 
 # ----------------------------------------------------------------- wrappers
@@ -294,7 +286,6 @@ def rows_to_caches(rows, caches, first: int, gap_start: int, gap_len: int, cos=N
     """Token-matrix rows f32 [n, L*H*D] into per-layer caches [1, H, T, D] (contiguous, one dtype): row i is token
     first + i, plus gap_len from token gap_start on; keys are rotated when cos / sin [T, D] are given."""
     head = caches[0]
-    _expect_caches("rows_to_caches", caches)
     _, heads, tokens, dim = head.shape
     _expect("rows_to_caches", head.device, (rows, "rows", torch.float32, (None, len(caches) * heads * dim)),
             *((t, "cos and sin", torch.float32, (tokens, dim)) for t in (cos, sin) if t is not None))
@@ -308,7 +299,9 @@ def rows_to_caches(rows, caches, first: int, gap_start: int, gap_len: int, cos=N
 
 def copy_tokens(src, dst, skip: int, skip_len: int) -> None:
     """Every token outside [skip, skip + skip_len) of per-layer caches [1, H, T, D] (contiguous, one dtype) into others."""
-    _expect_caches("copy_tokens", src, dst)
+    if len(dst) != len(src):
+        raise ValueError(f"copy_tokens: dst must be {len(src)} caches (got {len(dst)})")
+    _expect("copy_tokens", src[0].device, (dst[0], "dst", src[0].dtype, src[0].shape))
     _, heads, tokens, dim = src[0].shape
     a, b = _pointer_table(src), _pointer_table(dst)
     with _on_device_of(src[0]):
@@ -320,7 +313,6 @@ def copy_tokens(src, dst, skip: int, skip_len: int) -> None:
 def outside_tokens(src, skip: int, skip_len: int) -> torch.Tensor:
     """Every token outside [skip, skip + skip_len) of per-layer caches [1, H, T, D] (contiguous, one dtype):
     [L, 1, H, T - skip_len, D]."""
-    _expect_caches("outside_tokens", src)
     _, heads, tokens, dim = src[0].shape
     out = torch.empty(len(src), 1, heads, tokens - skip_len, dim, dtype=src[0].dtype, device=src[0].device)
     table = (c_i64 * len(src))(*[ptr(t) for t in src])
@@ -380,7 +372,6 @@ def project_caches(tensors, cos, sin, mean, start: int, end: int, basis, with_en
     """Centred rows of per-layer caches [1, H, T, D] times basis f32 [L*H*D, rank]: f32 [end - start, rank], and the rows'
     energies [end - start] or None (dkv_project_caches; contiguous 16-byte aligned tensors, cos and sin for keys)."""
     first = tensors[0]
-    _expect_caches("project_caches", tensors)
     _, heads, tokens, dim = first.shape
     (k, n), m = basis.shape, end - start
     _expect("project_caches", first.device, (basis, "basis", torch.float32, (len(tensors) * heads * dim, n)),
