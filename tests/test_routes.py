@@ -171,3 +171,16 @@ def test_recorded_calls_are_left_to_torch():
     torch.compile(watched, backend="eager")(x)
     watched(x)
     assert seen[0] is False and seen[-1] is False and len(seen) >= 8 and all(seen[1:-1])
+
+
+@pytest.mark.parametrize("rows,k,n,row_major,pays", [
+    (103, 28672, 2048, True, False), (128, 28672, 2048, True, False), (256, 28672, 2048, True, True),
+    (400, 4096, 4096, True, False), (480, 4096, 4096, True, True), (700, 8192, 1024, True, False),
+    (960, 8192, 1024, True, True), (256, 8192, 8192, True, False), (480, 8192, 8192, True, True),
+    (128, 2048, 28672, False, False), (192, 2048, 28672, False, False), (256, 2048, 28672, False, True),
+    (500, 1024, 8192, False, False), (720, 1024, 8192, False, True)])
+def test_split_products_where_they_measured_faster(rows, k, n, row_major, pays):
+    """Both sides of the line, at sizes timed against the library: few rows against a large basis are the library's."""
+    import kvtc
+
+    assert kvtc.split_pays(rows, k, n, row_major) is pays
