@@ -327,7 +327,11 @@ size_t dkv_attend_workspace_bytes(const dkv_attend_args_t* a);
  * codes depend on the streams only: call it
  * once before the layers of a decode step (and again after a stream
  * changes, e.g. dkv_gather_cold); every later dkv_attend_layer /
- * dkv_attend_scores / dkv_score_layer on the same workspace reads it.  Each
+ * dkv_attend_scores / dkv_score_layer on the same workspace reads it.  From
+ * then on the whole workspace is these calls': layers with more than four query
+ * rows per KV head also keep the values there for the next such layer (as fp16
+ * lines, past the decoded codes), so a caller who used any part of it for
+ * something else calls dkv_attend_prepare again before the next layer.  Each
  * stream's table (pieces + 1 rows, or rungs) holds at most 4,096 rows
  * (DKV_ESHAPE otherwise). */
 int dkv_attend_prepare(const dkv_attend_args_t* a, int32_t plane_cap, void* workspace, size_t workspace_bytes,
