@@ -251,9 +251,12 @@ int dkv_project_caches(const uint64_t* layer_ptrs, int32_t dtype, int32_t layers
  * scripts/progressive.py:147-148).  A is [M][lda]; B is [N][ldb], or with
  * b_is_kn [K][ldb]; C is [M][ldc].  Operands are split into two fp16 pieces per
  * element in the workspace (4 bytes per element of each padded operand, and
- * partial sums where a product has few tiles); errors against float64 are below a float32
- * product's.  Outputs of rows with infinities or NaN are where float32 puts
- * them. */
+ * partial sums where a product has few tiles).  An element is held to 2^-22 of
+ * itself, or to 2^-39 of its row's (of A, or column's of the product's right
+ * operand) largest where that is more: errors against float64 are below a
+ * float32 product's unless the result comes from elements 2^18 and more below
+ * their row's largest.  Outputs of rows with infinities or NaN are where
+ * float32 puts them. */
 size_t dkv_matmul_f32_workspace_bytes(int64_t M, int64_t N, int64_t K);
 int dkv_matmul_f32(const float* a, int64_t lda, const float* b, int64_t ldb, int32_t b_is_kn, const float* bias,
                    int64_t M, int64_t N, int64_t K, float* c, int64_t ldc, void* workspace, size_t workspace_bytes,

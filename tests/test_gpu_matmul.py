@@ -168,3 +168,25 @@ def test_projection_from_caches_with_every_row_flagged():
     out, flagged = timed()
     print(f"  {1e3 * plain:.0f} us, every row flagged {1e3 * flagged:.0f} us", flush=True)
     assert torch.isnan(out).all() and flagged < 4 * plain
+
+
+@pytest.mark.parametrize("above", [2.0 ** 12, 2.0 ** 18, 2.0 ** 26])
+def test_matmul_outliers_inside_rows_and_columns(above):
+    """One element of every row of A and of every column of B far above the rest, each against a zero: an element is
+    held to 2^-39 of its row's largest where 2^-22 of itself is less, so each side adds 2^-39 max |a| sum |b| at most."""
+    import dkv_hip
+
+    m, n, k = 200, 260, 1024
+    print(f"[case] matmul outliers of {above:.0f}", flush=True)
+    a, b, _ = _pair(m, n, k, True, 21)
+    a[:, 5] *= above
+    b[5] = 0.0
+    b[9] *= above
+    a[:, 9] = 0.0
+    got, ref = dkv_hip.matmul_f32(a, b).double(), a.double() @ b.double()
+    aa, bb = a.double().abs(), b.double().abs()
+    bound = (3 * 2.0 ** -22 + (3 * k / 16 + 24) * 2.0 ** -24) * (aa @ bb)
+    bound += 2.0 ** -39 * (aa.amax(1, keepdim=True) * bb.sum(0) + aa.sum(1, keepdim=True) * bb.amax(0))
+    assert ((got - ref).abs() <= bound).all()
+    if above <= 2.0 ** 12:  # within the range where the pieces hold every element
+        assert float((got - ref).norm()) <= float((torch.matmul(a, b).double() - ref).norm())
