@@ -134,3 +134,42 @@ def test_many_rows_with_zero_scale(name, tokens):
     assert torch.isfinite(got).all()
     # the weights are equal in both; their common power of two may differ
     assert torch.allclose(got, want, rtol=1e-5, atol=1e-6 * float(want.abs().max()))
+
+
+@pytest.mark.parametrize("shape,lengths", [
+    (synth.ModelShape(2, 8, 64, 40, 512), (700,)),                       # 5 query heads per KV head, one more than few rows
+    (synth.ModelShape(1, 8, 128, 64, 512), (4500,)),                     # 8, half a tile per workgroup
+    (synth.ModelShape(1, 4, 64, 32, 256), (500, 36, 37, 1300, 292, 293)),  # 8, sequences of no token, one, a tile and one more
+])
+def test_one_query_token_of_many_heads(shape, lengths):
+    """An ordinary decode step of a model with more than 4 query heads per KV head, single and ragged."""
+    from compressed_attention import CompressedContext, ModelTables
+    from hot_tier import OrderTables, PackedStream
+
+    print(f"[case] one query token, {shape.q_heads}/{shape.kv_heads} heads, {lengths}", flush=True)
+    basis = {k: synth.orthonormal_basis(shape.features, shape.rank, 51 + i) for i, k in enumerate(("key", "value"))}
+    mean = {k: torch.randn(shape.features, generator=torch.Generator().manual_seed(53)) * 0.01 for k in ("key", "value")}
+    cases = [build_case(shape, t, seed=60 + i, query_scale=100.0, q_len=1, basis=basis, mean=mean,
+                        rope_rows=max(lengths) + 1) for i, t in enumerate(lengths)]
+    for c in cases:
+        c.mask = None
+    first = cases[0]
+    tables = ModelTables(basis["key"].to(DEV), basis["value"].to(DEV), mean["key"].to(DEV), mean["value"].to(DEV),
+                         shape.layers, shape.kv_heads, shape.head_dim, first.cos.to(DEV), first.sin.to(DEV))
+    order = OrderTables(first.order.planes, first.order.prefix_bytes, DEV)
+    streams = {}
+    for kind in ("key", "value"):
+        cat = lambda f: torch.from_numpy(np.concatenate([getattr(c, f)[kind] for c in cases])).to(DEV)  # noqa: E731
+        streams[kind] = PackedStream.pack(cat("codes"), cat("low"), cat("span"), cat("pieces"), order)
+    cu = torch.tensor(np.concatenate([[0], np.cumsum([c.ctx.middle for c in cases])]), dtype=torch.int32)
+    ctx = CompressedContext(tables, streams["key"], streams["value"],
+                            torch.from_numpy(np.concatenate([c.positions for c in cases])), shape.q_heads, cu_seqlens=cu)
+    layer = shape.layers - 1
+    q = torch.cat([c.queries[layer] for c in cases]).to(DEV).contiguous()
+    ke, ve = (torch.cat([getattr(c, f)[layer] for c in cases], dim=1).to(DEV).contiguous() for f in ("key_exact", "value_exact"))
+    out = torch.empty(len(cases), 1, shape.q_heads, shape.head_dim, device=DEV)
+    ctx.run_layer(ctx.layer_args(layer, q, out, ke, ve, None, tuple(c.key_exact.shape[2] for c in cases), shape.head_dim ** -0.5))
+    torch.cuda.synchronize()
+    for b, c in enumerate(cases):
+        base = value_mean_base(c, layer) if c.ctx.middle else 0.0
+        assert_close(out[b:b + 1].cpu().numpy(), oracle_attend(c, layer), what=f"sequence {b}", base=base)
