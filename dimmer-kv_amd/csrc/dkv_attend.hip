@@ -129,13 +129,6 @@ DKV_DEVICE uint32_t pack_f16x2_rest(uint32_t packed, float lo, float hi) {
   return pack_f16x2(lo - (float)v[0], hi - (float)v[1]);
 }
 
-// s plus the two halves of a packed pair, in fp32 (subnormal halves count).
-DKV_DEVICE float add_pair(uint32_t pair, float s) {
-  typedef _Float16 half2_t __attribute__((ext_vector_type(2)));
-  const half2_t one = {(half_t)1.0f, (half_t)1.0f};
-  return __builtin_amdgcn_fdot2(__builtin_bit_cast(half2_t, pair), one, s, false);
-}
-
 DKV_DEVICE half8 lds_half8(const half_t* p) { return *(const half8*)p; }
 
 // The query type as a compile-time tag: a kernel section instantiated per type issues its query
@@ -1071,19 +1064,12 @@ __global__ __launch_bounds__(kK2Threads) void keys_scores_kernel(K2Args a) {
             for (int j = 0; j < 4; ++j)
               pw[tb][j] = make_uint2(pack_f16x2(sacc[tb][4 * j], sacc[tb][4 * j + 1]),
                                      pack_f16x2(sacc[tb][4 * j + 2], sacc[tb][4 * j + 3]));
-          // the quarter sum (lanes l32 and l32 + 32 hold the row's halves): of the fp32 probabilities, or decoding of
-          // the fp16 ones, so that a row's largest weights lose the same rounding above and below the line
+          // the quarter sum of the fp32 probabilities (lanes l32 and l32 + 32 hold the row's halves)
           float sm = 0.0f;
 #pragma unroll
-          for (int tb = 0; tb < 2; ++tb) {
-            if constexpr (ROWMAJOR) {
+          for (int tb = 0; tb < 2; ++tb)
 #pragma unroll
-              for (int v = 0; v < 16; ++v) sm += sacc[tb][v];
-            } else {
-#pragma unroll
-              for (int j = 0; j < 4; ++j) sm = add_pair(pw[tb][j].y, add_pair(pw[tb][j].x, sm));
-            }
-          }
+            for (int v = 0; v < 16; ++v) sm += sacc[tb][v];
           sm = sum_xor32(sm);
           // row l32 of the block into the staging rows
 #pragma unroll
@@ -1322,7 +1308,7 @@ DKV_DEVICE void many_rows_epilogue(const K2Args& a, floatx16 (&acc)[DB], float4 
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
         pw[j] = make_uint2(pack_f16x2(sacc[hh][4 * j], sacc[hh][4 * j + 1]), pack_f16x2(sacc[hh][4 * j + 2], sacc[hh][4 * j + 3]));
-        s = add_pair(pw[j].y, add_pair(pw[j].x, s));
+        s += (sacc[hh][4 * j] + sacc[hh][4 * j + 1]) + (sacc[hh][4 * j + 2] + sacc[hh][4 * j + 3]);
       }
       s = sum_xor32(s);
       if (lhi == 0) ssum[mb & 1][wave][hh][l32] = s;
@@ -2249,8 +2235,10 @@ __global__ __launch_bounds__(WAVES * 64) void value_weights_kernel(K3aArgs a) {
 // pairs of each token read from LDS, took 194.  416 rows x 2,965 tokens x 1,024: 12 us against 20, latency.
 //
 // Error against float64: the values' rounding to fp16 (2^-12 relative) takes the place of that of probability x scale,
-// and the sums below the line are of the fp16 probabilities; with K2's two-piece keys the outputs' distance from
-// float64 went from 5.3e-4 to 4.8e-4 (13 query tokens, fp16 out) and from 1.754e-3 to 1.743e-3 (64, bf16 out).
+// and K2 keeps its keys in two pieces for it: float32 outputs' distance went from 6.2e-4 to 5.7e-4 (1B shape, 3,001
+// tokens, 13 query tokens), 5.6e-4 to 4.8e-4 (6,007, 7, ladder codes), 5.7e-4 to 5.2e-4 (3B, 2,500, 64) and 5.3e-4 to
+// 4.7e-4 (3B, 9,000, 3).  A value's own rounding is the smaller one while a group's values lie on both sides of zero
+// or near it, as PCA coefficients do; in a group far from zero for its width it would be the larger.
 // ---------------------------------------------------------------------------
 struct K3RowsArgs {
   const uint8_t* probs;   // operand lines [rows][slots] (K2)
