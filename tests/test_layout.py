@@ -56,6 +56,49 @@ def _searched(lengths, q_heads, kv_heads, dim, rank, q_len) -> int:
     return sum(-(-x // 256) * 256 for x in areas)
 
 
+def _fixed(lengths, q_heads, kv_heads, dim, rank, q_len) -> int:
+    """Bytes of the layout by which dkv_attend_layer_noalloc takes a many-row context: no lines, one statistics entry
+    per tile, rows as they are, splits of 1,024 tokens (512 where those are fewer workgroups than CUs)."""
+    rows, tiles = q_heads * q_len, sum(-(-n // 256) for n in lengths)
+    splits = lambda tok: sum(-(-n // tok) for n in lengths)  # noqa: E731
+    n = splits(1024) if splits(1024) * (rank // 64) * -(-rows // 32) >= 256 else splits(512)
+    slots = tiles * 256 + 1024
+    areas = [slots * rank * 2, slots * rank, slots * (rank // 64) * 8, rows * slots * 2, rows * tiles * 4, rows * tiles * 4,
+             n * rows * rank * 4, rank // 128 * len(lengths) * rows * dim * 4, len(lengths) * rows * 4 * (dim + 2) * 4]
+    return sum(-(-x // 256) * 256 for x in areas)
+
+
+def _random_many_rows(rng, most_tokens):
+    batch = rng.choice([1, 1, 1, 2, 5, 20])
+    lengths = [rng.randint(1, int(10 ** rng.uniform(0, most_tokens))) for _ in range(batch)]
+    dim = rng.choice([64, 128])
+    kv_heads = 256 // dim * rng.randint(1, 8)
+    heads = kv_heads * rng.randint(1, 8)
+    q_len = rng.randint(4 * kv_heads // heads + 1, rng.choice([8, 80, 400]))
+    return lengths, (heads, kv_heads, dim, 256 * rng.randint(1, 8), q_len)
+
+
+def test_noalloc_takes_contexts_by_its_own_size():
+    """Refused exactly above the documented maximum (elsewhere the call goes on to look for a GPU), and every context
+    it takes fits the static array."""
+    rng, most = random.Random(9), dkv_hip.NOALLOC_MAX_BYTES
+    near = 0
+    for _ in range(3000):
+        lengths, shape = _random_many_rows(rng, 4.2)
+        need = _fixed(lengths, *shape)
+        if need < 4096 * 256:
+            continue
+        near += most // 2 < need < 2 * most
+        a, keep = _args(lengths, *shape)
+        a.value_basis = 256
+        if need > most:
+            assert dkv_hip.lib().dkv_attend_layer_noalloc(ctypes.byref(a), None) == -3
+            assert f"needs {need} B of scratch; the static maximum is {most} B" in dkv_hip.lib().dkv_last_error().decode()
+        else:
+            assert _bytes(lengths, *shape) <= 2 * most, (lengths, shape)
+    assert near > 200
+
+
 def test_choice_is_the_plain_search():
     rng = random.Random(4)
     for _ in range(150):
