@@ -247,10 +247,10 @@ class _Parsed:
 
     def coefficients_and_live(self, kind: str):
         """``coefficients(kind)`` and, from the same HIP pass where there is one, the groups some token uses (else None)."""
-        from kvtc import _plain_gpu
+        from kvtc import MOST_ELEMENTS, _plain_gpu
 
         codes, low, scale = self.codes[kind]
-        if codes.shape[0] > 0 and codes.shape[2] == 64 and _plain_gpu(codes, low, scale):
+        if 0 < codes.numel() < MOST_ELEMENTS and codes.shape[2] == 64 and _plain_gpu(codes, low, scale):
             values = torch.empty(codes.shape[0], codes.shape[1] * 64, dtype=torch.float32, device=codes.device)
             return values, dkv_hip.live_groups(values, codes, low, scale)
         values = codes.float() * scale.float().unsqueeze(2) + low.float().unsqueeze(2)

@@ -184,3 +184,17 @@ def test_split_products_where_they_measured_faster(rows, k, n, row_major, pays):
     import kvtc
 
     assert kvtc.split_pays(rows, k, n, row_major) is pays
+
+
+def test_launches_past_their_threads_are_left_to_torch(monkeypatch):
+    """Half a million tokens of a large model and more: sizes only, of one element expanded."""
+    import kvtc
+
+    monkeypatch.setattr(kvtc, "_plain_gpu", lambda *t: True)
+    one = torch.zeros(1)
+    for tokens, fits in ((599_186, True), (599_187, False)):
+        like = one.half().expand(1, 8, tokens, 128)
+        assert kvtc.fit_caches(one.expand(tokens, 28672), like, 28, (0, tokens), ()) is fits
+    assert kvtc.split_pays(2**21 - 1, 64, 64, True) and not kvtc.split_pays(2**21, 64, 64, True)
+    codec = _codec(rank=64)
+    assert codec._ladder_on_gpu(one.expand(2**28 - 1, 64), "key") and not codec._ladder_on_gpu(one.expand(2**28, 64), "key")
