@@ -9,6 +9,7 @@ scripts/methods.py:136-137 RuntimeError).
 
 from __future__ import annotations
 
+import contextlib
 import ctypes
 from pathlib import Path
 
@@ -143,9 +144,12 @@ def stream_handle() -> int:
     return torch.cuda.current_stream().cuda_stream
 
 
+_HERE = contextlib.nullcontext()
+
+
 def _on_device_of(t: torch.Tensor):
     """``t``'s GPU as the current device: ``stream_handle`` is then the stream that orders the work on its memory."""
-    return torch.cuda.device(t.device)
+    return _HERE if _current_device is not None and t.get_device() == _current_device() else torch.cuda.device(t.device)
 
 
 def dtype_code(dtype: torch.dtype) -> int:
@@ -374,11 +378,10 @@ def project_caches(tensors, cos, sin, mean, start: int, end: int, basis, with_en
     first = tensors[0]
     _, heads, tokens, dim = first.shape
     (k, n), m = basis.shape, end - start
-    _expect("project_caches", first.device, (basis, "basis", torch.float32, (len(tensors) * heads * dim, n)),
-            (mean, "mean", torch.float32, (k,)))
-    for t in (cos, sin):
-        if t is not None:
-            _expect("project_caches", first.device, (t, "cos and sin", torch.float32, (max(end, t.shape[0]), dim)))
+    if (k != len(tensors) * heads * dim or mean.shape != (k,)
+            or any(t is not None and (t.shape[0] < end or t.shape[1:] != (dim,)) for t in (cos, sin))):
+        raise ValueError(f"project_caches: basis and mean must be of {len(tensors) * heads * dim} columns, cos and sin of "
+                         f"{end} tokens and {dim} dimensions")
     kn = basis.stride(1) == 1 and basis.stride(0) >= n
     if not kn and not (basis.stride(0) == 1 and basis.stride(1) >= k):
         basis, kn = basis.contiguous(), True
@@ -410,9 +413,8 @@ def quantize8(coef, codes, low, span, errors=None) -> None:
 def quantize8_rungs(coef, planes, codes, low, span, errors, energy) -> None:
     """coef f32 [n, 64G], planes u8 [R, G] -> codes, low, span as quantize8's, errors f32 [n, R], energy f32 [n]."""
     n, groups = codes.shape[0], codes.shape[1]
-    _expect("quantize8_rungs", coef.device, (coef, "coef", torch.float32, (n, 64 * groups)),
-            (planes, "planes", torch.uint8, (None, groups)), (codes, "codes", torch.uint8, (n, groups, 64)),
-            (errors, "errors", torch.float32, (n, planes.shape[0])), (energy, "energy", torch.float32, (n,)))
+    if coef.shape != (n, 64 * groups) or errors.shape != (n, planes.shape[0]) or planes.shape[1:] != (groups,):
+        raise ValueError(f"quantize8_rungs: coef must be [{n}, {64 * groups}], planes [rungs, {groups}], errors [{n}, rungs]")
     with _on_device_of(codes):
         _check(lib().dkv_quantize8_rungs(c_vp(ptr(coef)), c_i32(n), c_i32(groups), c_vp(ptr(planes)), c_i32(planes.shape[0]),
                                          c_vp(ptr(codes)), c_vp(ptr(low)), c_vp(ptr(span)), c_vp(ptr(errors)),

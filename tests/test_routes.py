@@ -28,6 +28,7 @@ class Launches:
                 outer.current = self.before
 
         monkeypatch.setattr(torch.cuda, "device", Device)
+        monkeypatch.setattr(dkv_hip, "_current_device", lambda: 5)  # CPU tensors say -1
         monkeypatch.setattr(dkv_hip, "lib", lambda: self)
         monkeypatch.setattr(dkv_hip, "ptr", lambda t: None if t is None else t.data_ptr())
         monkeypatch.setattr(dkv_hip, "stream_handle", lambda: hash(self.current) & 0xFFFF)
@@ -198,3 +199,10 @@ def test_launches_past_their_threads_are_left_to_torch(monkeypatch):
     assert kvtc.split_pays(2**21 - 1, 64, 64, True) and not kvtc.split_pays(2**21, 64, 64, True)
     codec = _codec(rank=64)
     assert codec._ladder_on_gpu(one.expand(2**28 - 1, 64), "key") and not codec._ladder_on_gpu(one.expand(2**28, 64), "key")
+
+
+def test_launch_on_the_current_device_enters_nothing(monkeypatch):
+    launches = Launches(monkeypatch)
+    monkeypatch.setattr(dkv_hip, "_current_device", lambda: -1)
+    dkv_hip.ladder_errors(torch.zeros(3, 128), torch.zeros(4, 2, dtype=torch.uint8))
+    assert launches.log == [("dkv_ladder_errors", "elsewhere", hash("elsewhere") & 0xFFFF)]
