@@ -206,3 +206,18 @@ def test_launch_on_the_current_device_enters_nothing(monkeypatch):
     monkeypatch.setattr(dkv_hip, "_current_device", lambda: -1)
     dkv_hip.ladder_errors(torch.zeros(3, 128), torch.zeros(4, 2, dtype=torch.uint8))
     assert launches.log == [("dkv_ladder_errors", "elsewhere", hash("elsewhere") & 0xFFFF)]
+
+
+@pytest.mark.parametrize("kind,dtype", [("key", torch.float16), ("value", torch.bfloat16), ("key", torch.float32)])
+def test_rebuilt_caches_that_fit_take_the_kernels(kind, dtype, monkeypatch):
+    import kvtc
+
+    launches = Launches(monkeypatch)
+    monkeypatch.setattr(kvtc, "_plain_gpu", lambda *t: True)
+    codec, tokens, span = _codec(), 20, (4, 12)
+    monkeypatch.setattr(kvtc, "inverse_transform", lambda *a: torch.zeros(8, 256))
+    caches = [torch.zeros(1, 2, tokens, 64, dtype=dtype) for _ in range(2)]
+    cos = torch.ones(tokens, 64)
+    out = codec._rebuilt_caches(kind, None, caches, span, cos, cos)
+    assert [t.shape for t in out] == [t.shape for t in caches] and all(t.dtype == dtype for t in out)
+    assert [name for name, *_ in launches.log] == ["dkv_rows_to_caches", "dkv_copy_tokens"]
