@@ -342,7 +342,8 @@ def matmul_f32(a: torch.Tensor, b: torch.Tensor, bias: torch.Tensor | None = Non
     kn = b.stride(1) == 1 and b.stride(0) >= n
     if not kn and not (b.stride(0) == 1 and b.stride(1) >= k):
         b, kn = b.contiguous(), True
-    ldb = b.stride(0) if kn else b.stride(1)
+    # (a dimension of one element may have any stride, contiguous() or not)
+    lda, ldb = max(a.stride(0), k), max(b.stride(0), n) if kn else max(b.stride(1), k)
     if bias is not None:
         bias = bias.contiguous()
     out = torch.empty(m, n, dtype=torch.float32, device=a.device)
@@ -351,7 +352,7 @@ def matmul_f32(a: torch.Tensor, b: torch.Tensor, bias: torch.Tensor | None = Non
         _check(-2, "dkv_matmul_f32_workspace_bytes")
     workspace = torch.empty(need, dtype=torch.uint8, device=a.device)
     with _on_device_of(a):
-        _check(lib().dkv_matmul_f32(c_vp(a.data_ptr()), c_i64(a.stride(0)), c_vp(b.data_ptr()), c_i64(ldb), c_i32(kn),
+        _check(lib().dkv_matmul_f32(c_vp(a.data_ptr()), c_i64(lda), c_vp(b.data_ptr()), c_i64(ldb), c_i32(kn),
                                     c_vp(ptr(bias)), c_i64(m), c_i64(n), c_i64(k), c_vp(ptr(out)), c_i64(n),
                                     c_vp(ptr(workspace)), c_sz(need), c_vp(stream_handle())), "dkv_matmul_f32")
     return out
@@ -396,7 +397,7 @@ def project_caches(tensors, cos, sin, mean, start: int, end: int, basis, with_en
         _check(lib().dkv_project_caches(c_vp(ptr(table)), c_i32(dtype_code(first.dtype)), c_i32(len(tensors)), c_i32(heads),
                                         c_i32(tokens), c_i32(dim), c_vp(ptr(cos)), c_vp(ptr(sin)), c_vp(ptr(mean)),
                                         c_i32(start), c_i32(end), c_vp(basis.data_ptr()),
-                                        c_i64(basis.stride(0) if kn else basis.stride(1)), c_i32(kn), c_i64(n), c_vp(ptr(out)),
+                                        c_i64(max(basis.stride(0), n) if kn else max(basis.stride(1), k)), c_i32(kn), c_i64(n), c_vp(ptr(out)),
                                         c_i64(n), c_vp(ptr(energy)), c_vp(ptr(workspace)), c_sz(need), c_vp(stream_handle())),
                "dkv_project_caches")
     return out, energy

@@ -190,3 +190,18 @@ def test_matmul_outliers_inside_rows_and_columns(above):
     assert ((got - ref).abs() <= bound).all()
     if above <= 2.0 ** 12:  # within the range where the pieces hold every element
         assert float((got - ref).norm()) <= float((torch.matmul(a, b).double() - ref).norm())
+
+
+@pytest.mark.parametrize("m,n,k", [(1, 70, 300), (70, 90, 1), (70, 1, 300), (1, 1, 300)])
+def test_matmul_strides_of_single_rows_and_columns(m, n, k):
+    """A dimension of one element has any stride, and contiguous() leaves it."""
+    import dkv_hip
+
+    print(f"[case] matmul single {m} x {n} x {k}", flush=True)
+    a, b, _ = _pair(m, n, k, True, 31)
+    wide = torch.randn(m + k, 2 * (n + k), device=DEV)
+    views_a = [a, a.t().contiguous().t(), torch.as_strided(wide, (m, k), (1, 1)) if m == 1 else a]
+    views_b = [b, b.t().contiguous().t(), torch.as_strided(wide, (k, n), (3, 1)) if k == 1 else b]
+    for x in views_a:
+        for y in views_b:
+            _check(dkv_hip.matmul_f32(x, y), x, y)
